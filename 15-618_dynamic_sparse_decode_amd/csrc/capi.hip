@@ -128,6 +128,17 @@ struct PinnedBuffer {
   }
 };
 
+// The scratch of an attention launch that spreads heads over workgroups
+// (dsdk::AttentionArgs::piece_words, then its counters), zeroed.
+void ReservePieces(DeviceBuffer<unsigned long long>* pieces) {
+  pieces->Reserve(dsdk::AttentionPieceWords() + dsdk::AttentionPieceCounters() / 2);
+  DSD_HIP_CHECK(hipMemset(pieces->ptr, 0, pieces->count * sizeof(unsigned long long)));
+  DSD_HIP_CHECK(hipStreamSynchronize(nullptr));  // (the steps' streams do not wait for it)
+}
+unsigned* PieceArrivals(const DeviceBuffer<unsigned long long>& pieces) {
+  return reinterpret_cast<unsigned*>(pieces.ptr + dsdk::AttentionPieceWords());
+}
+
 constexpr uint64_t kLargeCopyBytes = 1ull << 20;  // src/device_page_pool.cpp:13
 
 // Polls of a cross-workgroup wait of the single-launch step before it gives
@@ -233,6 +244,12 @@ struct dsd_pool {
   PinnedBuffer<float> h_dense_q, h_dense_out;
   PinnedBuffer<int> h_dense_offsets, h_dense_ids;
   hipEvent_t dense_start = nullptr, dense_stop = nullptr;
+  // The dense attention's pieces (attention.hip): one scratch per pool, made
+  // by the first call that needs it.  piece_ev marks the end of the last
+  // launch that used it, and every launch waits for it, so calls on several
+  // streams take turns.
+  DeviceBuffer<unsigned long long> pieces;
+  hipEvent_t piece_ev = nullptr;
   uint64_t* k_offsets = nullptr;  // [capacity] element offset of each page
   uint64_t* v_offsets = nullptr;
   // The synthetic append returns once enqueued: `done` marks its end, its
@@ -266,6 +283,10 @@ struct dsd_pool {
     if (view.live) (void)hipFree(view.live);
     if (dense_start) (void)hipEventDestroy(dense_start);
     if (dense_stop) (void)hipEventDestroy(dense_stop);
+    if (piece_ev) {
+      (void)hipEventSynchronize(piece_ev);
+      (void)hipEventDestroy(piece_ev);
+    }
     if (stream) (void)hipStreamDestroy(stream);
   }
 
@@ -383,6 +404,9 @@ int dsd_pool_create(int num_heads, int head_dim, int page_size,
     DSD_HIP_CHECK(hipEventCreateWithFlags(&pool->done, hipEventDisableTiming));
     DSD_HIP_CHECK(hipEventCreate(&pool->dense_start));
     DSD_HIP_CHECK(hipEventCreate(&pool->dense_stop));
+    // (orders launches on this device only: no system-scope fence)
+    DSD_HIP_CHECK(hipEventCreateWithFlags(&pool->piece_ev,
+                                          hipEventDisableTiming | hipEventDisableSystemFence));
     pool->host_counts.assign(static_cast<size_t>(capacity_pages), 0);
     pool->host_live.assign(static_cast<size_t>(capacity_pages), 0);
     if (capacity_pages > 0) {
@@ -1355,6 +1379,11 @@ struct StepLaunch {
   unsigned* wide_seq = nullptr;       // device: captured wide launches so far
   int wide_counter_words = 0;
   unsigned* wide_launches = nullptr;  // host: wide launches so far (picks the set)
+  // The three-kernel step's attention: its pieces (0: one workgroup per head)
+  // and their scratch.
+  int piece_room = 0;
+  unsigned long long* piece_words = nullptr;
+  unsigned* piece_arrivals = nullptr;
   int* exact_pages = nullptr;         // may be null
   unsigned long long* fail_word = nullptr;
   unsigned epoch = 0;  // fresh (non-zero, below 2^30) for every launch
@@ -1425,6 +1454,9 @@ void EnqueueAttentionStage(const PoolView& v, const StepLaunch& L, hipStream_t s
   a.scale = L.scale;
   a.outputs = L.outputs;
   a.wide_partition = L.wide_shape;
+  a.piece_room = L.piece_room;
+  a.piece_words = L.piece_words;
+  a.piece_arrivals = L.piece_arrivals;
   dsdk::LaunchAttention(v, a, s);
 }
 
@@ -1579,6 +1611,7 @@ struct dsd_sparse_ctx {
   DeviceBuffer<unsigned long long> d_sel_rec;
   DeviceBuffer<unsigned> d_wide_counters;
   DeviceBuffer<unsigned> d_wide_seq;
+  DeviceBuffer<unsigned long long> d_pieces;  // the attention's (attention.hip)
   mutable unsigned wide_launches = 0;  // host count of wide launches (picks the counter set)
   // The epoch of the step being enqueued: it tags the fused step's
   // publication words and every failure report of the step's kernels.
@@ -1685,6 +1718,15 @@ struct dsd_sparse_ctx {
                    !dsdk::FusedStepSupported(v, max_n, top_k) &&
                    dsdk::WideStepSupported(v, max_n, top_k);
     L.wide = L.wide_shape && wide_enabled;
+    // Heads spread over workgroups, except for the shapes of the single
+    // launches, whose outputs the three kernels reproduce bit for bit.
+    if (d_pieces.ptr != nullptr && !L.wide_shape &&
+        !dsdk::FusedStepSupported(v, max_n, top_k)) {
+      L.piece_room = dsdk::AttentionPieceRoom(
+          v, batch, static_cast<long long>(std::max(1, top_k)) * v.page_size);
+      L.piece_words = d_pieces.ptr;
+      L.piece_arrivals = PieceArrivals(d_pieces);
+    }
     L.batch = batch;
     L.total = total;
     L.max_n = max_n;
@@ -1846,6 +1888,12 @@ int dsd_sparse_create(dsd_pool* pool, int top_k, int max_batch,
     DSD_HIP_CHECK(hipMemset(ctx->d_sel_rec.ptr, 0, (B * K + B) * sizeof(unsigned long long)));
     ctx->d_wide_counters.Reserve(4 * (B + 1));
     DSD_HIP_CHECK(hipMemset(ctx->d_wide_counters.ptr, 0, 4 * (B + 1) * sizeof(unsigned)));
+    if (dsdk::AttentionPieceRoom(pool->view, 1,
+                                 static_cast<long long>(K) * pool->view.page_size) > 0 &&
+        (!dsdk::FusedStepSupported(pool->view, 0, 0) ||
+         max_total_candidates > dsdk::WideStepMaxCandidates())) {
+      ReservePieces(&ctx->d_pieces);
+    }
     ctx->d_wide_seq.Reserve(1);
     DSD_HIP_CHECK(hipMemset(ctx->d_wide_seq.ptr, 0, sizeof(unsigned)));
     {
@@ -1902,6 +1950,7 @@ int dsd_sparse_create(dsd_pool* pool, int top_k, int max_batch,
       }
     }
     dsdk::PreloadStepKernels();
+    dsdk::PreloadAttentionKernels(pool->view);
     dsdk::PreloadFusedKernels();
     dsdk::PreloadPoolKernels();
     *out_ctx = ctx.release();
@@ -2766,6 +2815,24 @@ StaticScratch& StaticScratchOn(int device) {
   return st;
 }
 
+
+// The dense attention on stream s: spread over workgroups where few requests
+// would leave the chip idle, on the pool's one piece scratch (so it first
+// waits for the last launch that used it).  A captured launch has no place
+// in that order and stays unsplit.
+void LaunchDense(dsd_pool* pool, dsdk::AttentionArgs* a, hipStream_t s) {
+  const bool capturing = s != nullptr && StreamCapturing(s);
+  if (!capturing) a->piece_room = dsdk::AttentionPieceRoom(pool->view, a->batch, 0);
+  if (a->piece_room > 0) {
+    if (pool->pieces.ptr == nullptr) ReservePieces(&pool->pieces);
+    a->piece_words = pool->pieces.ptr;
+    a->piece_arrivals = PieceArrivals(pool->pieces);
+  }
+  if (a->piece_room > 0) DSD_HIP_CHECK(hipStreamWaitEvent(s, pool->piece_ev, 0));
+  dsdk::LaunchAttention(pool->view, *a, s);
+  if (a->piece_room > 0) DSD_HIP_CHECK(hipEventRecord(pool->piece_ev, s));
+}
+
 }  // namespace
 
 extern "C" {
@@ -2916,7 +2983,7 @@ int dsd_dense_run_batch(dsd_pool* pool, int batch, const float* queries,
     a.scale = 1.0f / std::sqrt(static_cast<float>(pool->view.head_dim));
     a.outputs = pool->h_dense_out.ptr;
     DSD_HIP_CHECK(hipEventRecord(pool->dense_start, pool->stream));
-    dsdk::LaunchAttention(pool->view, a, pool->stream);
+    LaunchDense(pool, &a, pool->stream);
     DSD_HIP_CHECK(hipEventRecord(pool->dense_stop, pool->stream));
     pool->Sync();
     std::memcpy(outputs, pool->h_dense_out.ptr, sizeof(float) * qn);
@@ -2948,7 +3015,7 @@ int dsd_dense_run_batch_device(dsd_pool* pool, int batch,
     a.batch = batch;
     a.scale = 1.0f / std::sqrt(static_cast<float>(pool->view.head_dim));
     a.outputs = d_outputs;
-    dsdk::LaunchAttention(pool->view, a, reinterpret_cast<hipStream_t>(stream));
+    LaunchDense(pool, &a, reinterpret_cast<hipStream_t>(stream));
   });
 }
 

@@ -246,7 +246,21 @@ struct AttentionArgs {
   // D = 128, E = 4096: split each head as the wide step's attention items
   // do (bit-identical outputs), for the batches that step takes.
   bool wide_partition = false;
+  // Spread each head's tokens over several workgroups (attention.hip):
+  // AttentionPieceRoom() > 0 and the scratch for it, AttentionPieceWords()
+  // words and AttentionPieceCounters() counters, all zero before the first
+  // launch that uses them (each launch leaves them zero).  Launches on one
+  // scratch must not overlap.
+  int piece_room = 0;
+  unsigned long long* piece_words = nullptr;
+  unsigned* piece_arrivals = nullptr;
 };
+size_t AttentionPieceWords();
+int AttentionPieceCounters();
+// The piece_room for a batch whose lists hold at most max_slots token slots
+// each (0: unknown); 0: one workgroup per (head, request).
+int AttentionPieceRoom(const PoolView& pool, int batch, long long max_slots);
+void PreloadAttentionKernels(const PoolView& pool);
 void LaunchAttention(const PoolView& pool, const AttentionArgs& args,
                      hipStream_t stream);
 

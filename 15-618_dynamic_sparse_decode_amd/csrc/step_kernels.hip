@@ -1,13 +1,11 @@
-// step_kernels.hip -- the three kernels of one sparse decode step (gfx950):
+// step_kernels.hip -- the kernels of one sparse decode step (gfx950):
 //   1. exact-order page scoring   (reference ScorePagesCpu, src/reference_kernels.cpp:59-80)
 //   2. per-request top-k select   (reference SelectTopKPagesCpu, :82-107)
-//   3. fused gather + attention   (reference GatherPagesCpu + SparseAttentionCpu, :109-194)
-// Dense attention (reference DenseAttentionCpu, :196-203) reuses kernel 3
-// with every candidate page as the list.
+//   3. fused gather + attention: attention.hip
+// and the wide step, all three in one launch.
 #include <cmath>
-#include <cstdio>
-#include <cstdlib>
 
+#include "attention_head.h"
 #include "dsd_internal.h"
 #include "score_slice.h"
 #include "step_common.h"
@@ -720,316 +718,6 @@ __global__ __launch_bounds__(kRankMax) void SelectCertifiedRankKernel(
 }
 
 // ---------------------------------------------------------------------------
-// 3. Fused gather + softmax attention (flash-decoding inside a workgroup).
-//
-// Workgroup = (head h, request r); its waves stride over 16-token chunks of
-// the request's page list.  Lane (g, j) = (lane/4, lane%4) owns token slot g
-// of the chunk and the j-th quarter of the head's dims, so a 4-lane group
-// reads one 4*DQ-float K row and one V row (contiguous, vectorised).  Each
-// lane keeps its own online-softmax stream (m, l, acc[DQ]) over the tokens
-// it sees: the only per-token cross-lane traffic is the 2-step dot-product
-// reduction within the group.  Streams are merged once at the end: across
-// the 16 token slots with xor shuffles, across waves through LDS.  Logits
-// live in the log2 domain (q pre-scaled by scale*log2 e) so each exponential
-// is one v_exp_f32.
-// ---------------------------------------------------------------------------
-constexpr int kAttnWaves = 4;
-constexpr int kAttnThreads = kAttnWaves * kWave;
-constexpr int kChunk = 16;
-// DQ > 0: head_dim == 4*DQ, lane j covers dims [j*DQ, (j+1)*DQ).
-// DQ == 0: generic head_dim <= 256, lane j covers dims j, j+4, j+8, ...
-template <int DQ>
-__global__ __launch_bounds__(kAttnThreads) void AttentionKernel(
-    PoolView pool, AttentionArgs args) {
-  constexpr int kRegs = DQ > 0 ? DQ : 64;
-  const int h = blockIdx.x;
-  const int r = blockIdx.y;
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x / kWave;
-  const int g = lane >> 2;
-  const int j = lane & 3;
-  const int D = pool.head_dim;
-  const int E = pool.elements;
-  const int ps = pool.page_size;
-
-  int start, count;
-  if (args.list_stride > 0) {
-    start = r * args.list_stride;
-    count = args.list_counts[r];
-  } else {
-    start = args.list_offsets[r];
-    count = args.list_offsets[r + 1] - start;
-  }
-
-  const int nd = DQ > 0 ? DQ : (D - j + 3) / 4;
-  const int dim0 = DQ > 0 ? j * DQ : j;
-  const int dstep = DQ > 0 ? 1 : 4;
-  const int head_off = h * D + dim0;
-
-  float q[kRegs];
-  float acc[kRegs];
-  {
-    const float qscale = args.scale * kLog2e;
-    const float* qp = args.queries + static_cast<size_t>(r) * E + head_off;
-    if constexpr (DQ > 0) {
-      LoadDims<DQ>(qp, q);
-    } else {
-#pragma unroll
-      for (int i = 0; i < kRegs; ++i) q[i] = i < nd ? qp[i * dstep] : 0.0f;
-    }
-#pragma unroll
-    for (int i = 0; i < kRegs; ++i) {
-      q[i] *= qscale;
-      acc[i] = 0.0f;
-    }
-  }
-
-  float m = -INFINITY;
-  float l = 0.0f;
-  const int total = count * ps;
-  for (int base = wave * kChunk; base < total; base += kAttnWaves * kChunk) {
-    const int f = base + g;
-    bool valid = false;
-    float kv[kRegs];
-    float vv[kRegs];
-    if (f < total) {
-      const int slot = f / ps;
-      const int t = f - slot * ps;
-      const int page = args.list_ids[start + slot];
-      valid = InPool(page, pool.capacity) && t < pool.token_counts[page];
-      if (valid) {
-        const size_t off = static_cast<size_t>(page) * pool.page_elems +
-                           static_cast<size_t>(t) * E + head_off;
-        if constexpr (DQ > 0) {
-          LoadDims<DQ>(pool.keys + off, kv);
-          LoadDims<DQ>(pool.values + off, vv);
-        } else {
-#pragma unroll
-          for (int i = 0; i < kRegs; ++i) {
-            kv[i] = i < nd ? pool.keys[off + i * dstep] : 0.0f;
-            vv[i] = i < nd ? pool.values[off + i * dstep] : 0.0f;
-          }
-        }
-      }
-    }
-    float dot = 0.0f;
-    if (valid) {
-#pragma unroll
-      for (int i = 0; i < kRegs; ++i) dot = fmaf(q[i], kv[i], dot);
-    }
-    dot += __shfl_xor(dot, 1, kWave);
-    dot += __shfl_xor(dot, 2, kWave);
-    if (valid) {
-      const float m_new = fmaxf(m, dot);
-      const float alpha = Exp2(m - m_new);
-      const float beta = Exp2(dot - m_new);
-      l = fmaf(l, alpha, beta);
-#pragma unroll
-      for (int i = 0; i < kRegs; ++i) acc[i] = fmaf(acc[i], alpha, beta * vv[i]);
-      m = m_new;
-    }
-  }
-
-  // Merge the 16 token-slot streams of this wave (lanes differing in g).
-  float wm = m;
-#pragma unroll
-  for (int o = 4; o < kWave; o <<= 1) wm = fmaxf(wm, __shfl_xor(wm, o, kWave));
-  const float sc = (m == -INFINITY) ? 0.0f : Exp2(m - wm);
-  float wl = l * sc;
-#pragma unroll
-  for (int i = 0; i < kRegs; ++i) acc[i] *= sc;
-#pragma unroll
-  for (int o = 4; o < kWave; o <<= 1) {
-    wl += __shfl_xor(wl, o, kWave);
-#pragma unroll
-    for (int i = 0; i < kRegs; ++i) acc[i] += __shfl_xor(acc[i], o, kWave);
-  }
-
-  // Merge the waves through LDS: s_acc[wave][D], s_m/s_l[wave].
-  extern __shared__ float smem[];
-  float* s_m = smem;
-  float* s_l = smem + kAttnWaves;
-  float* s_acc = smem + 2 * kAttnWaves;
-  if (g == 0) {
-    if (j == 0) {
-      s_m[wave] = wm;
-      s_l[wave] = wl;
-    }
-#pragma unroll
-    for (int i = 0; i < kRegs; ++i) {
-      if (i < nd) s_acc[wave * D + dim0 + i * dstep] = acc[i];
-    }
-  }
-  __syncthreads();
-  float mx = -INFINITY;
-#pragma unroll
-  for (int w = 0; w < kAttnWaves; ++w) mx = fmaxf(mx, s_m[w]);
-  float* out = args.outputs + static_cast<size_t>(r) * E + static_cast<size_t>(h) * D;
-  for (int d = threadIdx.x; d < D; d += kAttnThreads) {
-    float lt = 0.0f;
-    float at = 0.0f;
-    if (mx != -INFINITY) {
-#pragma unroll
-      for (int w = 0; w < kAttnWaves; ++w) {
-        const float s = (s_m[w] == -INFINITY) ? 0.0f : Exp2(s_m[w] - mx);
-        lt = fmaf(s_l[w], s, lt);
-        at = fmaf(s_acc[w * D + d], s, at);
-      }
-    }
-    // No valid token at all: the reference returns zeros
-    // (src/cuda/sparse_batched_attention.cu:364-369; CPU :159-161).
-    out[d] = lt == 0.0f ? 0.0f : at / lt;
-  }
-}
-
-// Fixed-D variant for the hot shape (D = 128) with the lane split, the
-// waves per workgroup and the chunks in flight per wave as parameters:
-// LPT lanes per token (each owns D/LPT contiguous dims), 64/LPT tokens per
-// chunk, UNROLL chunks whose K and V rows are all requested before any is
-// consumed (bytes in flight per wave = UNROLL * 64/LPT * 2 * D * 4).
-template <int WAVES, int D>
-struct AttnFastShared {
-  float m[WAVES];
-  float l[WAVES];
-  alignas(16) float acc[WAVES][D];
-};
-
-// Head h of request r over the `count` pages of `list` (global or LDS), by
-// WAVES waves whose thread index within the head is tid; ends with a
-// workgroup barrier (every thread of the workgroup must call it).
-template <int D, int LPT, int WAVES, int UNROLL, class List>
-__device__ __forceinline__ void AttentionFastHead(const PoolView& pool, const AttentionArgs& args,
-                                                  int h, int r, int tid, List list, int count,
-                                                  AttnFastShared<WAVES, D>& sh) {
-  constexpr int DQ = D / LPT;
-  constexpr int TPC = kWave / LPT;
-  static_assert(DQ % 4 == 0, "float4 rows");
-  const int lane = tid & (kWave - 1);
-  const int wave = tid / kWave;
-  const int g = lane / LPT;
-  const int j = lane % LPT;
-  const int E = pool.elements;
-  const int ps = pool.page_size;
-  const int head_off = h * D + j * DQ;
-  float q[DQ];
-  float acc[DQ];
-  {
-    const float qscale = args.scale * kLog2e;
-    LoadDims<DQ>(args.queries + static_cast<size_t>(r) * E + head_off, q);
-#pragma unroll
-    for (int i = 0; i < DQ; ++i) {
-      q[i] *= qscale;
-      acc[i] = 0.0f;
-    }
-  }
-  float m = -INFINITY;
-  float l = 0.0f;
-  const int total = count * ps;
-  for (int base = wave * TPC * UNROLL; base < total; base += WAVES * TPC * UNROLL) {
-    float kv[UNROLL][DQ];
-    float vv[UNROLL][DQ];
-    bool valid[UNROLL];
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-      const int f = base + u * TPC + g;
-      valid[u] = false;
-      if (f < total) {
-        const int slot = f / ps;
-        const int t = f - slot * ps;
-        const int page = list[slot];
-        valid[u] = InPool(page, pool.capacity) && t < pool.token_counts[page];
-        if (valid[u]) {
-          const size_t off = static_cast<size_t>(page) * pool.page_elems +
-                             static_cast<size_t>(t) * E + head_off;
-          LoadDims<DQ>(pool.keys + off, kv[u]);
-          LoadDims<DQ>(pool.values + off, vv[u]);
-        }
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-      float dot = 0.0f;
-      if (valid[u]) {
-#pragma unroll
-        for (int i = 0; i < DQ; ++i) dot = fmaf(q[i], kv[u][i], dot);
-      }
-#pragma unroll
-      for (int o = 1; o < LPT; o <<= 1) dot += __shfl_xor(dot, o, kWave);
-      if (valid[u]) {
-        const float m_new = fmaxf(m, dot);
-        const float alpha = Exp2(m - m_new);
-        const float beta = Exp2(dot - m_new);
-        l = fmaf(l, alpha, beta);
-#pragma unroll
-        for (int i = 0; i < DQ; ++i) acc[i] = fmaf(acc[i], alpha, beta * vv[u][i]);
-        m = m_new;
-      }
-    }
-  }
-  // merge the TPC token-slot streams of this wave
-  float wm = m;
-#pragma unroll
-  for (int o = LPT; o < kWave; o <<= 1) wm = fmaxf(wm, __shfl_xor(wm, o, kWave));
-  const float sc = (m == -INFINITY) ? 0.0f : Exp2(m - wm);
-  float wl = l * sc;
-#pragma unroll
-  for (int i = 0; i < DQ; ++i) acc[i] *= sc;
-#pragma unroll
-  for (int o = LPT; o < kWave; o <<= 1) {
-    wl += __shfl_xor(wl, o, kWave);
-#pragma unroll
-    for (int i = 0; i < DQ; ++i) acc[i] += __shfl_xor(acc[i], o, kWave);
-  }
-  float* s_m = sh.m;
-  float* s_l = sh.l;
-  float (&s_acc)[WAVES][D] = sh.acc;
-  if (g == 0) {
-    if (j == 0) {
-      s_m[wave] = wm;
-      s_l[wave] = wl;
-    }
-#pragma unroll
-    for (int i = 0; i < DQ; ++i) s_acc[wave][j * DQ + i] = acc[i];
-  }
-  __syncthreads();
-  float mx = -INFINITY;
-#pragma unroll
-  for (int w = 0; w < WAVES; ++w) mx = fmaxf(mx, s_m[w]);
-  float* out = args.outputs + static_cast<size_t>(r) * E + static_cast<size_t>(h) * D;
-  for (int d = tid; d < D; d += WAVES * kWave) {
-    float lt = 0.0f;
-    float at = 0.0f;
-    if (mx != -INFINITY) {
-#pragma unroll
-      for (int w = 0; w < WAVES; ++w) {
-        const float sw = (s_m[w] == -INFINITY) ? 0.0f : Exp2(s_m[w] - mx);
-        lt = fmaf(s_l[w], sw, lt);
-        at = fmaf(s_acc[w][d], sw, at);
-      }
-    }
-    out[d] = lt == 0.0f ? 0.0f : at / lt;
-  }
-}
-
-template <int D, int LPT, int WAVES, int UNROLL>
-__global__ __launch_bounds__(WAVES * kWave) void AttentionFastKernel(
-    PoolView pool, AttentionArgs args) {
-  __shared__ AttnFastShared<WAVES, D> sh;
-  const int r = blockIdx.y;
-  int start, count;
-  if (args.list_stride > 0) {
-    start = r * args.list_stride;
-    count = args.list_counts[r];
-  } else {
-    start = args.list_offsets[r];
-    count = args.list_offsets[r + 1] - start;
-  }
-  AttentionFastHead<D, LPT, WAVES, UNROLL>(pool, args, blockIdx.x, r, threadIdx.x,
-                                           args.list_ids + start, count, sh);
-}
-
-
-// ---------------------------------------------------------------------------
 // 4. The wide step: the three-kernel step (E = 4096, head_dim 128, up to
 // kCertMaxKeys candidates per request) in one launch.
 //
@@ -1080,15 +768,7 @@ __global__ __launch_bounds__(WAVES * kWave) void AttentionFastKernel(
 // loop stay live across all three item kinds.
 // ---------------------------------------------------------------------------
 constexpr int kWideStamps = 5;  // per item in timing mode
-
-// An attention item is one head of one request, all kFWaves waves on it,
-// with the lane split of the three-kernel step's attention for the same
-// batches (kWideAttnLpt, kWideAttnUnroll; LaunchAttention with
-// wide_partition): both step forms give bit-identical outputs.  Two heads
-// per item (8 waves each) measured 10 us slower at 32 requests of 2048
-// pages: the attention of the requests selected last ends later.
-constexpr int kWideAttnLpt = 16;
-constexpr int kWideAttnUnroll = 4;
+static_assert(kWideAttnWaves == kFWaves, "an attention item is a whole workgroup");
 
 struct WideShared {
   union {
@@ -1250,7 +930,7 @@ __device__ __forceinline__ void WideStepItem(const PoolView& pool, const WideArg
     args.queries = a.queries;
     args.scale = a.scale;
     args.outputs = a.outputs;
-    AttentionFastHead<128, kWideAttnLpt, kFWaves, kWideAttnUnroll>(
+    AttentionFastHead<128, kWideAttnLpt, kWideAttnWaves, kWideAttnUnroll>(
         pool, args, head, r, threadIdx.x, sh.page, count, sh.attn);
   }
   if (a.stamps != nullptr && threadIdx.x == 0) {
@@ -1309,50 +989,6 @@ __global__ __launch_bounds__(kFThreads) void WideStepKernel(PoolView pool, WideA
     item = sh.item;
   }
   if (item < w.items) WideStepItem(pool, w, item, sh);
-}
-
-using AttnKernelFn = void (*)(PoolView, AttentionArgs);
-
-struct AttnVariant {
-  int lpt, waves, unroll;
-  AttnKernelFn fn;
-};
-
-#define DSD_ATTN_VARIANT(L, W, U) \
-  AttnVariant{L, W, U, AttentionFastKernel<128, L, W, U>}
-const AttnVariant kAttnVariants[] = {
-    DSD_ATTN_VARIANT(4, 4, 1),  DSD_ATTN_VARIANT(4, 4, 2),  DSD_ATTN_VARIANT(4, 8, 1),
-    DSD_ATTN_VARIANT(8, 4, 1),  DSD_ATTN_VARIANT(8, 4, 2),  DSD_ATTN_VARIANT(8, 4, 4),
-    DSD_ATTN_VARIANT(8, 8, 1),  DSD_ATTN_VARIANT(8, 8, 2),  DSD_ATTN_VARIANT(16, 4, 2),
-    DSD_ATTN_VARIANT(16, 4, 4), DSD_ATTN_VARIANT(16, 8, 2), DSD_ATTN_VARIANT(16, 8, 4),
-    DSD_ATTN_VARIANT(16, 16, 4),
-};
-#undef DSD_ATTN_VARIANT
-
-// The D = 128 variant in use: DSD_ATTN_VARIANT="LPTxWAVESxUNROLL" selects
-// one of kAttnVariants (a tuning knob); otherwise the measured default.
-const AttnVariant& SelectAttnVariant() {
-  int lpt = 16, waves = 8, unroll = 4;
-  if (const char* env = std::getenv("DSD_ATTN_VARIANT")) {
-    int a = 0, b = 0, c = 0;
-    if (std::sscanf(env, "%dx%dx%d", &a, &b, &c) == 3) {
-      lpt = a;
-      waves = b;
-      unroll = c;
-    }
-  }
-  for (const auto& v : kAttnVariants) {
-    if (v.lpt == lpt && v.waves == waves && v.unroll == unroll) return v;
-  }
-  throw std::invalid_argument("unknown DSD_ATTN_VARIANT");
-}
-
-template <int DQ>
-void LaunchAttentionT(const PoolView& pool, const AttentionArgs& args,
-                      hipStream_t stream) {
-  const size_t lds = sizeof(float) * (2 * kAttnWaves + kAttnWaves * pool.head_dim);
-  hipLaunchKernelGGL(AttentionKernel<DQ>, dim3(pool.num_heads, args.batch),
-                     dim3(kAttnThreads), lds, stream, pool, args);
 }
 
 }  // namespace
@@ -1510,46 +1146,9 @@ void LaunchSelectTopK(const float* d_scores, const int* d_cand_offsets,
   DSD_HIP_CHECK(hipGetLastError());
 }
 
-void LaunchAttention(const PoolView& pool, const AttentionArgs& args,
-                     hipStream_t stream) {
-  if (args.batch <= 0 || pool.num_heads <= 0) return;
-  const int D = pool.head_dim;
-  if (D <= 0 || D > 256) {
-    throw std::invalid_argument("head_dim must be in (0, 256]");
-  }
-  if (D == 128 && args.wide_partition && pool.elements == kFE) {
-    // the wide step's partition of a head (kFWaves waves)
-    hipLaunchKernelGGL((AttentionFastKernel<128, kWideAttnLpt, kFWaves, kWideAttnUnroll>),
-                       dim3(pool.num_heads, args.batch), dim3(kFThreads), 0, stream, pool, args);
-    DSD_HIP_CHECK(hipGetLastError());
-    return;
-  }
-  if (D == 128) {
-    const AttnVariant& v = SelectAttnVariant();
-    hipLaunchKernelGGL(v.fn, dim3(pool.num_heads, args.batch), dim3(v.waves * kWave), 0,
-                       stream, pool, args);
-    DSD_HIP_CHECK(hipGetLastError());
-    return;
-  }
-  switch (D % 4 == 0 ? D / 4 : 0) {
-    case 1: LaunchAttentionT<1>(pool, args, stream); break;
-    case 2: LaunchAttentionT<2>(pool, args, stream); break;
-    case 4: LaunchAttentionT<4>(pool, args, stream); break;
-    case 8: LaunchAttentionT<8>(pool, args, stream); break;
-    case 16: LaunchAttentionT<16>(pool, args, stream); break;
-    case 20: LaunchAttentionT<20>(pool, args, stream); break;
-    case 32: LaunchAttentionT<32>(pool, args, stream); break;
-    case 64: LaunchAttentionT<64>(pool, args, stream); break;
-    default: LaunchAttentionT<0>(pool, args, stream); break;
-  }
-  DSD_HIP_CHECK(hipGetLastError());
-}
-
 void PreloadStepKernels() {
   PreloadKernel(WideStepKernel);
   PreloadKernel(WideBumpKernel);
-  PreloadKernel(AttentionFastKernel<128, kWideAttnLpt, kFWaves, kWideAttnUnroll>);
-  PreloadKernel(SelectAttnVariant().fn);
   PreloadKernel(SelectCertifiedKernel);
   PreloadKernel(SelectCertifiedRankKernel);
   PreloadKernel(ScoreBoundGenericKernel);

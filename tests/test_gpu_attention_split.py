@@ -1,0 +1,125 @@
+"""Attention whose heads are spread over several workgroups (attention.hip):
+pieces at their edges, the scratch left clean for the next launch, launches on
+two streams, and a captured step.
+
+Tolerance: outputs within 1e-4 of the oracle, the path's bar.  The rounding
+bound behind it: a logit is a dot of D <= 256 products summed in fp32 along
+paths of at most D/LPT + 6 additions, so its error is below
+26 * 2^-24 * sum|q_i k_i| / sqrt(D) (about 1.6e-5 for N(0, 1) rows at D = 256),
+and an output moves by at most twice that times the largest |value| (about 5)
+in the worst case.  Merging pieces adds one exponential and one product per
+piece, the same as merging waves.
+"""
+import numpy as np
+import pytest
+
+import _oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+def make_pool(gpu, H, D, ps, lengths, seed):
+    batch = gpu.SyntheticBatch(H, D, ps, lengths, seed=seed)
+    pool = gpu.DevicePagePool(H, D, ps, batch.capacity)
+    batch.upload(pool)
+    return batch, pool
+
+
+@pytest.mark.parametrize("H,D,ps,lengths", [
+    (2, 128, 16, [1, 0, 127, 128, 129, 384, 385, 3000]),  # steps of 128 slots, 3 and 4 of them
+    (2, 128, 1, [700, 256, 257]),       # one token per page: several tiles of 256 entries
+    (4, 128, 48, [5000, 49]),           # pieces that start inside a page
+    (1, 64, 16, [767, 768, 769, 9000]),
+    (3, 80, 16, [1300, 1]),             # 128-slot steps, 6 merge groups
+    (3, 96, 16, [2000, 17]),
+    (2, 256, 16, [600, 1025]),          # two merge groups
+    (2, 32, 16, [900]),                 # no float4 lane split: one workgroup per head
+])
+def test_dense_pieces_match_oracle(gpu, H, D, ps, lengths):
+    import torch
+    batch, pool = make_pool(gpu, H, D, ps, lengths, seed=sum(lengths) + D)
+    want = orc.dense_batch(batch.queries, batch.key_pool, batch.value_pool, batch.token_counts,
+                           batch.cand_offsets, batch.cand_ids, H, D, ps)
+    dev = [torch.from_numpy(a).cuda() for a in (batch.queries, batch.cand_offsets,
+                                                batch.cand_ids)]
+    outs = [torch.full((len(lengths), H * D), 7.0, device="cuda") for _ in range(6)]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    # back to back, the streams in turn: one scratch, launches in order
+    for i, out in enumerate(outs):
+        gpu.dense_run_batch_device(pool, len(lengths), *[t.data_ptr() for t in dev],
+                                   out.data_ptr(), streams[i % 2].cuda_stream)
+    torch.cuda.synchronize()
+    host, _ = gpu.dense_run_batch(pool, batch.queries, batch.cand_offsets, batch.cand_ids)
+    assert orc.max_abs_diff(host, np.asarray(want).reshape(host.shape)) <= 1e-4
+    for out in outs:
+        assert np.array_equal(out.cpu().numpy().view(np.uint32), host.view(np.uint32))
+    pool.close()
+
+
+def test_captured_dense_step(gpu):
+    import torch
+    H, D, ps = 2, 128, 16
+    batch, pool = make_pool(gpu, H, D, ps, [1500, 40], seed=3)
+    want = orc.dense_batch(batch.queries, batch.key_pool, batch.value_pool, batch.token_counts,
+                           batch.cand_offsets, batch.cand_ids, H, D, ps)
+    dev = [torch.from_numpy(a).cuda() for a in (batch.queries, batch.cand_offsets,
+                                                batch.cand_ids)]
+    out = torch.zeros(2, H * D, device="cuda")
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=side):
+        gpu.dense_run_batch_device(pool, 2, *[t.data_ptr() for t in dev], out.data_ptr(),
+                                   side.cuda_stream)
+    for _ in range(3):
+        out.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert orc.max_abs_diff(out.cpu().numpy(),
+                                np.asarray(want).reshape(2, H * D)) <= 1e-4
+    pool.close()
+
+
+def test_sparse_step_with_pieces_eager_and_captured(gpu):
+    """Lists of up to 40 x 16 slots (five steps) of a few heads: the sparse
+    step's attention in pieces, the same bits from a graph's replays."""
+    import torch
+    H, D, ps, k = 8, 128, 16, 40
+    lengths = [2100, 90, 700]
+    batch, pool = make_pool(gpu, H, D, ps, lengths, seed=11)
+    summ = orc.pool_summaries(batch.key_pool, batch.token_counts, H * D)
+    rng = np.random.default_rng(12)
+    sets = [batch.queries, rng.standard_normal(batch.queries.shape).astype(np.float32)]
+    offs, ids = (torch.from_numpy(a).cuda() for a in (batch.cand_offsets, batch.cand_ids))
+    q = torch.zeros(3, H * D, device="cuda")
+    out = torch.zeros(3, H * D, device="cuda")
+    total, most = batch.total_candidates, batch.max_candidates
+    with gpu.SparseContext(pool, k, 3, total, 3 * k) as ctx:
+        def step(stream):
+            ctx.run_batch_device(3, total, most, q.data_ptr(), offs.data_ptr(), ids.data_ptr(),
+                                 out.data_ptr(), stream=stream)
+
+        main = torch.cuda.Stream()
+        eager = []
+        for qs in sets:
+            q.copy_(torch.from_numpy(qs))
+            torch.cuda.synchronize()
+            step(main.cuda_stream)
+            torch.cuda.synchronize()
+            eager.append(out.cpu().numpy().copy())
+            _, _, want = orc.sparse_batch(qs, batch.key_pool, batch.value_pool, summ,
+                                          batch.token_counts, batch.cand_offsets,
+                                          batch.cand_ids, H, D, ps, k)
+            assert orc.max_abs_diff(eager[-1], want) <= 1e-4
+        side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            step(side.cuda_stream)
+        for i in (1, 0, 1):
+            q.copy_(torch.from_numpy(sets[i]))
+            out.fill_(7.0)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(out.cpu().numpy().view(np.uint32), eager[i].view(np.uint32))
+        ctx.device_status()
+    pool.close()
