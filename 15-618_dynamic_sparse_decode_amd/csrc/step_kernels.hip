@@ -3,6 +3,7 @@
 //   2. per-request top-k select   (reference SelectTopKPagesCpu, :82-107)
 //   3. fused gather + attention: attention.hip
 // and the wide step, all three in one launch.
+#include <algorithm>
 #include <cmath>
 
 #include "attention_head.h"
@@ -82,64 +83,143 @@ __global__ __launch_bounds__(kWave) void ScoreExactKernel(
 // sequential fp32 sum can be from that sum:
 //   acc_i = fl(acc_{i-1} + p_i)  =>  |acc_n - S| <= u * sum_i |T_i| / (1 - n u)
 // with S = sum p_i, T_i the exact prefix sums and u = 2^-24 (plus 2^-150 per
-// step for subnormal results).  Each lane owns a contiguous block of BL
-// products: pass 1 sums the block, a wave exclusive scan gives the block's
-// starting prefix, pass 2 accumulates |T_i|.  Double rounding of the scan is
-// covered by generous slack terms.  The page's score interval
+// step for subnormal results).  The page's score interval
 // [fl(lo*scale), fl(hi*scale)] (lo/hi rounded outward to float) provably
 // contains the reference score, because fl(x*scale) is monotone in x.
 // At E = 4096 the fused step's float score passes (ScorePagesKernel in
 // fused_step.hip) take this role; the kernel below serves the other E.
+//
+// Bound by the summary rows (4*E bytes a page against about 11 fp64 and 40
+// other instructions per 256 products).  A row of 256 products is one float4
+// per lane, so every load reads 1 KiB contiguously (a block of E/64
+// consecutive products per lane, read one at a time, took 94 us for the 40 MB
+// of 32 requests of 8 x 128 heads, about 300 pages each; this form
+// 17 us).  Prefix sums: within the float4, then a wave scan of the lanes'
+// sums, then the rows' totals one after the other; on any product's path at
+// most 3 + 6 + E/256 + 2 double additions, far below the n roundings that
+// WriteBounds allows for.  A wave takes `per_wave` pages of its request: their
+// ids and token counts load once, lane i holding page i's, the next kRows rows
+// load while this one's are summed, and page i's sums end in lane i, so the
+// interval arithmetic runs once for all of them.  The query is staged in LDS
+// up to kQueryLds bytes.
 // ---------------------------------------------------------------------------
 constexpr int kBoundWaves = 4;
+constexpr int kBoundRows = 4;                     // rows of 256 products in flight
+constexpr size_t kBoundQueryLds = 64 * 1024;
 
-// Any E that is a multiple of 64: runtime block length, products re-formed
-// from the (cache-resident) operands in pass 2.
+
+// Any E that is a multiple of 64 (the last row may be part empty).
+template <bool kQueryLds>
 __global__ __launch_bounds__(kBoundWaves * kWave) void ScoreBoundGenericKernel(
     const float* __restrict__ queries, const float* __restrict__ summaries,
     const int* __restrict__ token_counts, int capacity, const int* __restrict__ cand_offsets,
-    const int* __restrict__ cand_ids, int total, int E, float scale, float* __restrict__ mid_out,
-    float* __restrict__ lo_out, float* __restrict__ hi_out, FailReport fail) {
-  const int BL = E / kWave;
+    const int* __restrict__ cand_ids, int total, int per_wave, int E, float scale,
+    float* __restrict__ mid_out, float* __restrict__ lo_out, float* __restrict__ hi_out,
+    FailReport fail) {
+  extern __shared__ float4 q_lds[];
   const int r = blockIdx.y;
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
+  const int groups = E / 4;  // float4 groups
+  const float4* __restrict__ q4 =
+      reinterpret_cast<const float4*>(queries + static_cast<size_t>(r) * E);
   int begin, n;
-  if (!RequestRange(cand_offsets, r, total, fail, &begin, &n)) return;
-  const int c = begin + blockIdx.x * kBoundWaves + wave;
-  if (c >= begin + n) return;
-  int page = cand_ids[c];
-  bool zero = false;
-  if (!InPool(page, capacity)) {  // scores as an empty page, reported
-    if (lane == 0) ReportFailure(fail, kFailPageId);
-    page = 0;
-    zero = true;
+  const bool ok = RequestRange(cand_offsets, r, total, fail, &begin, &n);
+  const int first = (static_cast<int>(blockIdx.x) * kBoundWaves + wave) * per_wave;
+  if (!ok || static_cast<int>(blockIdx.x) * kBoundWaves * per_wave >= n) return;
+  if constexpr (kQueryLds) {
+    for (int i = threadIdx.x; i < groups; i += kBoundWaves * kWave) q_lds[i] = q4[i];
   }
-  zero = zero || token_counts[page] == 0;
-  const float* __restrict__ q = queries + static_cast<size_t>(r) * E + lane * BL;
-  const float* __restrict__ s = summaries + static_cast<size_t>(page) * E + lane * BL;
-  double block = 0.0, abs_p = 0.0;
-  for (int i = 0; i < BL; ++i) {
-    const float pi = __fmul_rn(q[i], zero ? 0.0f : s[i]);
-    block += static_cast<double>(pi);
-    abs_p += fabs(static_cast<double>(pi));
+  const int pages = n - first < per_wave ? n - first : per_wave;  // <= kWave
+  // Lane i: page i of this wave; -1 (an id outside the pool, reported, or a
+  // page holding no tokens) scores as an all-zero summary.
+  int my_page = -1;
+  if (lane < pages) {
+    const int id = cand_ids[begin + first + lane];
+    if (!InPool(id, capacity)) {
+      ReportFailure(fail, kFailPageId);
+    } else if (token_counts[id] != 0) {
+      my_page = id;
+    }
   }
-  double incl = block;
-  for (int o = 1; o < kWave; o <<= 1) {
-    const double t = __shfl_up(incl, o, kWave);
-    if (lane >= o) incl += t;
+  if constexpr (kQueryLds) __syncthreads();
+  if (pages <= 0) return;
+  const int rows = (groups + kWave - 1) / kWave;
+  const int steps = (rows + kBoundRows - 1) / kBoundRows;
+  float4 next[kBoundRows];
+  auto load = [&](int i, int step) {
+    const int page = __builtin_amdgcn_readlane(my_page, i);
+    const float4* s4 = reinterpret_cast<const float4*>(
+        summaries + static_cast<size_t>(page < 0 ? 0 : page) * E);
+#pragma unroll
+    for (int u = 0; u < kBoundRows; ++u) {
+      const int g = (step * kBoundRows + u) * kWave + lane;
+      next[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if (page >= 0 && g < groups) next[u] = s4[g];
+    }
+  };
+  double my_sum = 0.0, my_prefix = 0.0, my_abs = 0.0;
+  double carry = 0.0, abs_prefix = 0.0, abs_p = 0.0;
+  load(0, 0);
+  int i = 0, step = 0;
+  for (int unit = 0; unit < pages * steps; ++unit) {
+    float4 sv[kBoundRows];
+#pragma unroll
+    for (int u = 0; u < kBoundRows; ++u) sv[u] = next[u];
+    const bool last_step = step + 1 == steps;
+    const int ni = last_step ? i + 1 : i;
+    const int nstep = last_step ? 0 : step + 1;
+    if (ni < pages) load(ni, nstep);
+#pragma unroll
+    for (int u = 0; u < kBoundRows; ++u) {
+      const int row = step * kBoundRows + u;
+      if (row >= rows) break;
+      const int g = row * kWave + lane;
+      float4 qv = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if (g < groups) {
+        if constexpr (kQueryLds) {
+          qv = q_lds[g];
+        } else {
+          qv = q4[g];
+        }
+      }
+      const double p0 = static_cast<double>(__fmul_rn(qv.x, sv[u].x));
+      const double p1 = static_cast<double>(__fmul_rn(qv.y, sv[u].y));
+      const double p2 = static_cast<double>(__fmul_rn(qv.z, sv[u].z));
+      const double p3 = static_cast<double>(__fmul_rn(qv.w, sv[u].w));
+      const double l1 = p0 + p1;
+      const double l2 = l1 + p2;
+      const double l3 = l2 + p3;
+      abs_p += (fabs(p0) + fabs(p1)) + (fabs(p2) + fabs(p3));
+      const double incl = WaveInclusiveScanD(l3);
+      // The prefix before this lane's group: exactly the lane below's scan.
+      const double start = carry + DppMoveD<kWaveShr1>(incl);
+      // (an empty group past E adds no prefix)
+      if (g < groups) {
+        abs_prefix += (fabs(start + p0) + fabs(start + l1)) +
+                      (fabs(start + l2) + fabs(start + l3));
+      }
+      carry += ReadLaneD(incl, kWave - 1);
+    }
+    if (last_step) {
+      const double tp = WaveSum(abs_prefix);
+      const double ta = WaveSum(abs_p);
+      if (lane == i) {
+        my_sum = carry;
+        my_prefix = tp;
+        my_abs = ta;
+      }
+      carry = 0.0;
+      abs_prefix = 0.0;
+      abs_p = 0.0;
+    }
+    i = ni;
+    step = nstep;
   }
-  double prefix = __shfl_up(incl, 1, kWave);
-  if (lane == 0) prefix = 0.0;
-  double abs_prefix = 0.0;
-  for (int i = 0; i < BL; ++i) {
-    prefix += static_cast<double>(__fmul_rn(q[i], zero ? 0.0f : s[i]));
-    abs_prefix += fabs(prefix);
+  if (lane < pages) {
+    WriteBounds(my_sum, my_prefix, my_abs, E, scale, mid_out, lo_out, hi_out,
+                begin + first + lane);
   }
-  const double s_hat = __shfl(incl, kWave - 1, kWave);
-  abs_prefix = WaveSum(abs_prefix);
-  abs_p = WaveSum(abs_p);
-  if (lane == 0) WriteBounds(s_hat, abs_prefix, abs_p, E, scale, mid_out, lo_out, hi_out, c);
 }
 
 // ---------------------------------------------------------------------------
@@ -1024,18 +1104,34 @@ void LaunchScoreBounds(const PoolView& pool, const float* d_queries,
                        int total_candidates, int max_candidates, float scale, float* d_mid,
                        float* d_lo, float* d_hi, FailReport fail, hipStream_t stream) {
   if (batch <= 0 || max_candidates <= 0) return;
-  const dim3 grid((max_candidates + kBoundWaves - 1) / kBoundWaves, batch);
-  const dim3 block(kBoundWaves * kWave);
   if (pool.elements == 4096) {
     // The fused step's float score passes, 8..128 pages per workgroup.
     LaunchScorePages(pool, d_queries, d_cand_offsets, d_cand_ids, batch, total_candidates,
                      max_candidates, scale, d_mid, d_lo, d_hi, fail, stream);
     return;
-  } else {
-    hipLaunchKernelGGL(ScoreBoundGenericKernel, grid, block, 0, stream, d_queries,
+  }
+  // Enough waves for the chip to hold (8192; 32 requests of 8 x 128 heads and
+  // 300 pages each: the step took 49.5 us, 51.6 with 4096 and 54.4 with 1024),
+  // fewer where a workgroup's copy of a long query weighs more (16 requests of
+  // 64 x 128 heads: 120.7 us with 4096, 124.0 with 8192, 137 with 1024); 1 to
+  // 64 pages each.
+  const int target_waves = pool.elements > 4096 ? 4096 : 8192;
+  const int per_wave = std::min(
+      kWave, std::max(1, (total_candidates + target_waves - 1) / target_waves));
+  const int per_group = per_wave * kBoundWaves;
+  const dim3 grid((max_candidates + per_group - 1) / per_group, batch);
+  const dim3 block(kBoundWaves * kWave);
+  const size_t query_bytes = sizeof(float) * static_cast<size_t>(pool.elements);
+  if (query_bytes <= kBoundQueryLds) {
+    hipLaunchKernelGGL(ScoreBoundGenericKernel<true>, grid, block, query_bytes, stream, d_queries,
                        pool.summaries, pool.token_counts, pool.capacity, d_cand_offsets,
-                       d_cand_ids, total_candidates, pool.elements, scale, d_mid, d_lo, d_hi,
-                       fail);
+                       d_cand_ids, total_candidates, per_wave, pool.elements, scale, d_mid, d_lo,
+                       d_hi, fail);
+  } else {
+    hipLaunchKernelGGL(ScoreBoundGenericKernel<false>, grid, block, 0, stream, d_queries,
+                       pool.summaries, pool.token_counts, pool.capacity, d_cand_offsets,
+                       d_cand_ids, total_candidates, per_wave, pool.elements, scale, d_mid, d_lo,
+                       d_hi, fail);
   }
   DSD_HIP_CHECK(hipGetLastError());
 }
@@ -1151,7 +1247,7 @@ void PreloadStepKernels() {
   PreloadKernel(WideBumpKernel);
   PreloadKernel(SelectCertifiedKernel);
   PreloadKernel(SelectCertifiedRankKernel);
-  PreloadKernel(ScoreBoundGenericKernel);
+  PreloadKernel(ScoreBoundGenericKernel<true>);
 }
 
 }  // namespace dsdk
