@@ -148,6 +148,10 @@ constexpr uint64_t kLargeCopyBytes = 1ull << 20;  // src/device_page_pool.cpp:13
 // process holding them), which then fails instead of hanging.
 constexpr unsigned kDefaultSpinLimit = 1u << 17;
 
+// The same for the large select's helper workgroups, whose wait falls back to
+// other work: about 0.2 ms.
+constexpr unsigned kAssistSpins = 256;
+
 // Uploads from pageable memory of at least kStageMinBytes go through pinned
 // staging: the host threads copy one chunk while the DMA engine moves the
 // previous one (the runtime's own pageable path copies at about 27 GB/s on
@@ -1414,9 +1418,16 @@ float StepScale(const PoolView& v) {
 // Certified scoring unless exact scores are requested or the shape is
 // outside what the certified kernels handle; the single-launch step for
 // certified selection on the hot shape.
-bool StepCertified(const PoolView& v, int score_mode, int max_n, bool need_exact_scores) {
+bool StepCertified(const PoolView& v, int score_mode, int max_n, int top_k,
+                   bool need_exact_scores) {
   return score_mode == DSD_SCORE_CERTIFIED && !need_exact_scores &&
-         dsdk::CertifiedScoringSupported(v.elements, max_n);
+         dsdk::CertifiedScoringSupported(v.elements, max_n, top_k);
+}
+// A device step that returns its scores gets midpoints from certified
+// scoring; from the candidate count on where that may defer to exact scores
+// it always gets exact ones.
+bool StepWantsExactScores(const float* d_scores, int max_n) {
+  return d_scores != nullptr && dsdk::CertifiedSelectMayDefer(max_n);
 }
 bool StepFused(const PoolView& v, bool certified, bool enabled, int max_n, int top_k) {
   return certified && enabled && dsdk::FusedStepSupported(v, max_n, top_k);
@@ -1435,9 +1446,21 @@ void EnqueueScoreStage(const PoolView& v, const StepLaunch& L, hipStream_t s) {
 
 void EnqueueSelectStage(const PoolView& v, const StepLaunch& L, hipStream_t s) {
   if (L.certified) {
+    dsdk::SelectAssist assist;
+    assist.words = L.rec;
+    // (a captured step's epoch would repeat: no helpers)
+    assist.epoch = L.epoch_src != nullptr || L.never_ready ? 0u : L.epoch;
+    assist.spin_limit = std::min(L.spin_limit, kAssistSpins);
+    assist.compute_units = L.compute_units;
     dsdk::LaunchSelectCertified(v, L.scores, L.lo, L.hi, L.queries, L.offsets, L.ids, L.batch,
                                 L.total, L.max_n, L.scale, L.top_k, L.selected, L.counts,
-                                L.exact_pages, L.Fail(), s);
+                                L.exact_pages, L.Fail(), s, assist);
+    if (dsdk::CertifiedSelectMayDefer(L.max_n)) {
+      dsdk::LaunchScoreExact(v, L.queries, L.offsets, L.ids, L.batch, L.total, L.max_n, L.scale,
+                             L.scores, L.Fail(), s, L.counts);
+      dsdk::LaunchSelectTopK(L.scores, L.offsets, L.ids, L.batch, L.total, L.max_n, L.top_k,
+                             L.selected, L.counts, L.Fail(), s, true);
+    }
   } else {
     dsdk::LaunchSelectTopK(L.scores, L.offsets, L.ids, L.batch, L.total, L.max_n, L.top_k,
                            L.selected, L.counts, L.Fail(), s);
@@ -1710,7 +1733,7 @@ struct dsd_sparse_ctx {
     StepLaunch L;
     const PoolView& v = pool->view;
     L.valid = true;
-    L.certified = StepCertified(v, score_mode, max_n, need_exact_scores);
+    L.certified = StepCertified(v, score_mode, max_n, top_k, need_exact_scores);
     L.fused = StepFused(v, L.certified, fused_enabled, max_n, top_k);
     // The wide step takes the batches the single launch cannot (a request
     // beyond 256 candidates); DSD_FUSED_STEP=0 alone keeps three kernels.
@@ -2602,7 +2625,8 @@ int dsd_sparse_run_batch_device(dsd_sparse_ctx* ctx, int batch,
     Require(d_queries != nullptr && d_cand_offsets != nullptr && d_outputs != nullptr,
             "device inputs must be non-null");
     if (total_candidates > 0) Require(d_cand_ids != nullptr, "cand_ids must be non-null");
-    StepLaunch L = ctx->Plan(batch, total_candidates, max_candidates, false);
+    StepLaunch L = ctx->Plan(batch, total_candidates, max_candidates,
+                              StepWantsExactScores(d_scores, max_candidates));
     L.queries = d_queries;
     L.offsets = d_cand_offsets;
     L.ids = d_cand_ids;
@@ -2879,7 +2903,8 @@ int dsd_sparse_run_batch_device_static(dsd_pool* pool, int top_k, int batch,
     const PoolView& v = pool->view;
     StepLaunch L;
     L.valid = true;
-    L.certified = StepCertified(v, DSD_SCORE_CERTIFIED, max_candidates, false);
+    L.certified = StepCertified(v, DSD_SCORE_CERTIFIED, max_candidates, top_k,
+                                StepWantsExactScores(d_scores, max_candidates));
     L.fused = StepFused(v, L.certified, true, max_candidates, top_k);
     // (three kernels where a context would run the wide step, with its
     // attention partition: the same outputs)

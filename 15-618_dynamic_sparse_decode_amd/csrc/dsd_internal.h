@@ -188,16 +188,21 @@ void LaunchStepMark(unsigned long long* words, unsigned long long ticket, hipStr
 // ---- decode-step kernels (step_kernels.hip) --------------------------------
 
 // Exact-order page scores: scores[c] = fl(sum_seq q*s) * scale, bit-equal to
-// the reference's sequential CPU loop.
+// the reference's sequential CPU loop.  With d_undecided, only the requests
+// whose entry is negative.
 void LaunchScoreExact(const PoolView& pool, const float* d_queries,
                       const int* d_cand_offsets, const int* d_cand_ids,
                       int batch, int total_candidates, int max_candidates, float scale,
-                      float* d_scores, FailReport fail, hipStream_t stream);
+                      float* d_scores, FailReport fail, hipStream_t stream,
+                      const int* d_undecided = nullptr);
 
 // Certified scoring: per candidate an interval [lo, hi] that provably holds
 // the reference's sequential-fp32 score, and its midpoint.  Needs E % 64 == 0
-// and at most 2048 candidates per request (next power of two).
-bool CertifiedScoringSupported(int elements, int max_candidates);
+// and at most 2048 candidates per request, or 8192 with top_k <= 1024.
+bool CertifiedScoringSupported(int elements, int max_candidates, int top_k);
+// Whether LaunchSelectCertified may leave requests of such a batch undecided
+// (count -1): LaunchScoreExact and LaunchSelectTopK then finish those.
+bool CertifiedSelectMayDefer(int max_candidates);
 void LaunchScoreBounds(const PoolView& pool, const float* d_queries,
                        const int* d_cand_offsets, const int* d_cand_ids, int batch,
                        int total_candidates, int max_candidates, float scale, float* d_mid,
@@ -212,23 +217,36 @@ void LaunchScoreBounds(const PoolView& pool, const float* d_queries,
 // candidate list is longer than max_candidates (the score kernels covered
 // only that many) or whose offsets leave [0, total_candidates] selects
 // nothing and is reported (kFailShape).
+// assist: for more than 2048 candidates per request, helper workgroups that
+// refine a request's flagged pages.  words: the publication words of the
+// candidates (3 each, FusedArgs::rec), epoch a tag no earlier launch on them
+// used (0: no helpers), spin_limit polls until a wait gives up (its request
+// then goes to the exact chains).
+struct SelectAssist {
+  unsigned long long* words = nullptr;
+  unsigned epoch = 0;
+  unsigned spin_limit = 0;
+  int compute_units = 0;
+  int helpers = 0;  // per request; set by the launch
+};
 void LaunchSelectCertified(const PoolView& pool, const float* d_mid, const float* d_lo,
                            const float* d_hi,
                            const float* d_queries,
                            const int* d_cand_offsets, const int* d_cand_ids, int batch,
                            int total_candidates, int max_candidates, float scale, int top_k,
                            int* d_selected, int* d_counts, int* d_exact_pages, FailReport fail,
-                           hipStream_t stream);
+                           hipStream_t stream, const SelectAssist& assist);
 
 // Largest next-pow2 candidate count the LDS select handles.
 int SelectMaxCandidates();
 
 // Per-request top-k by (score desc, id asc): selected[r*top_k + j],
-// counts[r] = min(top_k, n_r).
+// counts[r] = min(top_k, n_r).  With undecided_only, only the requests whose
+// count is negative.
 void LaunchSelectTopK(const float* d_scores, const int* d_cand_offsets,
                       const int* d_cand_ids, int batch, int total_candidates,
                       int max_candidates, int top_k, int* d_selected, int* d_counts,
-                      FailReport fail, hipStream_t stream);
+                      FailReport fail, hipStream_t stream, bool undecided_only = false);
 
 // Fused gather + softmax attention over page lists.  Request r attends over
 // list_ids[start_r .. start_r + count_r): with list_stride > 0, start_r =

@@ -30,8 +30,9 @@ __global__ __launch_bounds__(kWave) void ScoreExactKernel(
     const float* __restrict__ queries, const float* __restrict__ summaries,
     const int* __restrict__ token_counts, int capacity, const int* __restrict__ cand_offsets,
     const int* __restrict__ cand_ids, int total, int E, float scale,
-    float* __restrict__ scores, FailReport fail) {
+    float* __restrict__ scores, const int* __restrict__ only, FailReport fail) {
   const int r = blockIdx.y;
+  if (only != nullptr && only[r] >= 0) return;  // decided without exact scores
   int begin, n;
   if (!RequestRange(cand_offsets, r, total, fail, &begin, &n)) return;
   const int end = begin + n;
@@ -236,9 +237,10 @@ constexpr int kSelectMaxKeys = 8192;  // 64 KiB of LDS
 __global__ __launch_bounds__(256) void SelectTopKKernel(
     const float* __restrict__ scores, const int* __restrict__ cand_offsets,
     const int* __restrict__ cand_ids, int total, int max_candidates, int top_k,
-    int* __restrict__ selected, int* __restrict__ counts, FailReport fail) {
+    int* __restrict__ selected, int* __restrict__ counts, bool undecided_only, FailReport fail) {
   extern __shared__ uint64_t keys[];
   const int r = blockIdx.x;
+  if (undecided_only && counts[r] >= 0) return;
   int begin, n;
   RequestRange(cand_offsets, r, total, fail, &begin, &n);
   if (n > max_candidates) {
@@ -302,6 +304,36 @@ constexpr int kCertMaxKeys = 2048;   // next-pow2 candidates per request
 constexpr int kSelRescoreGroup = 32;  // exact chains per rescore group (lanes of wave 0)
 constexpr int kSelThreads = 1024;    // one compare-exchange per thread per stage at 2048 keys
 
+// One wave: the bucket of a 256-bin histogram that holds the need-th largest
+// key: *s_prefix = prefix with the bucket's 8 bits appended, *s_need the
+// members it still owes, *s_all whether it owes all its keys.
+__device__ __forceinline__ void RadixBucket(const int* hist, uint64_t prefix, int need,
+                                            unsigned long long* s_prefix, int* s_need,
+                                            int* s_all) {
+  const int lane = threadIdx.x & (kWave - 1);
+  // Lane l holds bins 4l .. 4l+3; suffix sums from the top bin down find
+  // the bucket b with sum(bins > b) < need <= sum(bins >= b).
+  const int b0 = 4 * lane;
+  const int c3 = hist[b0 + 3], c2 = hist[b0 + 2], c1 = hist[b0 + 1], c0 = hist[b0];
+  int suffix = c0 + c1 + c2 + c3;  // becomes the sum over lanes >= l
+  for (int o = 1; o < kWave; o <<= 1) {
+    const int other = __shfl_down(suffix, o, kWave);
+    if (lane + o < kWave) suffix += other;
+  }
+  int above = __shfl_down(suffix, 1, kWave);  // sum over lanes > l
+  if (lane == kWave - 1) above = 0;
+  if (suffix >= need && above < need) {
+    int b = b0 + 3;
+    int count = c3;
+    if (above + c3 < need) { above += c3; b = b0 + 2; count = c2;
+      if (above + c2 < need) { above += c2; b = b0 + 1; count = c1;
+        if (above + c1 < need) { above += c1; b = b0; count = c0; } } }
+    *s_prefix = (static_cast<unsigned long long>(prefix) << 8) | static_cast<unsigned>(b);
+    *s_need = need - above;
+    *s_all = count == need - above;
+  }
+}
+
 // Radix select of the kk-th largest 64-bit key among keys[0, n): 8 bits a
 // round from the top, stopping as soon as the boundary bucket holds exactly
 // the members still needed.  On return *shift is the last round's shift,
@@ -313,7 +345,6 @@ __device__ void RadixSelectKth(const uint64_t* keys, int n, int kk, int* hist,
                                unsigned long long* s_prefix, int* s_need, int* s_all,
                                int* shift_out, uint64_t* prefix_out, int* need_out,
                                bool* all_out) {
-  const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
   uint64_t prefix = 0;
   int need = kk;
@@ -330,29 +361,7 @@ __device__ void RadixSelectKth(const uint64_t* keys, int n, int kk, int* hist,
       }
     }
     __syncthreads();
-    if (wave == 0) {
-      // Lane l holds bins 4l .. 4l+3; suffix sums from the top bin down find
-      // the bucket b with sum(bins > b) < need <= sum(bins >= b).
-      const int b0 = 4 * lane;
-      const int c3 = hist[b0 + 3], c2 = hist[b0 + 2], c1 = hist[b0 + 1], c0 = hist[b0];
-      int suffix = c0 + c1 + c2 + c3;  // becomes the sum over lanes >= l
-      for (int o = 1; o < kWave; o <<= 1) {
-        const int other = __shfl_down(suffix, o, kWave);
-        if (lane + o < kWave) suffix += other;
-      }
-      int above = __shfl_down(suffix, 1, kWave);  // sum over lanes > l
-      if (lane == kWave - 1) above = 0;
-      if (suffix >= need && above < need) {
-        int b = b0 + 3;
-        int count = c3;
-        if (above + c3 < need) { above += c3; b = b0 + 2; count = c2;
-          if (above + c2 < need) { above += c2; b = b0 + 1; count = c1;
-            if (above + c1 < need) { above += c1; b = b0; count = c0; } } }
-        *s_prefix = (static_cast<unsigned long long>(prefix) << 8) | static_cast<unsigned>(b);
-        *s_need = need - above;
-        *s_all = count == need - above;
-      }
-    }
+    if (wave == 0) RadixBucket(hist, prefix, need, s_prefix, s_need, s_all);
     __syncthreads();
     prefix = *s_prefix;
     need = *s_need;
@@ -650,6 +659,423 @@ __global__ __launch_bounds__(kSelThreads) void SelectCertifiedKernel(
       scale, top_k, exact_pages, fail);
 }
 
+// A tagged word once it carries `tag` (spin_limit polls, sleeping between),
+// or false.
+__device__ __forceinline__ bool AwaitTagged(unsigned long long* p, unsigned tag,
+                                            unsigned spin_limit, unsigned long long* out) {
+  unsigned long long w = LoadWord(p);
+  for (unsigned i = 0; static_cast<unsigned>(w >> 32) != tag; ++i) {
+    if (i >= spin_limit) return false;
+    __builtin_amdgcn_s_sleep(1);
+    w = LoadWord(p);
+  }
+  *out = w;
+  return true;
+}
+
+// Certified select for 2049 to 8192 candidates per request: a candidate's key
+// and interval stay in the registers of one thread (candidate i in thread
+// i mod 1024) until the set that can still be selected is in LDS, and order
+// and certification then only see that set.  Latency-bound: a request is one
+// workgroup's chain of loads, radix rounds, sort and certification, 14.6 us of
+// one request's 8192 candidates; with 64 selected, whose order some 8 pages'
+// intervals leave open, 24 us (42 us with one thread per member in the sort
+// and certification and the radix rounds run again after the refinement; the
+// same with the refinement in this workgroup 53 us).  It replaces exact
+// chains for every page (154 us for 4 requests of up to 8192 pages) and a
+// bitonic sort of them (165 us): that step took 363 us and takes 140.
+// A request with more than kLargeMaxFlags candidates open (equal pages, a zero
+// query) is left undecided, counts[r] = kUndecided, for the exact score and
+// select kernels that the launch enqueues after this one and that return at
+// once for every other request: chains here take 25 us per 32 candidates.
+constexpr int kLargeMaxKeys = 8192;
+constexpr int kLargeMaxK = 1024;
+constexpr int kLargeMaxFlags = 128;
+constexpr int kUndecided = -1;
+// Flagged pages that the helper workgroups refine: fewer are as quick in the
+// selecting workgroup (no exchange), more go to the exact chains.
+constexpr int kAssistLeastPages = 3;
+constexpr int kAssistMaxPages = 64;
+constexpr int kAssistMaxHelpers = 32;
+constexpr int kAssistLeastCandidates = 256;  // room for the words
+static_assert(1 + 4 * kAssistMaxPages <= 3 * kAssistLeastCandidates, "the words fit");
+static_assert(3 * kAssistMaxPages <= kSelThreads, "a thread per word");
+
+// The candidates that can still be in the top kk: the members (the kk largest
+// midpoints) and the outsiders whose interval reaches the members' smallest
+// lower bound.  Every other outsider's score lies below every member's, so it
+// is out whatever the open intervals hide.
+constexpr int kLargeSet = kLargeMaxK + kLargeMaxFlags;
+struct LargeSet {
+  uint64_t key[kLargeSet];
+  int c[kLargeSet];  // candidate
+  float lo[kLargeSet], hi[kLargeSet];
+};
+struct LargeShared {
+  LargeSet a, b;  // one is sorted into the other
+  int open[kLargeMaxFlags];  // positions whose order is open
+  int flag_c[kLargeMaxFlags];  // a helper's pages
+  float flag_mid[kLargeMaxFlags], flag_lo[kLargeMaxFlags], flag_hi[kLargeMaxFlags];
+  int hist[256];
+  float red[2][kSelThreads / kWave];
+  unsigned long long prefix;
+  int need, all, count, tie, nopen;
+  alignas(16) float tile[RescoreFloats<kSelRescoreGroup>()];
+};
+
+// Threads per element of a loop over `count` elements (a power of two, <= 16).
+__device__ __forceinline__ int LargeParts(int count) {
+  int parts = 16;
+  while (parts > 1 && parts * count > kSelThreads) parts >>= 1;
+  return parts;
+}
+
+// from, sorted by key (descending; equal keys by position), into to: ranks by
+// counting, `parts` threads per element.  Ends with a barrier.
+__device__ void LargeSort(const LargeSet& from, LargeSet& to, int count) {
+  const int parts = LargeParts(count);
+  const int part = threadIdx.x & (parts - 1);
+  for (int base = 0; base < count; base += kSelThreads / parts) {
+    const int t = base + static_cast<int>(threadIdx.x) / parts;
+    const uint64_t k = t < count ? from.key[t] : 0ull;
+    int rank = 0;
+    for (int u0 = part; u0 < count; u0 += 4 * parts) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int u = u0 + v * parts;
+        const uint64_t ku = u < count ? from.key[u] : 0ull;
+        rank += (u < count) & ((ku > k) | ((ku == k) & (u < t)));
+      }
+    }
+    for (int o = 1; o < parts; o <<= 1) rank += __shfl_xor(rank, o, kWave);
+    if (t < count && part == 0) {
+      to.key[rank] = k;
+      to.c[rank] = from.c[t];
+      to.lo[rank] = from.lo[t];
+      to.hi[rank] = from.hi[t];
+    }
+  }
+  __syncthreads();
+}
+
+// The positions of the sorted set whose order among the first kk, or across
+// that line, its intervals leave open: a position below kk whose interval
+// meets any other's, and one from kk on whose interval meets a member's.
+// Appends them to sh.open (sh.nopen counts all of them).  Ends with a barrier.
+__device__ void LargeCertify(LargeShared& sh, const LargeSet& set, int count, int kk) {
+  const int parts = LargeParts(count);
+  const int part = threadIdx.x & (parts - 1);
+  for (int base = 0; base < count; base += kSelThreads / parts) {
+    const int t = base + static_cast<int>(threadIdx.x) / parts;
+    const bool in = t < count;
+    const float l = in ? set.lo[t] : INFINITY;
+    const float h = in ? set.hi[t] : -INFINITY;
+    const int others = t < kk ? count : kk;
+    int open = 0;
+    for (int u0 = part; u0 < others; u0 += 4 * parts) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int u = u0 + v * parts;
+        const float lu = u < others ? set.lo[u] : INFINITY;
+        const float hu = u < others ? set.hi[u] : -INFINITY;
+        open |= (u != t) & (l <= hu) & (lu <= h);
+      }
+    }
+    for (int o = 1; o < parts; o <<= 1) open |= __shfl_xor(open, o, kWave);
+    if (in && open != 0 && part == 0) {
+      const int pos = atomicAdd(&sh.nopen, 1);
+      if (pos < kLargeMaxFlags) sh.open[pos] = t;
+    }
+  }
+  __syncthreads();
+}
+
+// A helper workgroup of a large request's select: once the request's
+// workgroup has published its flagged candidates, refines every helpers-th of
+// them from its first-pass interval and publishes the result.  One workgroup
+// refines a page in 4-6 us with half its waves, and refining 8 to 64 pages in
+// the selecting workgroup, or running their exact chains (25 us a group of 32),
+// is what its time went to while the rest of the chip stood idle.
+__device__ __forceinline__ void LargeAssist(LargeShared& sh, const SelectAssist& assist,
+                                            unsigned long long* words, int index,
+                                            const float* __restrict__ lo,
+                                            const float* __restrict__ hi,
+                                            const float* __restrict__ q,
+                                            const float* __restrict__ summaries,
+                                            const int* __restrict__ token_counts, int capacity,
+                                            const int* __restrict__ cand, int n, int E,
+                                            float scale) {
+  const int tid = threadIdx.x;
+  if (tid == 0) {
+    unsigned long long w = 0;
+    const bool ok = AwaitTagged(words, assist.epoch, assist.spin_limit, &w);
+    const int pages = ok ? static_cast<int>(static_cast<uint32_t>(w)) : 0;
+    sh.nopen = pages <= kAssistMaxPages ? pages : 0;
+    sh.all = 1;
+  }
+  __syncthreads();
+  const int pages = sh.nopen;
+  const int mine = index < pages ? (pages - index + assist.helpers - 1) / assist.helpers : 0;
+  if (mine == 0) return;
+  if (tid < mine) {
+    unsigned long long w = 0;
+    const bool ok = AwaitTagged(words + 1 + index + tid * assist.helpers, assist.epoch,
+                                assist.spin_limit, &w);
+    const int c = static_cast<int>(static_cast<uint32_t>(w));
+    if (!ok || c < 0 || c >= n) {
+      sh.all = 0;
+    } else {
+      sh.flag_c[tid] = c;
+      sh.flag_lo[tid] = lo[c];
+      sh.flag_hi[tid] = hi[c];
+    }
+  }
+  __syncthreads();
+  if (sh.all == 0) return;  // (the request's workgroup gives up waiting, too)
+  RefineScores<kSelThreads>(
+      mine,
+      [&](int f) -> const float* {
+        const int pg = cand[sh.flag_c[f]];
+        const bool live = InPool(pg, capacity) && token_counts[pg] != 0;
+        return live ? summaries + static_cast<size_t>(pg) * E : nullptr;
+      },
+      [&](int f) { return dsd_refine::FirstPassBound(sh.flag_lo[f], sh.flag_hi[f], scale, E); },
+      [&](int f, float m, float l, float h) {
+        unsigned long long* to =
+            words + 1 + kAssistMaxPages + 3 * (index + f * assist.helpers);
+        PutTagged(to, assist.epoch, __float_as_uint(m));
+        PutTagged(to + 1, assist.epoch, __float_as_uint(l));
+        PutTagged(to + 2, assist.epoch, __float_as_uint(h));
+      },
+      q, E, scale, reinterpret_cast<double*>(sh.tile));
+}
+
+template <int PER>
+__global__ __launch_bounds__(kSelThreads) void SelectCertifiedLargeKernel(
+    const float* __restrict__ mid, const float* __restrict__ lo,
+    const float* __restrict__ hi, const float* __restrict__ queries,
+    const float* __restrict__ summaries, const int* __restrict__ token_counts, int capacity,
+    const int* __restrict__ cand_offsets, const int* __restrict__ cand_ids, int batch, int total,
+    int max_candidates, int E, float scale, int top_k, int* __restrict__ selected,
+    int* __restrict__ counts, int* __restrict__ exact_pages, SelectAssist assist,
+    FailReport fail) {
+  static_assert(PER * kSelThreads <= kLargeMaxKeys && PER <= 32, "a member bit per candidate");
+  __shared__ LargeShared sh;
+  const bool helper = static_cast<int>(blockIdx.x) >= batch;
+  const int r = static_cast<int>(blockIdx.x) % batch;
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = tid / kWave;
+  int begin, n;
+  RequestRange(cand_offsets, r, total, helper ? FailReport{} : fail, &begin, &n);
+  if (n > max_candidates || n > PER * kSelThreads) {
+    // Only max_candidates were scored: select nothing and report it.
+    if (tid == 0 && !helper) ReportFailure(fail, kFailShape);
+    n = 0;
+  }
+  const int kk = top_k <= 0 ? 0 : (top_k < n ? top_k : n);
+  const int* cand = cand_ids + begin;
+  // The request's assist words lie in its candidates' publication words
+  // (idle in this step form): [0] the pages to refine, [1 ..] which
+  // candidates, then three words of interval per page.
+  const bool assisted = assist.helpers > 0 && n > kAssistLeastCandidates;
+  unsigned long long* words = assisted ? assist.words + 3 * static_cast<size_t>(begin) : nullptr;
+  if (helper) {
+    if (kk > 0 && assisted) {
+      LargeAssist(sh, assist, words, (static_cast<int>(blockIdx.x) - batch) / batch, lo + begin,
+                  hi + begin, queries + static_cast<size_t>(r) * E, summaries, token_counts,
+                  capacity, cand, n, E, scale);
+    }
+    return;
+  }
+  if (kk == 0) {
+    if (tid == 0) counts[r] = 0;
+    return;
+  }
+  uint64_t key[PER];
+  float clo[PER], chi[PER];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int i = tid + kSelThreads * j;
+    key[j] = 0;
+    clo[j] = INFINITY;
+    chi[j] = -INFINITY;
+    if (i < n) {
+      key[j] = SelectKey(mid[begin + i], cand[i]);
+      clo[j] = lo[begin + i];
+      chi[j] = hi[begin + i];
+    }
+  }
+  if (tid == 0) {
+    sh.count = 0;
+    sh.tie = 0;
+    sh.nopen = 0;
+  }
+  const float* q = queries + static_cast<size_t>(r) * E;
+  // 1. The kk-th largest key, 8 bits a round (RadixSelectKth).
+  uint64_t prefix = 0;
+  int need = kk;
+  int shift = 56;
+  bool all = false;
+  for (int round = 0; round < 8 && !all; ++round) {
+    shift = 56 - 8 * round;
+    if (tid < 256) sh.hist[tid] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const bool in = tid + kSelThreads * j < n &&
+                      (round == 0 || (key[j] >> (shift + 8)) == prefix);
+      if (in) atomicAdd(&sh.hist[static_cast<int>((key[j] >> shift) & 255u)], 1);
+    }
+    __syncthreads();
+    if (wave == 0) {
+      RadixBucket(sh.hist, prefix, need, &sh.prefix, &sh.need, &sh.all);
+    }
+    __syncthreads();
+    prefix = sh.prefix;
+    need = sh.need;
+    all = sh.all != 0;
+  }
+  // 2. The set: the members, then the outsiders that reach them.
+  unsigned members = 0;
+  float my_min = INFINITY;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int i = tid + kSelThreads * j;
+    const uint64_t top = key[j] >> shift;
+    bool in = i < n && top > prefix;
+    if (i < n && top == prefix) in = all || atomicAdd(&sh.tie, 1) < need;
+    if (in) {
+      members |= 1u << j;
+      const int pos = atomicAdd(&sh.count, 1);
+      sh.a.key[pos] = key[j];
+      sh.a.c[pos] = i;
+      sh.a.lo[pos] = clo[j];
+      sh.a.hi[pos] = chi[j];
+      my_min = fminf(my_min, clo[j]);
+    }
+  }
+  for (int o = 1; o < kWave; o <<= 1) my_min = fminf(my_min, __shfl_xor(my_min, o, kWave));
+  if (lane == 0) sh.red[0][wave] = my_min;
+  __syncthreads();
+  float min_t_lo = INFINITY;
+  for (int w = 0; w < kSelThreads / kWave; ++w) min_t_lo = fminf(min_t_lo, sh.red[0][w]);
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int i = tid + kSelThreads * j;
+    if (i < n && !((members >> j) & 1u) && chi[j] >= min_t_lo) {
+      const int pos = atomicAdd(&sh.count, 1);
+      if (pos < kk + kLargeMaxFlags) {
+        sh.a.key[pos] = key[j];
+        sh.a.c[pos] = i;
+        sh.a.lo[pos] = clo[j];
+        sh.a.hi[pos] = chi[j];
+      }
+    }
+  }
+  __syncthreads();
+  const int count = sh.count;
+  const bool too_many = count > kk + kLargeMaxFlags;
+  // 3. Their order, and what the first-pass intervals leave open.  (A member
+  //    that meets an outsider meets one of the set.)
+  if (!too_many) {
+    LargeSort(sh.a, sh.b, count);
+    LargeCertify(sh, sh.b, count, kk);
+  }
+  int nopen = too_many ? kLargeMaxFlags + 1 : sh.nopen;
+  const bool refine = E % 256 == 0 && nopen > 0;
+  const bool share =
+      refine && assisted && nopen >= kAssistLeastPages && nopen <= kAssistMaxPages;
+  if (assisted) {
+    // The helpers' share (0: they leave).
+    if (tid < (share ? nopen : 0)) {
+      PutTagged(words + 1 + tid, assist.epoch, static_cast<uint32_t>(sh.b.c[sh.open[tid]]));
+    }
+    if (tid == 0) {
+      PutTagged(words, assist.epoch, static_cast<uint32_t>(share ? nopen : 0));
+    }
+  }
+  if (nopen > kLargeMaxFlags) {
+    if (tid == 0) counts[r] = kUndecided;
+    return;
+  }
+  LargeSet* order = &sh.b;
+  if (share || (refine && RefineWorthwhile<kSelThreads>(nopen))) {
+    // 4. Refined intervals of the open positions (sh.flag_*), by the helpers
+    //    or here, and the set's order again.  A wait that gives up leaves the
+    //    first-pass intervals, which are sound, to the exact chains.
+    if (tid == 0) sh.all = 1;
+    __syncthreads();
+    if (share) {
+      // Thread 3f + x: word x of open position f's interval.
+      if (tid < 3 * nopen) {
+        unsigned long long w = 0;
+        if (AwaitTagged(words + 1 + kAssistMaxPages + tid, assist.epoch, assist.spin_limit, &w)) {
+          float* to = tid % 3 == 0 ? sh.flag_mid : (tid % 3 == 1 ? sh.flag_lo : sh.flag_hi);
+          to[tid / 3] = __uint_as_float(static_cast<uint32_t>(w));
+        } else {
+          sh.all = 0;
+        }
+      }
+      __syncthreads();
+    } else {
+      RefineScores<kSelThreads>(
+          nopen,
+          [&](int f) -> const float* {
+            const int pg = cand[sh.b.c[sh.open[f]]];
+            const bool live = InPool(pg, capacity) && token_counts[pg] != 0;
+            return live ? summaries + static_cast<size_t>(pg) * E : nullptr;
+          },
+          [&](int f) {
+            const int t = sh.open[f];
+            return dsd_refine::FirstPassBound(sh.b.lo[t], sh.b.hi[t], scale, E);
+          },
+          [&](int f, float m, float l, float h) {
+            sh.flag_mid[f] = m;
+            sh.flag_lo[f] = l;
+            sh.flag_hi[f] = h;
+          },
+          q, E, scale, reinterpret_cast<double*>(sh.tile));
+    }
+    if (sh.all != 0) {
+      if (tid < nopen) {
+        const int t = sh.open[tid];
+        sh.b.key[t] = SelectKey(sh.flag_mid[tid], cand[sh.b.c[t]]);
+        sh.b.lo[t] = sh.flag_lo[tid];
+        sh.b.hi[t] = sh.flag_hi[tid];
+      }
+      if (tid == 0) sh.nopen = 0;
+      __syncthreads();
+      LargeSort(sh.b, sh.a, count);
+      LargeCertify(sh, sh.a, count, kk);
+      order = &sh.a;
+      nopen = sh.nopen;
+      if (nopen > kLargeMaxFlags) {
+        if (tid == 0) counts[r] = kUndecided;
+        return;
+      }
+    }
+  }
+  if (nopen > 0) {
+    // 5. Exact chains for what is still open, and the order once more.
+    if (tid == 0 && exact_pages != nullptr) atomicAdd(exact_pages, nopen);
+    LargeSet& set = *order;
+    RescoreChains<kSelRescoreGroup, kSelThreads>(
+        nopen, [&](int f) { return cand[set.c[sh.open[f]]]; },
+        [&](int f, float score) {
+          const int t = sh.open[f];
+          set.key[t] = SelectKey(score, cand[set.c[t]]);
+        },
+        q, summaries, token_counts, capacity, E, scale, sh.tile);
+    LargeSet* other = order == &sh.a ? &sh.b : &sh.a;
+    LargeSort(set, *other, count);
+    order = other;
+  }
+  int* out = selected + static_cast<size_t>(r) * top_k;
+  for (int i = tid; i < kk; i += kSelThreads) out[i] = KeyPage(order->key[i]);
+  if (tid == 0) counts[r] = kk;
+}
+
 // Certified select for up to 256 candidates per request: thread i owns
 // candidate i and finds its rank by counting larger keys (broadcast LDS reads,
 // no barrier chain), ties broken by position so ranks are distinct.
@@ -863,20 +1289,6 @@ struct WideShared {
   unsigned long long stamp[3];  // timing mode: start, select start and end
 };
 
-// A tagged word once it carries `tag` (spin_limit polls, sleeping between),
-// or false.
-__device__ __forceinline__ bool AwaitTagged(unsigned long long* p, unsigned tag,
-                                            unsigned spin_limit, unsigned long long* out) {
-  unsigned long long w = LoadWord(p);
-  for (unsigned i = 0; static_cast<unsigned>(w >> 32) != tag; ++i) {
-    if (i >= spin_limit) return false;
-    __builtin_amdgcn_s_sleep(1);
-    w = LoadWord(p);
-  }
-  *out = w;
-  return true;
-}
-
 // Item i's kind (0 score slice, 1 attention), request and slice or head:
 // request r's G slices, then (for r >= lag) request r - lag's Q heads,
 // request by request; after the last request the remaining lag requests'
@@ -1076,28 +1488,31 @@ __global__ __launch_bounds__(kFThreads) void WideStepKernel(PoolView pool, WideA
 void LaunchScoreExact(const PoolView& pool, const float* d_queries,
                       const int* d_cand_offsets, const int* d_cand_ids,
                       int batch, int total_candidates, int max_candidates, float scale,
-                      float* d_scores, FailReport fail, hipStream_t stream) {
+                      float* d_scores, FailReport fail, hipStream_t stream,
+                      const int* d_undecided) {
   if (batch <= 0 || max_candidates <= 0) return;
   const dim3 grid((max_candidates + kWave - 1) / kWave, batch);
   if (pool.elements % 4 == 0) {
     hipLaunchKernelGGL(ScoreExactKernel<true>, grid, dim3(kWave), 0, stream,
                        d_queries, pool.summaries, pool.token_counts, pool.capacity,
                        d_cand_offsets, d_cand_ids, total_candidates, pool.elements, scale,
-                       d_scores, fail);
+                       d_scores, d_undecided, fail);
   } else {
     hipLaunchKernelGGL(ScoreExactKernel<false>, grid, dim3(kWave), 0, stream,
                        d_queries, pool.summaries, pool.token_counts, pool.capacity,
                        d_cand_offsets, d_cand_ids, total_candidates, pool.elements, scale,
-                       d_scores, fail);
+                       d_scores, d_undecided, fail);
   }
   DSD_HIP_CHECK(hipGetLastError());
 }
 
-bool CertifiedScoringSupported(int elements, int max_candidates) {
-  int m = 1;
-  while (m < max_candidates) m <<= 1;
-  return elements % kWave == 0 && elements >= kWave && m <= kCertMaxKeys;
+bool CertifiedScoringSupported(int elements, int max_candidates, int top_k) {
+  if (elements % kWave != 0 || elements < kWave) return false;
+  if (max_candidates <= kCertMaxKeys) return true;
+  return max_candidates <= kLargeMaxKeys && top_k <= kLargeMaxK;
 }
+
+bool CertifiedSelectMayDefer(int max_candidates) { return max_candidates > kCertMaxKeys; }
 
 void LaunchScoreBounds(const PoolView& pool, const float* d_queries,
                        const int* d_cand_offsets, const int* d_cand_ids, int batch,
@@ -1142,7 +1557,7 @@ void LaunchSelectCertified(const PoolView& pool, const float* d_mid, const float
                            const int* d_cand_offsets, const int* d_cand_ids, int batch,
                            int total_candidates, int max_candidates, float scale, int top_k,
                            int* d_selected, int* d_counts, int* d_exact_pages, FailReport fail,
-                           hipStream_t stream) {
+                           hipStream_t stream, const SelectAssist& assist) {
   if (batch <= 0) return;
   if (max_candidates <= kRankMax) {
     // Always four waves: three of them form products while wave 0 runs the
@@ -1155,14 +1570,32 @@ void LaunchSelectCertified(const PoolView& pool, const float* d_mid, const float
     DSD_HIP_CHECK(hipGetLastError());
     return;
   }
-  int m = 1;
-  while (m < max_candidates) m <<= 1;
-  if (m > kCertMaxKeys) {
-    throw std::invalid_argument("certified select supports up to " +
-                                std::to_string(kCertMaxKeys) + " candidates per request");
-  }
   if (pool.elements % kWave != 0) {
     throw std::invalid_argument("certified select needs E % 64 == 0");
+  }
+  if (max_candidates > kCertMaxKeys) {
+    if (max_candidates > kLargeMaxKeys || top_k > kLargeMaxK) {
+      throw std::invalid_argument("certified select supports up to " +
+                                  std::to_string(kLargeMaxKeys) + " candidates per request and " +
+                                  std::to_string(kLargeMaxK) + " of them selected");
+    }
+    const auto kernel = max_candidates <= kLargeMaxKeys / 2
+                            ? SelectCertifiedLargeKernel<kLargeMaxKeys / 2 / kSelThreads>
+                            : SelectCertifiedLargeKernel<kLargeMaxKeys / kSelThreads>;
+    // Helpers only where every workgroup is resident at once, so that a
+    // request's workgroup and its helpers do run side by side (one that does
+    // not run in time costs the bounded wait, nothing else).
+    SelectAssist a = assist;
+    a.helpers = a.words == nullptr || a.epoch == 0
+                    ? 0
+                    : std::min(kAssistMaxHelpers, a.compute_units / batch - 1);
+    if (a.helpers < kAssistLeastPages) a.helpers = 0;
+    hipLaunchKernelGGL(kernel, dim3(batch * (1 + a.helpers)), dim3(kSelThreads), 0, stream, d_mid,
+                       d_lo, d_hi, d_queries, pool.summaries, pool.token_counts, pool.capacity,
+                       d_cand_offsets, d_cand_ids, batch, total_candidates, max_candidates,
+                       pool.elements, scale, top_k, d_selected, d_counts, d_exact_pages, a, fail);
+    DSD_HIP_CHECK(hipGetLastError());
+    return;
   }
   hipLaunchKernelGGL(SelectCertifiedKernel, dim3(batch), dim3(kSelThreads), 0, stream, d_mid,
                      d_lo, d_hi, d_queries, pool.summaries, pool.token_counts, pool.capacity,
@@ -1223,7 +1656,7 @@ void LaunchWideStep(const PoolView& pool, const WideArgs& w, hipStream_t stream)
 void LaunchSelectTopK(const float* d_scores, const int* d_cand_offsets,
                       const int* d_cand_ids, int batch, int total_candidates,
                       int max_candidates, int top_k, int* d_selected, int* d_counts,
-                      FailReport fail, hipStream_t stream) {
+                      FailReport fail, hipStream_t stream, bool undecided_only) {
   if (batch <= 0) return;
   int m = 1;
   while (m < max_candidates) m <<= 1;
@@ -1238,7 +1671,7 @@ void LaunchSelectTopK(const float* d_scores, const int* d_cand_offsets,
   hipLaunchKernelGGL(SelectTopKKernel, dim3(batch), dim3(threads),
                      sizeof(uint64_t) * static_cast<size_t>(m), stream, d_scores,
                      d_cand_offsets, d_cand_ids, total_candidates, max_candidates, top_k,
-                     d_selected, d_counts, fail);
+                     d_selected, d_counts, undecided_only, fail);
   DSD_HIP_CHECK(hipGetLastError());
 }
 
