@@ -288,21 +288,45 @@ __global__ __launch_bounds__(256) void SelectTopKKernel(
 }
 
 // ---------------------------------------------------------------------------
-// 2b. Certified top-k select.
+// 2b. Certified top-k select (257 to 8192 candidates per request; up to 256:
+// SelectCertifiedRankKernel below).
 //
-// Candidates are sorted by (interval midpoint desc, id asc).  With T the
+// Candidates are ordered by (interval midpoint desc, id asc).  With T the
 // first k, a candidate needs its exact score only if its interval overlaps
 // another relevant one: an outsider whose hi reaches min(lo over T), or a
 // member of T whose interval meets an outsider's or another member's.  Every
 // other comparison is already decided by disjoint intervals, so replacing the
-// flagged candidates' keys by their exact scores and sorting again yields the
-// reference order exactly.  Exact scores come from the reference's sequential
-// chain (RescoreChains: the lanes of wave 0 run the dependent adds of up to
-// 32 pages while the other waves form the next stretch of products).
+// open candidates' keys by their exact scores and sorting again yields the
+// reference order exactly.  Before that the open candidates get refined
+// intervals (RefineScores), which usually decide them.  Exact scores come from
+// the reference's sequential chain (RescoreChains: the lanes of wave 0 run the
+// dependent adds of up to 32 pages while the other waves form the next stretch
+// of products).
+//
+// One request is one workgroup's chain of loads, radix rounds, sort and
+// certification, so it is latency-bound.  A candidate's key and interval stay
+// in the registers of one thread (candidate i in thread i mod 1024) until the
+// set that can still be selected is in LDS, and order and certification then
+// only see that set, several threads per element.  8192 candidates of one
+// request take 14.6 us with one selected; with 64, whose order some 8 pages'
+// intervals leave open, 24 us (42 us with one thread per member in the sort and
+// the certification and the radix rounds run again after the refinement).
+// Beyond 2048 candidates this replaces exact chains for every page (154 us for
+// 4 requests of up to 8192 pages) and a bitonic sort of them (165 us): that
+// step took 363 us and takes 137.  Up to 2048 candidates it replaces a select
+// that kept every candidate in LDS and gave each member one thread (32 requests
+// of 8 x 128 heads, 300 pages each: the step 50 us, now 45.5; the wide step of
+// one request of 2048 pages, 64 selected: 71 us, now 59).
+//
+// Beyond 2048 candidates LDS holds kLargeMaxK members and kLargeMaxOpen open
+// candidates: a request with more open (equal pages, a zero query) is left
+// undecided, counts[r] = kUndecided, for the exact score and select kernels
+// that the launch enqueues after this one and that return at once for every
+// other request; chains here take 25 us per 32 candidates.
 // ---------------------------------------------------------------------------
-constexpr int kCertMaxKeys = 2048;   // next-pow2 candidates per request
+constexpr int kCertMaxKeys = 2048;    // candidates per request with no bound on the open ones
 constexpr int kSelRescoreGroup = 32;  // exact chains per rescore group (lanes of wave 0)
-constexpr int kSelThreads = 1024;    // one compare-exchange per thread per stage at 2048 keys
+constexpr int kSelThreads = 1024;
 
 // One wave: the bucket of a 256-bin histogram that holds the need-th largest
 // key: *s_prefix = prefix with the bucket's 8 bits appended, *s_need the
@@ -334,331 +358,6 @@ __device__ __forceinline__ void RadixBucket(const int* hist, uint64_t prefix, in
   }
 }
 
-// Radix select of the kk-th largest 64-bit key among keys[0, n): 8 bits a
-// round from the top, stopping as soon as the boundary bucket holds exactly
-// the members still needed.  On return *shift is the last round's shift,
-// *prefix the kept bucket's key bits above it, *need how many keys of that
-// bucket are members and *all whether they all are (need == bucket size).
-// Keys above the bucket (key >> shift > prefix) are members.  Whole
-// workgroup; hist is 256 ints of LDS.
-__device__ void RadixSelectKth(const uint64_t* keys, int n, int kk, int* hist,
-                               unsigned long long* s_prefix, int* s_need, int* s_all,
-                               int* shift_out, uint64_t* prefix_out, int* need_out,
-                               bool* all_out) {
-  const int wave = threadIdx.x / kWave;
-  uint64_t prefix = 0;
-  int need = kk;
-  int shift = 56;
-  bool all = false;
-  for (int round = 0; round < 8; ++round) {
-    shift = 56 - 8 * round;
-    for (int b = threadIdx.x; b < 256; b += kSelThreads) hist[b] = 0;
-    __syncthreads();
-    for (int i = threadIdx.x; i < n; i += kSelThreads) {
-      const uint64_t key = keys[i];
-      if (round == 0 || (key >> (shift + 8)) == prefix) {
-        atomicAdd(&hist[static_cast<int>((key >> shift) & 255u)], 1);
-      }
-    }
-    __syncthreads();
-    if (wave == 0) RadixBucket(hist, prefix, need, s_prefix, s_need, s_all);
-    __syncthreads();
-    prefix = *s_prefix;
-    need = *s_need;
-    all = *s_all != 0;
-    __syncthreads();  // the next round rewrites hist and the shared words
-    if (all) break;
-  }
-  *shift_out = shift;
-  *prefix_out = prefix;
-  *need_out = need;
-  *all_out = all;
-}
-
-// (key, idx) pairs [0, count) into out_keys / out_idx in descending key
-// order, by counting: rank(i) = #{j : key_j > key_i} + #{j < i : key_j ==
-// key_i} (a permutation even with equal keys).  Cheaper than a bitonic sort
-// for the few dozen members (no stage chain); O(count^2) work in all.  Whole
-// workgroup; the outputs are complete after the closing barrier.
-__device__ void RankSortDesc(const uint64_t* keys, const int* idx, int count,
-                             uint64_t* out_keys, int* out_idx) {
-  for (int i = threadIdx.x; i < count; i += kSelThreads) {
-    const uint64_t key = keys[i];
-    int rank = 0;
-    int j = 0;
-    for (; j + 8 <= count; j += 8) {
-      uint64_t kj[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) kj[u] = keys[j + u];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) rank += (kj[u] > key) | ((kj[u] == key) & (j + u < i));
-    }
-    for (; j < count; ++j) {
-      const uint64_t kj = keys[j];
-      rank += (kj > key) | ((kj == key) & (j < i));
-    }
-    out_keys[rank] = key;
-    out_idx[rank] = idx[i];
-  }
-  __syncthreads();
-}
-
-// The LDS of one request's certified select (kSelThreads threads).
-struct CertShared {
-  uint64_t keys[kCertMaxKeys];   // by candidate
-  float s_lo[kCertMaxKeys];
-  float s_hi[kCertMaxKeys];
-  uint8_t member[kCertMaxKeys];  // by candidate
-  uint64_t skeys[kCertMaxKeys];  // the members, then the final set, sorted
-  int sidx[kCertMaxKeys];
-  int flagged[kCertMaxKeys];
-  int hist[256];
-  alignas(16) float tile[RescoreFloats<kSelRescoreGroup>()];
-  float s_red[2][kSelThreads / kWave];
-  unsigned long long s_prefix;
-  int s_need, s_all, s_count, s_tie, s_nflag, s_bad;
-};
-
-// Request r's certified top-k (up to kCertMaxKeys candidates, the whole
-// workgroup of kSelThreads threads).  load(c, &mid, &lo, &hi) gives candidate
-// c's first-pass interval (c indexes the batch's CSR); with kPolled it may
-// report that an interval never became readable (false), and the request
-// then selects nothing (kFailWait).  emit(i, page) writes member i of the
-// selection (rank order), emit_count(kk) the count; emit_count runs once, in
-// thread 0, after the emits.
-template <bool kPolled, class Load, class Emit, class EmitCount>
-__device__ __forceinline__ void SelectCertifiedRequest(
-    CertShared& sh, int r, Load load, Emit emit, EmitCount emit_count,
-    const float* __restrict__ queries, const float* __restrict__ summaries,
-    const int* __restrict__ token_counts, int capacity, const int* __restrict__ cand_offsets,
-    const int* __restrict__ cand_ids, int total, int max_candidates, int E, float scale,
-    int top_k, int* __restrict__ exact_pages, FailReport fail) {
-  uint64_t* keys = sh.keys;
-  float* s_lo = sh.s_lo;
-  float* s_hi = sh.s_hi;
-  uint8_t* member = sh.member;
-  uint64_t* skeys = sh.skeys;
-  int* sidx = sh.sidx;
-  int* flagged = sh.flagged;
-  int* hist = sh.hist;
-  float* tile = sh.tile;
-  float (&s_red)[2][kSelThreads / kWave] = sh.s_red;
-  unsigned long long& s_prefix = sh.s_prefix;
-  int& s_need = sh.s_need;
-  int& s_all = sh.s_all;
-  int& s_count = sh.s_count;
-  int& s_tie = sh.s_tie;
-  int& s_nflag = sh.s_nflag;
-  int begin, n;
-  RequestRange(cand_offsets, r, total, fail, &begin, &n);
-  if (n > max_candidates || n > kCertMaxKeys) {
-    // Only max_candidates were scored (and this kernel holds kCertMaxKeys):
-    // select nothing and report it.
-    if (threadIdx.x == 0) ReportFailure(fail, kFailShape);
-    n = 0;
-  }
-  const int kk = top_k <= 0 ? 0 : (top_k < n ? top_k : n);
-  if (kk == 0) {
-    if (threadIdx.x == 0) emit_count(0);
-    return;
-  }
-  const int* cand = cand_ids + begin;
-  if constexpr (kPolled) {
-    if (threadIdx.x == 0) sh.s_bad = 0;
-    __syncthreads();
-  }
-  for (int i = threadIdx.x; i < n; i += kSelThreads) {
-    float m, l, h;
-    if (!load(begin + i, &m, &l, &h)) sh.s_bad = 1;
-    keys[i] = SelectKey(m, cand[i]);
-    s_lo[i] = l;
-    s_hi[i] = h;
-  }
-  if (threadIdx.x == 0) {
-    s_count = 0;
-    s_tie = 0;
-    s_nflag = 0;
-  }
-  __syncthreads();
-  if constexpr (kPolled) {
-    if (sh.s_bad != 0) {
-      if (threadIdx.x == 0) {
-        ReportFailure(fail, kFailWait);
-        emit_count(0);
-      }
-      return;
-    }
-  }
-
-  const int wave = threadIdx.x / kWave;
-  constexpr int nwaves = kSelThreads / kWave;
-  uint64_t* tkeys = reinterpret_cast<uint64_t*>(tile);
-  int* tidx = reinterpret_cast<int*>(tile + 2 * kCertMaxKeys);
-  // Pass 0 certifies with the score kernel's intervals; the candidates it
-  // flags get refined intervals (RefineScores, several waves per page; E a
-  // multiple of 256) and pass 1 selects and certifies again.  What pass 1
-  // leaves open gets the exact chain (step 3).
-  for (int pass = 0; pass < 2; ++pass) {
-    // 1. The members: the kk largest keys (equal keys are the same page listed
-    //    twice, so which of them counts is immaterial).
-    int shift;
-    uint64_t prefix;
-    int need;
-    bool all;
-    RadixSelectKth(keys, n, kk, hist, &s_prefix, &s_need, &s_all, &shift, &prefix, &need, &all);
-    // The members, unordered, into the rescoring tile (idle until step 3),
-    // then in key order into skeys / sidx.
-    for (int i = threadIdx.x; i < n; i += kSelThreads) {
-      const uint64_t top = keys[i] >> shift;
-      bool in = top > prefix;
-      if (top == prefix) in = all || atomicAdd(&s_tie, 1) < need;
-      member[i] = in ? 1 : 0;
-      if (in) {
-        const int pos = atomicAdd(&s_count, 1);
-        tkeys[pos] = keys[i];
-        tidx[pos] = i;
-      }
-    }
-    __syncthreads();
-    RankSortDesc(tkeys, tidx, kk, skeys, sidx);
-
-    // 2. Certification.  Member intervals in rank order go to the rescoring
-    //    tile (idle until step 3): mlo = tile[0, kk), mhi = tile[kk, 2kk).
-    float* mlo = tile;
-    float* mhi = tile + kCertMaxKeys;
-    float my_min = INFINITY, my_max = -INFINITY;
-    for (int t = threadIdx.x; t < kk; t += kSelThreads) {
-      const int c = sidx[t];
-      mlo[t] = s_lo[c];
-      mhi[t] = s_hi[c];
-      my_min = fminf(my_min, s_lo[c]);
-    }
-    for (int i = threadIdx.x; i < n; i += kSelThreads) {
-      if (!member[i]) my_max = fmaxf(my_max, s_hi[i]);
-    }
-    for (int o = 1; o < kWave; o <<= 1) {
-      my_min = fminf(my_min, __shfl_xor(my_min, o, kWave));
-      my_max = fmaxf(my_max, __shfl_xor(my_max, o, kWave));
-    }
-    if ((threadIdx.x & (kWave - 1)) == 0) {
-      s_red[0][wave] = my_min;
-      s_red[1][wave] = my_max;
-    }
-    __syncthreads();
-    float min_t_lo = INFINITY, max_o_hi = -INFINITY;
-    for (int w = 0; w < nwaves; ++w) {
-      min_t_lo = fminf(min_t_lo, s_red[0][w]);
-      max_o_hi = fmaxf(max_o_hi, s_red[1][w]);
-    }
-    // An outsider is flagged when its hi reaches the members' smallest lo; a
-    // member when its lo reaches the outsiders' largest hi or its interval
-    // meets another member's.
-    for (int i = threadIdx.x; i < n; i += kSelThreads) {
-      if (!member[i] && s_hi[i] >= min_t_lo) flagged[atomicAdd(&s_nflag, 1)] = i;
-    }
-    for (int t = threadIdx.x; t < kk; t += kSelThreads) {
-      const float l = mlo[t];
-      const float h = mhi[t];
-      bool flag = l <= max_o_hi;
-      // Eight independent reads per round (an early exit would serialise them).
-      for (int u0 = 0; u0 < kk && !flag; u0 += 8) {
-  #pragma unroll
-        for (int v = 0; v < 8; ++v) {
-          const int u = u0 + v;
-          const bool in = u < kk;
-          const float lu = in ? mlo[u] : INFINITY;
-          const float hu = in ? mhi[u] : -INFINITY;
-          flag |= (u != t) & (l <= hu) & (lu <= h);
-        }
-      }
-      if (flag) flagged[atomicAdd(&s_nflag, 1)] = sidx[t];
-    }
-    __syncthreads();
-    if (s_nflag == 0 || pass == 1 || E % 256 != 0 || !RefineWorthwhile<kSelThreads>(s_nflag)) break;
-    RefineScores<kSelThreads>(
-        s_nflag,
-        [&](int f) -> const float* {
-          const int pg = cand[flagged[f]];
-          const bool live = pg >= 0 && pg < capacity && token_counts[pg] != 0;
-          return live ? summaries + static_cast<size_t>(pg) * E : nullptr;
-        },
-        [&](int f) {
-          const int c = flagged[f];
-          return dsd_refine::FirstPassBound(s_lo[c], s_hi[c], scale, E);
-        },
-        [&](int f, float m, float l, float h) {
-          const int c = flagged[f];
-          // LDS only: the global intervals stay the score kernel's
-          // first-pass ones, which a later select over the same buffers
-          // (a stage replay) needs for FirstPassBound's precondition.
-          keys[c] = SelectKey(m, cand[c]);
-          s_lo[c] = l;
-          s_hi[c] = h;
-        },
-        queries + static_cast<size_t>(r) * E, E, scale, reinterpret_cast<double*>(tile));
-    if (threadIdx.x == 0) {
-      s_count = 0;
-      s_tie = 0;
-      s_nflag = 0;
-    }
-    __syncthreads();
-  }
-  const int nflag = s_nflag;
-  if (nflag > 0) {
-    // 3. Exact chains for the flagged candidates, then the final order over
-    //    the members and the flagged outsiders: every other outsider's hi
-    //    is below every member's lo, so it cannot enter the top kk.
-    if (threadIdx.x == 0 && exact_pages != nullptr) atomicAdd(exact_pages, nflag);
-    RescoreChains<kSelRescoreGroup, kSelThreads>(
-        nflag, [&](int f) { return cand[flagged[f]]; },
-        [&](int f, float score) {
-          const int c = flagged[f];
-          keys[c] = SelectKey(score, cand[c]);
-        },
-        queries + static_cast<size_t>(r) * E, summaries, token_counts, capacity, E, scale, tile);
-    if (threadIdx.x == 0) s_count = kk;
-    __syncthreads();
-    for (int t = threadIdx.x; t < kk; t += kSelThreads) skeys[t] = keys[sidx[t]];
-    for (int f = threadIdx.x; f < nflag; f += kSelThreads) {
-      const int c = flagged[f];
-      if (!member[c]) {
-        const int pos = atomicAdd(&s_count, 1);
-        skeys[pos] = keys[c];
-        sidx[pos] = c;
-      }
-    }
-    __syncthreads();
-    RankSortDesc(skeys, sidx, s_count, tkeys, tidx);
-  }
-  const uint64_t* final_keys = nflag > 0 ? tkeys : skeys;
-  for (int i = threadIdx.x; i < kk; i += kSelThreads) emit(i, KeyPage(final_keys[i]));
-  if constexpr (kPolled) __syncthreads();  // every member out before the count
-  if (threadIdx.x == 0) emit_count(kk);
-}
-
-__global__ __launch_bounds__(kSelThreads) void SelectCertifiedKernel(
-    const float* __restrict__ mid, const float* __restrict__ lo,
-    const float* __restrict__ hi, const float* __restrict__ queries,
-    const float* __restrict__ summaries, const int* __restrict__ token_counts, int capacity,
-    const int* __restrict__ cand_offsets, const int* __restrict__ cand_ids, int total,
-    int max_candidates, int E, float scale, int top_k, int* __restrict__ selected,
-    int* __restrict__ counts, int* __restrict__ exact_pages, FailReport fail) {
-  __shared__ CertShared sh;
-  const int r = blockIdx.x;
-  int* out = selected + static_cast<size_t>(r) * top_k;
-  SelectCertifiedRequest<false>(
-      sh, r,
-      [&](int c, float* m, float* l, float* h) {
-        *m = mid[c];
-        *l = lo[c];
-        *h = hi[c];
-        return true;
-      },
-      [&](int i, int page) { out[i] = page; }, [&](int kk) { counts[r] = kk; }, queries,
-      summaries, token_counts, capacity, cand_offsets, cand_ids, total, max_candidates, E,
-      scale, top_k, exact_pages, fail);
-}
-
 // A tagged word once it carries `tag` (spin_limit polls, sleeping between),
 // or false.
 __device__ __forceinline__ bool AwaitTagged(unsigned long long* p, unsigned tag,
@@ -673,24 +372,9 @@ __device__ __forceinline__ bool AwaitTagged(unsigned long long* p, unsigned tag,
   return true;
 }
 
-// Certified select for 2049 to 8192 candidates per request: a candidate's key
-// and interval stay in the registers of one thread (candidate i in thread
-// i mod 1024) until the set that can still be selected is in LDS, and order
-// and certification then only see that set.  Latency-bound: a request is one
-// workgroup's chain of loads, radix rounds, sort and certification, 14.6 us of
-// one request's 8192 candidates; with 64 selected, whose order some 8 pages'
-// intervals leave open, 24 us (42 us with one thread per member in the sort
-// and certification and the radix rounds run again after the refinement; the
-// same with the refinement in this workgroup 53 us).  It replaces exact
-// chains for every page (154 us for 4 requests of up to 8192 pages) and a
-// bitonic sort of them (165 us): that step took 363 us and takes 140.
-// A request with more than kLargeMaxFlags candidates open (equal pages, a zero
-// query) is left undecided, counts[r] = kUndecided, for the exact score and
-// select kernels that the launch enqueues after this one and that return at
-// once for every other request: chains here take 25 us per 32 candidates.
 constexpr int kLargeMaxKeys = 8192;
 constexpr int kLargeMaxK = 1024;
-constexpr int kLargeMaxFlags = 128;
+constexpr int kLargeMaxOpen = 128;
 constexpr int kUndecided = -1;
 // Flagged pages that the helper workgroups refine: fewer are as quick in the
 // selecting workgroup (no exchange), more go to the exact chains.
@@ -705,26 +389,33 @@ static_assert(3 * kAssistMaxPages <= kSelThreads, "a thread per word");
 // midpoints) and the outsiders whose interval reaches the members' smallest
 // lower bound.  Every other outsider's score lies below every member's, so it
 // is out whatever the open intervals hide.
-constexpr int kLargeSet = kLargeMaxK + kLargeMaxFlags;
-struct LargeSet {
-  uint64_t key[kLargeSet];
-  int c[kLargeSet];  // candidate
-  float lo[kLargeSet], hi[kLargeSet];
+template <int kSet>
+struct CertSet {
+  uint64_t key[kSet];
+  int c[kSet];  // candidate
+  float lo[kSet], hi[kSet];
 };
-struct LargeShared {
-  LargeSet a, b;  // one is sorted into the other
-  int open[kLargeMaxFlags];  // positions whose order is open
-  int flag_c[kLargeMaxFlags];  // a helper's pages
-  float flag_mid[kLargeMaxFlags], flag_lo[kLargeMaxFlags], flag_hi[kLargeMaxFlags];
+// The LDS of one request's certified select.  kSet: candidates the set holds;
+// kOpen: how many may be open.
+template <int kSet_, int kOpen_>
+struct CertSharedT {
+  static constexpr int kSet = kSet_;
+  static constexpr int kOpen = kOpen_;
+  CertSet<kSet> a, b;  // one is sorted into the other
+  int open[kOpen];     // positions whose order is open
+  int page_c[kAssistMaxPages];  // a helper's pages
+  float r_mid[kAssistMaxPages], r_lo[kAssistMaxPages], r_hi[kAssistMaxPages];
   int hist[256];
-  float red[2][kSelThreads / kWave];
+  float red[kSelThreads / kWave];
   unsigned long long prefix;
-  int need, all, count, tie, nopen;
+  int need, all, count, tie, nopen, bad;
   alignas(16) float tile[RescoreFloats<kSelRescoreGroup>()];
 };
+using CertShared = CertSharedT<kCertMaxKeys, kCertMaxKeys>;
+using CertSharedLarge = CertSharedT<kLargeMaxK + kLargeMaxOpen, kLargeMaxOpen>;
 
 // Threads per element of a loop over `count` elements (a power of two, <= 16).
-__device__ __forceinline__ int LargeParts(int count) {
+__device__ __forceinline__ int SetParts(int count) {
   int parts = 16;
   while (parts > 1 && parts * count > kSelThreads) parts >>= 1;
   return parts;
@@ -732,8 +423,9 @@ __device__ __forceinline__ int LargeParts(int count) {
 
 // from, sorted by key (descending; equal keys by position), into to: ranks by
 // counting, `parts` threads per element.  Ends with a barrier.
-__device__ void LargeSort(const LargeSet& from, LargeSet& to, int count) {
-  const int parts = LargeParts(count);
+template <class Set>
+__device__ __forceinline__ void SortSet(const Set& from, Set& to, int count) {
+  const int parts = SetParts(count);
   const int part = threadIdx.x & (parts - 1);
   for (int base = 0; base < count; base += kSelThreads / parts) {
     const int t = base + static_cast<int>(threadIdx.x) / parts;
@@ -762,8 +454,9 @@ __device__ void LargeSort(const LargeSet& from, LargeSet& to, int count) {
 // that line, its intervals leave open: a position below kk whose interval
 // meets any other's, and one from kk on whose interval meets a member's.
 // Appends them to sh.open (sh.nopen counts all of them).  Ends with a barrier.
-__device__ void LargeCertify(LargeShared& sh, const LargeSet& set, int count, int kk) {
-  const int parts = LargeParts(count);
+template <class Shared, class Set>
+__device__ __forceinline__ void CertifySet(Shared& sh, const Set& set, int count, int kk) {
+  const int parts = SetParts(count);
   const int part = threadIdx.x & (parts - 1);
   for (int base = 0; base < count; base += kSelThreads / parts) {
     const int t = base + static_cast<int>(threadIdx.x) / parts;
@@ -784,7 +477,7 @@ __device__ void LargeCertify(LargeShared& sh, const LargeSet& set, int count, in
     for (int o = 1; o < parts; o <<= 1) open |= __shfl_xor(open, o, kWave);
     if (in && open != 0 && part == 0) {
       const int pos = atomicAdd(&sh.nopen, 1);
-      if (pos < kLargeMaxFlags) sh.open[pos] = t;
+      if (pos < Shared::kOpen) sh.open[pos] = t;
     }
   }
   __syncthreads();
@@ -796,7 +489,8 @@ __device__ void LargeCertify(LargeShared& sh, const LargeSet& set, int count, in
 // refines a page in 4-6 us with half its waves, and refining 8 to 64 pages in
 // the selecting workgroup, or running their exact chains (25 us a group of 32),
 // is what its time went to while the rest of the chip stood idle.
-__device__ __forceinline__ void LargeAssist(LargeShared& sh, const SelectAssist& assist,
+template <class Shared>
+__device__ __forceinline__ void AssistSelect(Shared& sh, const SelectAssist& assist,
                                             unsigned long long* words, int index,
                                             const float* __restrict__ lo,
                                             const float* __restrict__ hi,
@@ -825,9 +519,9 @@ __device__ __forceinline__ void LargeAssist(LargeShared& sh, const SelectAssist&
     if (!ok || c < 0 || c >= n) {
       sh.all = 0;
     } else {
-      sh.flag_c[tid] = c;
-      sh.flag_lo[tid] = lo[c];
-      sh.flag_hi[tid] = hi[c];
+      sh.page_c[tid] = c;
+      sh.r_lo[tid] = lo[c];
+      sh.r_hi[tid] = hi[c];
     }
   }
   __syncthreads();
@@ -835,11 +529,11 @@ __device__ __forceinline__ void LargeAssist(LargeShared& sh, const SelectAssist&
   RefineScores<kSelThreads>(
       mine,
       [&](int f) -> const float* {
-        const int pg = cand[sh.flag_c[f]];
+        const int pg = cand[sh.page_c[f]];
         const bool live = InPool(pg, capacity) && token_counts[pg] != 0;
         return live ? summaries + static_cast<size_t>(pg) * E : nullptr;
       },
-      [&](int f) { return dsd_refine::FirstPassBound(sh.flag_lo[f], sh.flag_hi[f], scale, E); },
+      [&](int f) { return dsd_refine::FirstPassBound(sh.r_lo[f], sh.r_hi[f], scale, E); },
       [&](int f, float m, float l, float h) {
         unsigned long long* to =
             words + 1 + kAssistMaxPages + 3 * (index + f * assist.helpers);
@@ -850,48 +544,32 @@ __device__ __forceinline__ void LargeAssist(LargeShared& sh, const SelectAssist&
       q, E, scale, reinterpret_cast<double*>(sh.tile));
 }
 
-template <int PER>
-__global__ __launch_bounds__(kSelThreads) void SelectCertifiedLargeKernel(
-    const float* __restrict__ mid, const float* __restrict__ lo,
-    const float* __restrict__ hi, const float* __restrict__ queries,
-    const float* __restrict__ summaries, const int* __restrict__ token_counts, int capacity,
-    const int* __restrict__ cand_offsets, const int* __restrict__ cand_ids, int batch, int total,
-    int max_candidates, int E, float scale, int top_k, int* __restrict__ selected,
-    int* __restrict__ counts, int* __restrict__ exact_pages, SelectAssist assist,
-    FailReport fail) {
-  static_assert(PER * kSelThreads <= kLargeMaxKeys && PER <= 32, "a member bit per candidate");
-  __shared__ LargeShared sh;
-  const bool helper = static_cast<int>(blockIdx.x) >= batch;
-  const int r = static_cast<int>(blockIdx.x) % batch;
+// Request r's certified top-k (up to PER * kSelThreads candidates, the whole
+// workgroup of kSelThreads threads).  load(c, &mid, &lo, &hi) gives candidate
+// c's first-pass interval (c indexes the batch's CSR); with kPolled it may
+// report that an interval never became readable (false), and the request
+// then selects nothing (kFailWait).  emit(i, page) writes member i of the
+// selection (rank order), emit_count(kk) the count (or kUndecided); emit_count
+// runs once, in thread 0, after the emits.  words: the request's assist words,
+// or null.
+template <int PER, bool kPolled, class Shared, class Load, class Emit, class EmitCount>
+__device__ __forceinline__ void SelectCertifiedRequest(
+    Shared& sh, int begin, int n, int kk, Load load, Emit emit, EmitCount emit_count,
+    const float* __restrict__ q, const float* __restrict__ summaries,
+    const int* __restrict__ token_counts, int capacity, const int* __restrict__ cand, int E,
+    float scale, int* __restrict__ exact_pages, const SelectAssist& assist,
+    unsigned long long* words, FailReport fail) {
+  static_assert(PER <= 32, "a member bit per candidate");
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = tid / kWave;
-  int begin, n;
-  RequestRange(cand_offsets, r, total, helper ? FailReport{} : fail, &begin, &n);
-  if (n > max_candidates || n > PER * kSelThreads) {
-    // Only max_candidates were scored: select nothing and report it.
-    if (tid == 0 && !helper) ReportFailure(fail, kFailShape);
-    n = 0;
+  if (tid == 0) {
+    sh.count = 0;
+    sh.tie = 0;
+    sh.nopen = 0;
+    sh.bad = 0;
   }
-  const int kk = top_k <= 0 ? 0 : (top_k < n ? top_k : n);
-  const int* cand = cand_ids + begin;
-  // The request's assist words lie in its candidates' publication words
-  // (idle in this step form): [0] the pages to refine, [1 ..] which
-  // candidates, then three words of interval per page.
-  const bool assisted = assist.helpers > 0 && n > kAssistLeastCandidates;
-  unsigned long long* words = assisted ? assist.words + 3 * static_cast<size_t>(begin) : nullptr;
-  if (helper) {
-    if (kk > 0 && assisted) {
-      LargeAssist(sh, assist, words, (static_cast<int>(blockIdx.x) - batch) / batch, lo + begin,
-                  hi + begin, queries + static_cast<size_t>(r) * E, summaries, token_counts,
-                  capacity, cand, n, E, scale);
-    }
-    return;
-  }
-  if (kk == 0) {
-    if (tid == 0) counts[r] = 0;
-    return;
-  }
+  if constexpr (kPolled) __syncthreads();
   uint64_t key[PER];
   float clo[PER], chi[PER];
 #pragma unroll
@@ -901,17 +579,21 @@ __global__ __launch_bounds__(kSelThreads) void SelectCertifiedLargeKernel(
     clo[j] = INFINITY;
     chi[j] = -INFINITY;
     if (i < n) {
-      key[j] = SelectKey(mid[begin + i], cand[i]);
-      clo[j] = lo[begin + i];
-      chi[j] = hi[begin + i];
+      float m;
+      if (!load(begin + i, &m, &clo[j], &chi[j])) sh.bad = 1;
+      key[j] = SelectKey(m, cand[i]);
     }
   }
-  if (tid == 0) {
-    sh.count = 0;
-    sh.tie = 0;
-    sh.nopen = 0;
+  if constexpr (kPolled) {
+    __syncthreads();
+    if (sh.bad != 0) {
+      if (tid == 0) {
+        ReportFailure(fail, kFailWait);
+        emit_count(0);
+      }
+      return;
+    }
   }
-  const float* q = queries + static_cast<size_t>(r) * E;
   // 1. The kk-th largest key, 8 bits a round (RadixSelectKth).
   uint64_t prefix = 0;
   int need = kk;
@@ -956,16 +638,16 @@ __global__ __launch_bounds__(kSelThreads) void SelectCertifiedLargeKernel(
     }
   }
   for (int o = 1; o < kWave; o <<= 1) my_min = fminf(my_min, __shfl_xor(my_min, o, kWave));
-  if (lane == 0) sh.red[0][wave] = my_min;
+  if (lane == 0) sh.red[wave] = my_min;
   __syncthreads();
   float min_t_lo = INFINITY;
-  for (int w = 0; w < kSelThreads / kWave; ++w) min_t_lo = fminf(min_t_lo, sh.red[0][w]);
+  for (int w = 0; w < kSelThreads / kWave; ++w) min_t_lo = fminf(min_t_lo, sh.red[w]);
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const int i = tid + kSelThreads * j;
     if (i < n && !((members >> j) & 1u) && chi[j] >= min_t_lo) {
       const int pos = atomicAdd(&sh.count, 1);
-      if (pos < kk + kLargeMaxFlags) {
+      if (pos < Shared::kSet && pos < kk + Shared::kOpen) {
         sh.a.key[pos] = key[j];
         sh.a.c[pos] = i;
         sh.a.lo[pos] = clo[j];
@@ -975,18 +657,18 @@ __global__ __launch_bounds__(kSelThreads) void SelectCertifiedLargeKernel(
   }
   __syncthreads();
   const int count = sh.count;
-  const bool too_many = count > kk + kLargeMaxFlags;
+  const bool too_many = count > Shared::kSet || count > kk + Shared::kOpen;
   // 3. Their order, and what the first-pass intervals leave open.  (A member
   //    that meets an outsider meets one of the set.)
   if (!too_many) {
-    LargeSort(sh.a, sh.b, count);
-    LargeCertify(sh, sh.b, count, kk);
+    SortSet(sh.a, sh.b, count);
+    CertifySet(sh, sh.b, count, kk);
   }
-  int nopen = too_many ? kLargeMaxFlags + 1 : sh.nopen;
+  int nopen = too_many ? Shared::kOpen + 1 : sh.nopen;
   const bool refine = E % 256 == 0 && nopen > 0;
   const bool share =
-      refine && assisted && nopen >= kAssistLeastPages && nopen <= kAssistMaxPages;
-  if (assisted) {
+      refine && words != nullptr && nopen >= kAssistLeastPages && nopen <= kAssistMaxPages;
+  if (words != nullptr) {
     // The helpers' share (0: they leave).
     if (tid < (share ? nopen : 0)) {
       PutTagged(words + 1 + tid, assist.epoch, static_cast<uint32_t>(sh.b.c[sh.open[tid]]));
@@ -995,11 +677,11 @@ __global__ __launch_bounds__(kSelThreads) void SelectCertifiedLargeKernel(
       PutTagged(words, assist.epoch, static_cast<uint32_t>(share ? nopen : 0));
     }
   }
-  if (nopen > kLargeMaxFlags) {
-    if (tid == 0) counts[r] = kUndecided;
+  if (nopen > Shared::kOpen) {
+    if (tid == 0) emit_count(kUndecided);
     return;
   }
-  LargeSet* order = &sh.b;
+  auto* order = &sh.b;
   if (share || (refine && RefineWorthwhile<kSelThreads>(nopen))) {
     // 4. Refined intervals of the open positions (sh.flag_*), by the helpers
     //    or here, and the set's order again.  A wait that gives up leaves the
@@ -1011,7 +693,7 @@ __global__ __launch_bounds__(kSelThreads) void SelectCertifiedLargeKernel(
       if (tid < 3 * nopen) {
         unsigned long long w = 0;
         if (AwaitTagged(words + 1 + kAssistMaxPages + tid, assist.epoch, assist.spin_limit, &w)) {
-          float* to = tid % 3 == 0 ? sh.flag_mid : (tid % 3 == 1 ? sh.flag_lo : sh.flag_hi);
+          float* to = tid % 3 == 0 ? sh.r_mid : (tid % 3 == 1 ? sh.r_lo : sh.r_hi);
           to[tid / 3] = __uint_as_float(static_cast<uint32_t>(w));
         } else {
           sh.all = 0;
@@ -1031,27 +713,27 @@ __global__ __launch_bounds__(kSelThreads) void SelectCertifiedLargeKernel(
             return dsd_refine::FirstPassBound(sh.b.lo[t], sh.b.hi[t], scale, E);
           },
           [&](int f, float m, float l, float h) {
-            sh.flag_mid[f] = m;
-            sh.flag_lo[f] = l;
-            sh.flag_hi[f] = h;
+            sh.r_mid[f] = m;
+            sh.r_lo[f] = l;
+            sh.r_hi[f] = h;
           },
           q, E, scale, reinterpret_cast<double*>(sh.tile));
     }
     if (sh.all != 0) {
       if (tid < nopen) {
         const int t = sh.open[tid];
-        sh.b.key[t] = SelectKey(sh.flag_mid[tid], cand[sh.b.c[t]]);
-        sh.b.lo[t] = sh.flag_lo[tid];
-        sh.b.hi[t] = sh.flag_hi[tid];
+        sh.b.key[t] = SelectKey(sh.r_mid[tid], cand[sh.b.c[t]]);
+        sh.b.lo[t] = sh.r_lo[tid];
+        sh.b.hi[t] = sh.r_hi[tid];
       }
       if (tid == 0) sh.nopen = 0;
       __syncthreads();
-      LargeSort(sh.b, sh.a, count);
-      LargeCertify(sh, sh.a, count, kk);
+      SortSet(sh.b, sh.a, count);
+      CertifySet(sh, sh.a, count, kk);
       order = &sh.a;
       nopen = sh.nopen;
-      if (nopen > kLargeMaxFlags) {
-        if (tid == 0) counts[r] = kUndecided;
+      if (nopen > Shared::kOpen) {
+        if (tid == 0) emit_count(kUndecided);
         return;
       }
     }
@@ -1059,7 +741,7 @@ __global__ __launch_bounds__(kSelThreads) void SelectCertifiedLargeKernel(
   if (nopen > 0) {
     // 5. Exact chains for what is still open, and the order once more.
     if (tid == 0 && exact_pages != nullptr) atomicAdd(exact_pages, nopen);
-    LargeSet& set = *order;
+    auto& set = *order;
     RescoreChains<kSelRescoreGroup, kSelThreads>(
         nopen, [&](int f) { return cand[set.c[sh.open[f]]]; },
         [&](int f, float score) {
@@ -1067,13 +749,75 @@ __global__ __launch_bounds__(kSelThreads) void SelectCertifiedLargeKernel(
           set.key[t] = SelectKey(score, cand[set.c[t]]);
         },
         q, summaries, token_counts, capacity, E, scale, sh.tile);
-    LargeSet* other = order == &sh.a ? &sh.b : &sh.a;
-    LargeSort(set, *other, count);
+    auto* other = order == &sh.a ? &sh.b : &sh.a;
+    SortSet(set, *other, count);
     order = other;
   }
+  for (int i = tid; i < kk; i += kSelThreads) emit(i, KeyPage(order->key[i]));
+  if constexpr (kPolled) __syncthreads();  // every member out before the count
+  if (tid == 0) emit_count(kk);
+}
+
+// Request r's candidates and how many to select; none (reported) when there
+// are more than the score kernel covered or the select holds.
+__device__ __forceinline__ int SelectRange(const int* cand_offsets, int r, int total,
+                                           int max_candidates, int most, int top_k,
+                                           const FailReport& fail, bool report, int* begin,
+                                           int* n) {
+  RequestRange(cand_offsets, r, total, report ? fail : FailReport{}, begin, n);
+  if (*n > max_candidates || *n > most) {
+    if (report && threadIdx.x == 0) ReportFailure(fail, kFailShape);
+    *n = 0;
+  }
+  return top_k <= 0 ? 0 : (top_k < *n ? top_k : *n);
+}
+
+// Workgroup r < batch: request r's select; the others its helpers.
+template <int PER, class Shared>
+__global__ __launch_bounds__(kSelThreads) void SelectCertifiedKernel(
+    const float* __restrict__ mid, const float* __restrict__ lo,
+    const float* __restrict__ hi, const float* __restrict__ queries,
+    const float* __restrict__ summaries, const int* __restrict__ token_counts, int capacity,
+    const int* __restrict__ cand_offsets, const int* __restrict__ cand_ids, int batch, int total,
+    int max_candidates, int E, float scale, int top_k, int* __restrict__ selected,
+    int* __restrict__ counts, int* __restrict__ exact_pages, SelectAssist assist,
+    FailReport fail) {
+  __shared__ Shared sh;
+  const bool helper = static_cast<int>(blockIdx.x) >= batch;
+  const int r = static_cast<int>(blockIdx.x) % batch;
+  int begin, n;
+  const int kk = SelectRange(cand_offsets, r, total, max_candidates, PER * kSelThreads, top_k,
+                             fail, !helper, &begin, &n);
+  const int* cand = cand_ids + begin;
+  const float* q = queries + static_cast<size_t>(r) * E;
+  // The request's assist words lie in its candidates' publication words
+  // (idle in this step form): [0] the pages to refine, [1 ..] which
+  // candidates, then three words of interval per page.
+  unsigned long long* words = assist.helpers > 0 && n > kAssistLeastCandidates
+                                  ? assist.words + 3 * static_cast<size_t>(begin)
+                                  : nullptr;
+  if (helper) {
+    if (kk > 0 && words != nullptr) {
+      AssistSelect(sh, assist, words, (static_cast<int>(blockIdx.x) - batch) / batch, lo + begin,
+                   hi + begin, q, summaries, token_counts, capacity, cand, n, E, scale);
+    }
+    return;
+  }
+  if (kk == 0) {
+    if (threadIdx.x == 0) counts[r] = 0;
+    return;
+  }
   int* out = selected + static_cast<size_t>(r) * top_k;
-  for (int i = tid; i < kk; i += kSelThreads) out[i] = KeyPage(order->key[i]);
-  if (tid == 0) counts[r] = kk;
+  SelectCertifiedRequest<PER, false>(
+      sh, begin, n, kk,
+      [&](int c, float* m, float* l, float* h) {
+        *m = mid[c];
+        *l = lo[c];
+        *h = hi[c];
+        return true;
+      },
+      [&](int i, int page) { out[i] = page; }, [&](int count) { counts[r] = count; }, q,
+      summaries, token_counts, capacity, cand, E, scale, exact_pages, assist, words, fail);
 }
 
 // Certified select for up to 256 candidates per request: thread i owns
@@ -1280,9 +1024,11 @@ struct WideShared {
   union {
     ScoreShared score;
     CertShared cert;
-    AttnFastShared<kFWaves, 128> attn;
+    struct {
+      AttnFastShared<kFWaves, 128> attn;
+      int page[kCertMaxKeys];  // the item's selected pages
+    };
   };
-  int page[kCertMaxKeys];  // an attention item's selected pages
   int item;
   int last;
   int count;
@@ -1358,30 +1104,37 @@ __device__ __forceinline__ void WideStepItem(const PoolView& pool, const WideArg
       if (a.stamps != nullptr && threadIdx.x == 0) sh.stamp[1] = wall_clock64();
       unsigned long long* sel = w.sel_rec + static_cast<size_t>(r) * stride;
       int* out = a.selected + static_cast<size_t>(r) * stride;
-      SelectCertifiedRequest<true>(
-          sh.cert, r,
-          [&](int c, float* m, float* l, float* h) {
-            unsigned long long* p = a.rec + 3 * static_cast<size_t>(c);
-            unsigned long long w0 = 0, w1 = 0, w2 = 0;
-            const bool ok = AwaitTagged(p, a.wait_tag, a.spin_limit, &w0) &&
-                            AwaitTagged(p + 1, a.wait_tag, a.spin_limit, &w1) &&
-                            AwaitTagged(p + 2, a.wait_tag, a.spin_limit, &w2);
-            *m = __uint_as_float(static_cast<uint32_t>(w0));
-            *l = __uint_as_float(static_cast<uint32_t>(w1));
-            *h = __uint_as_float(static_cast<uint32_t>(w2));
-            return ok;
-          },
-          [&](int i, int page) {
-            out[i] = page;
-            PutTagged(sel + i, a.epoch, static_cast<uint32_t>(page));
-          },
-          [&](int kk) {
-            a.counts[r] = kk;
-            PutTagged(w.cnt_rec + r, a.epoch, static_cast<uint32_t>(kk));
-          },
-          a.queries, pool.summaries, pool.token_counts, pool.capacity, a.cand_offsets,
-          a.cand_ids, a.total, a.max_candidates, pool.elements, a.scale, a.top_k,
-          a.exact_pages, a.fail);
+      int begin, n;
+      const int kk = SelectRange(a.cand_offsets, r, a.total, a.max_candidates, kCertMaxKeys,
+                                 a.top_k, a.fail, true, &begin, &n);
+      auto emit_count = [&](int count) {
+        a.counts[r] = count;
+        PutTagged(w.cnt_rec + r, a.epoch, static_cast<uint32_t>(count));
+      };
+      if (kk == 0) {
+        if (threadIdx.x == 0) emit_count(0);
+      } else {
+        SelectCertifiedRequest<kCertMaxKeys / kSelThreads, true>(
+            sh.cert, begin, n, kk,
+            [&](int c, float* m, float* l, float* h) {
+              unsigned long long* p = a.rec + 3 * static_cast<size_t>(c);
+              unsigned long long w0 = 0, w1 = 0, w2 = 0;
+              const bool ok = AwaitTagged(p, a.wait_tag, a.spin_limit, &w0) &&
+                              AwaitTagged(p + 1, a.wait_tag, a.spin_limit, &w1) &&
+                              AwaitTagged(p + 2, a.wait_tag, a.spin_limit, &w2);
+              *m = __uint_as_float(static_cast<uint32_t>(w0));
+              *l = __uint_as_float(static_cast<uint32_t>(w1));
+              *h = __uint_as_float(static_cast<uint32_t>(w2));
+              return ok;
+            },
+            [&](int i, int page) {
+              out[i] = page;
+              PutTagged(sel + i, a.epoch, static_cast<uint32_t>(page));
+            },
+            emit_count, a.queries + static_cast<size_t>(r) * pool.elements, pool.summaries,
+            pool.token_counts, pool.capacity, a.cand_ids + begin, pool.elements, a.scale,
+            a.exact_pages, SelectAssist{}, nullptr, a.fail);
+      }
       if (a.stamps != nullptr && threadIdx.x == 0) sh.stamp[2] = wall_clock64();
     }
   } else {
@@ -1573,34 +1326,28 @@ void LaunchSelectCertified(const PoolView& pool, const float* d_mid, const float
   if (pool.elements % kWave != 0) {
     throw std::invalid_argument("certified select needs E % 64 == 0");
   }
-  if (max_candidates > kCertMaxKeys) {
-    if (max_candidates > kLargeMaxKeys || top_k > kLargeMaxK) {
-      throw std::invalid_argument("certified select supports up to " +
-                                  std::to_string(kLargeMaxKeys) + " candidates per request and " +
-                                  std::to_string(kLargeMaxK) + " of them selected");
-    }
-    const auto kernel = max_candidates <= kLargeMaxKeys / 2
-                            ? SelectCertifiedLargeKernel<kLargeMaxKeys / 2 / kSelThreads>
-                            : SelectCertifiedLargeKernel<kLargeMaxKeys / kSelThreads>;
-    // Helpers only where every workgroup is resident at once, so that a
-    // request's workgroup and its helpers do run side by side (one that does
-    // not run in time costs the bounded wait, nothing else).
-    SelectAssist a = assist;
-    a.helpers = a.words == nullptr || a.epoch == 0
-                    ? 0
-                    : std::min(kAssistMaxHelpers, a.compute_units / batch - 1);
-    if (a.helpers < kAssistLeastPages) a.helpers = 0;
-    hipLaunchKernelGGL(kernel, dim3(batch * (1 + a.helpers)), dim3(kSelThreads), 0, stream, d_mid,
-                       d_lo, d_hi, d_queries, pool.summaries, pool.token_counts, pool.capacity,
-                       d_cand_offsets, d_cand_ids, batch, total_candidates, max_candidates,
-                       pool.elements, scale, top_k, d_selected, d_counts, d_exact_pages, a, fail);
-    DSD_HIP_CHECK(hipGetLastError());
-    return;
+  if (max_candidates > kCertMaxKeys && (max_candidates > kLargeMaxKeys || top_k > kLargeMaxK)) {
+    throw std::invalid_argument("certified select supports up to " +
+                                std::to_string(kLargeMaxKeys) + " candidates per request and " +
+                                std::to_string(kLargeMaxK) + " of them selected");
   }
-  hipLaunchKernelGGL(SelectCertifiedKernel, dim3(batch), dim3(kSelThreads), 0, stream, d_mid,
+  const auto kernel = max_candidates <= kCertMaxKeys
+                          ? SelectCertifiedKernel<kCertMaxKeys / kSelThreads, CertShared>
+                      : max_candidates <= kLargeMaxKeys / 2
+                          ? SelectCertifiedKernel<kLargeMaxKeys / 2 / kSelThreads, CertSharedLarge>
+                          : SelectCertifiedKernel<kLargeMaxKeys / kSelThreads, CertSharedLarge>;
+  // Helpers only where every workgroup is resident at once, so that a
+  // request's workgroup and its helpers do run side by side (one that does
+  // not run in time costs the bounded wait, nothing else).
+  SelectAssist a = assist;
+  a.helpers = a.words == nullptr || a.epoch == 0
+                  ? 0
+                  : std::min(kAssistMaxHelpers, a.compute_units / batch - 1);
+  if (a.helpers < kAssistLeastPages) a.helpers = 0;
+  hipLaunchKernelGGL(kernel, dim3(batch * (1 + a.helpers)), dim3(kSelThreads), 0, stream, d_mid,
                      d_lo, d_hi, d_queries, pool.summaries, pool.token_counts, pool.capacity,
-                     d_cand_offsets, d_cand_ids, total_candidates, max_candidates,
-                     pool.elements, scale, top_k, d_selected, d_counts, d_exact_pages, fail);
+                     d_cand_offsets, d_cand_ids, batch, total_candidates, max_candidates,
+                     pool.elements, scale, top_k, d_selected, d_counts, d_exact_pages, a, fail);
   DSD_HIP_CHECK(hipGetLastError());
 }
 
@@ -1678,7 +1425,7 @@ void LaunchSelectTopK(const float* d_scores, const int* d_cand_offsets,
 void PreloadStepKernels() {
   PreloadKernel(WideStepKernel);
   PreloadKernel(WideBumpKernel);
-  PreloadKernel(SelectCertifiedKernel);
+  PreloadKernel(SelectCertifiedKernel<kCertMaxKeys / kSelThreads, CertShared>);
   PreloadKernel(SelectCertifiedRankKernel);
   PreloadKernel(ScoreBoundGenericKernel<true>);
 }
