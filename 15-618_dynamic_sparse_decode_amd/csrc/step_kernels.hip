@@ -19,12 +19,54 @@ namespace {
 //
 // The reference scores a page as acc = 0; acc = fl(acc + fl(q[i]*s[i])) for
 // i = 0..E-1, then fl(acc*scale).  That chain must be reproduced in order to
-// keep page selection bit-exact, so one lane owns one candidate page and
-// walks its summary row sequentially with separately rounded multiply and
-// add (__fmul_rn / __fadd_rn; never contracted to FMA).  A wave covers 64
-// candidates of one request, so the query operand is wave-uniform and is
-// fetched through the scalar cache.
+// keep page selection bit-exact, so one lane owns one candidate page and adds
+// its products in order with separately rounded multiply and add (__fmul_rn /
+// __fadd_rn; never contracted to FMA).
+//
+// ScoreChainsKernel (E a multiple of 64): a workgroup takes 8, 16 or 32 pages
+// of one request; the lanes of its first wave run their chains from products
+// that the other waves form in LDS, a stretch ahead, from rows read whole
+// (RescoreChains).  Bound by the chain, E dependent adds fed from LDS at
+// about 7 cycles each (E = 4096: 12 us), so a small batch takes few pages per
+// workgroup and spreads them over the chip.  16 requests of 512-2048 tokens
+// (1207 pages): 25 us; 108 us with the kernel below, whose 32 waves were all
+// there was and read 64 rows a line at a time.
+//
+// ScoreExactKernel (other E): a wave of 64 candidates, each lane walking its
+// own row in memory.
 // ---------------------------------------------------------------------------
+constexpr int kChainPages = 32;
+constexpr int kChainThreads = 512;
+
+__global__ __launch_bounds__(kChainThreads) void ScoreChainsKernel(
+    const float* __restrict__ queries, const float* __restrict__ summaries,
+    const int* __restrict__ token_counts, int capacity, const int* __restrict__ cand_offsets,
+    const int* __restrict__ cand_ids, int total, int pages_per_group, int E, float scale,
+    float* __restrict__ scores, const int* __restrict__ only, FailReport fail) {
+  __shared__ __align__(16) float tile[RescoreFloats<kChainPages>()];
+  __shared__ int s_page[kChainPages];
+  const int r = blockIdx.y;
+  if (only != nullptr && only[r] >= 0) return;  // decided without exact scores
+  int begin, n;
+  if (!RequestRange(cand_offsets, r, total, fail, &begin, &n)) return;
+  const int first = static_cast<int>(blockIdx.x) * pages_per_group;
+  if (first >= n) return;
+  const int pages = n - first < pages_per_group ? n - first : pages_per_group;
+  if (static_cast<int>(threadIdx.x) < pages) {
+    // A page holding no tokens reads as an all-zero summary
+    // (src/paged_kv_cache.cpp:457-459); the products q*0 are still formed.  An
+    // id outside the pool scores as such a page and is reported.
+    const int page = cand_ids[begin + first + threadIdx.x];
+    if (!InPool(page, capacity)) ReportFailure(fail, kFailPageId);
+    s_page[threadIdx.x] = page;
+  }
+  __syncthreads();
+  RescoreChains<kChainPages, kChainThreads>(
+      pages, [&](int f) { return s_page[f]; },
+      [&](int f, float score) { scores[begin + first + f] = score; },
+      queries + static_cast<size_t>(r) * E, summaries, token_counts, capacity, E, scale, tile);
+}
+
 template <bool kVec4>
 __global__ __launch_bounds__(kWave) void ScoreExactKernel(
     const float* __restrict__ queries, const float* __restrict__ summaries,
@@ -1244,6 +1286,18 @@ void LaunchScoreExact(const PoolView& pool, const float* d_queries,
                       float* d_scores, FailReport fail, hipStream_t stream,
                       const int* d_undecided) {
   if (batch <= 0 || max_candidates <= 0) return;
+  if (pool.elements % kWave == 0) {
+    // The fewest pages per workgroup that keep the batch within a round of
+    // workgroups (two per CU).
+    int pages = kChainPages / 4;
+    while (pages < kChainPages && total_candidates > 512 * pages) pages *= 2;
+    hipLaunchKernelGGL(ScoreChainsKernel, dim3((max_candidates + pages - 1) / pages, batch),
+                       dim3(kChainThreads), 0, stream, d_queries, pool.summaries,
+                       pool.token_counts, pool.capacity, d_cand_offsets, d_cand_ids,
+                       total_candidates, pages, pool.elements, scale, d_scores, d_undecided, fail);
+    DSD_HIP_CHECK(hipGetLastError());
+    return;
+  }
   const dim3 grid((max_candidates + kWave - 1) / kWave, batch);
   if (pool.elements % 4 == 0) {
     hipLaunchKernelGGL(ScoreExactKernel<true>, grid, dim3(kWave), 0, stream,
