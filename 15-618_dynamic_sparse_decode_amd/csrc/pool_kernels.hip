@@ -15,8 +15,33 @@ namespace {
 
 constexpr int kPoolThreads = 256;
 
-// One workgroup per uploaded page; threads stride the E summary elements so
-// each token row is read with contiguous, coalesced loads.
+// kVec consecutive floats (4 only where rows are 16-byte aligned: E % 4 == 0).
+template <int kVec>
+__device__ __forceinline__ void LoadVec(const float* __restrict__ p, float (&v)[kVec]) {
+  if constexpr (kVec == 4) {
+    const float4 x = *reinterpret_cast<const float4*>(p);
+    v[0] = x.x;
+    v[1] = x.y;
+    v[2] = x.z;
+    v[3] = x.w;
+  } else {
+#pragma unroll
+    for (int i = 0; i < kVec; ++i) v[i] = p[i];
+  }
+}
+template <int kVec>
+__device__ __forceinline__ void StoreVec(float* __restrict__ p, const float (&v)[kVec]) {
+  if constexpr (kVec == 4) {
+    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < kVec; ++i) p[i] = v[i];
+  }
+}
+
+// Workgroup (i, y): uploaded page i, kPoolThreads * kVec of its summary's
+// elements; each token row is read with contiguous loads.
+template <int kVec>
 __global__ __launch_bounds__(kPoolThreads) void FinishPageUploadKernel(
     PoolView pool, const int* __restrict__ page_ids,
     const int* __restrict__ token_counts, const float* __restrict__ rows,
@@ -26,29 +51,36 @@ __global__ __launch_bounds__(kPoolThreads) void FinishPageUploadKernel(
   const int page = page_ids[i];
   const int count = token_counts[i];
   const int E = pool.elements;
-  float* summary = pool.summaries + static_cast<size_t>(page) * E;
-  if (rows != nullptr) {
-    const float* src = rows + static_cast<size_t>(i) * E;
-    for (int e = threadIdx.x; e < E; e += blockDim.x) summary[e] = src[e];
-  } else {
-    const float* keys = pool.keys + static_cast<size_t>(page) * pool.page_elems;
-    const float inv = __fdiv_rn(1.0f, static_cast<float>(count));
-    for (int e = threadIdx.x; e < E; e += blockDim.x) {
-      float acc = 0.0f;
-      for (int t = 0; t < count; ++t) {
-        acc = __fadd_rn(acc, keys[static_cast<size_t>(t) * E + e]);
-      }
-      summary[e] = __fmul_rn(acc, inv);
-    }
-  }
-  if (threadIdx.x == 0) {
+  const int e = (static_cast<int>(blockIdx.y) * kPoolThreads + static_cast<int>(threadIdx.x)) * kVec;
+  if (blockIdx.y == 0 && threadIdx.x == 0) {
     pool.token_counts[page] = count;
     pool.live[page] = 1;
   }
+  if (e >= E) return;
+  float acc[kVec] = {};
+  if (rows != nullptr) {
+    LoadVec<kVec>(rows + static_cast<size_t>(i) * E + e, acc);
+  } else {
+    const float* keys = pool.keys + static_cast<size_t>(page) * pool.page_elems + e;
+    const float inv = __fdiv_rn(1.0f, static_cast<float>(count));
+    for (int t = 0; t < count; ++t) {
+      float k[kVec];
+      LoadVec<kVec>(keys + static_cast<size_t>(t) * E, k);
+#pragma unroll
+      for (int x = 0; x < kVec; ++x) acc[x] = __fadd_rn(acc[x], k[x]);
+    }
+#pragma unroll
+    for (int x = 0; x < kVec; ++x) acc[x] = __fmul_rn(acc[x], inv);
+  }
+  StoreVec<kVec>(pool.summaries + static_cast<size_t>(page) * E + e, acc);
 }
 
-// One workgroup per page segment; tokens of a segment are applied in offset
-// order so the running mean matches the host's sequence of updates.
+// Workgroup (s, y): page segment s, kPoolThreads * kVec elements of its rows;
+// tokens of a segment are applied in offset order so the running mean matches
+// the host's sequence of updates.  (One workgroup per segment took 17 us for
+// the 32 tokens of a serving step at E = 4096, this grid
+// 5 us.)
+template <int kVec>
 __global__ __launch_bounds__(kPoolThreads) void AppendTokensKernel(
     PoolView pool, const int* __restrict__ seg_start,
     const int* __restrict__ order, const int* __restrict__ page_ids,
@@ -61,41 +93,39 @@ __global__ __launch_bounds__(kPoolThreads) void AppendTokensKernel(
   const int end = seg_start[seg + 1];
   const int E = pool.elements;
   const int page = page_ids[order[begin]];
-  const size_t page_base = static_cast<size_t>(page) * pool.page_elems;
-
-  for (int q = begin; q < end; ++q) {
-    const int tok = order[q];
-    const size_t dst = page_base + static_cast<size_t>(offsets[tok]) * E;
-    const size_t src = static_cast<size_t>(tok) * E;
-    for (int e = threadIdx.x; e < E; e += blockDim.x) {
-      pool.keys[dst + e] = keys[src + e];
-      pool.values[dst + e] = values[src + e];
-    }
-  }
-
-  float* summary = pool.summaries + static_cast<size_t>(page) * E;
-  if (rows != nullptr) {
-    const float* src = rows + static_cast<size_t>(order[end - 1]) * E;
-    for (int e = threadIdx.x; e < E; e += blockDim.x) summary[e] = src[e];
-  } else {
-    const bool fresh = offsets[order[begin]] == 0;
-    for (int e = threadIdx.x; e < E; e += blockDim.x) {
-      float s = fresh ? 0.0f : summary[e];
-      for (int q = begin; q < end; ++q) {
-        const int tok = order[q];
-        const float old_count = static_cast<float>(offsets[tok]);
-        const float new_count = __fadd_rn(old_count, 1.0f);
-        s = __fdiv_rn(__fadd_rn(__fmul_rn(s, old_count),
-                                keys[static_cast<size_t>(tok) * E + e]),
-                      new_count);
-      }
-      summary[e] = s;
-    }
-  }
-  if (threadIdx.x == 0) {
+  const int e = (static_cast<int>(blockIdx.y) * kPoolThreads + static_cast<int>(threadIdx.x)) * kVec;
+  if (blockIdx.y == 0 && threadIdx.x == 0) {
     pool.token_counts[page] = counts[order[end - 1]];
     pool.live[page] = 1;
   }
+  if (e >= E) return;
+  const size_t page_base = static_cast<size_t>(page) * pool.page_elems + e;
+  float* summary = pool.summaries + static_cast<size_t>(page) * E + e;
+  float s[kVec] = {};
+  if (rows != nullptr) {
+    LoadVec<kVec>(rows + static_cast<size_t>(order[end - 1]) * E + e, s);
+  } else if (offsets[order[begin]] != 0) {
+    LoadVec<kVec>(summary, s);
+  }
+  for (int q = begin; q < end; ++q) {
+    const int tok = order[q];
+    const size_t dst = page_base + static_cast<size_t>(offsets[tok]) * E;
+    const size_t src = static_cast<size_t>(tok) * E + e;
+    float k[kVec], v[kVec];
+    LoadVec<kVec>(keys + src, k);
+    LoadVec<kVec>(values + src, v);
+    StoreVec<kVec>(pool.keys + dst, k);
+    StoreVec<kVec>(pool.values + dst, v);
+    if (rows == nullptr) {
+      const float old_count = static_cast<float>(offsets[tok]);
+      const float new_count = __fadd_rn(old_count, 1.0f);
+#pragma unroll
+      for (int x = 0; x < kVec; ++x) {
+        s[x] = __fdiv_rn(__fadd_rn(__fmul_rn(s[x], old_count), k[x]), new_count);
+      }
+    }
+  }
+  StoreVec<kVec>(summary, s);
 }
 
 __global__ __launch_bounds__(kPoolThreads) void MarkFreeKernel(
@@ -125,18 +155,28 @@ __device__ __forceinline__ float HashValue(uint32_t x) {
   x ^= x >> 15;
   x *= 0x846ca68bu;
   x ^= x >> 16;
-  return static_cast<float>(static_cast<int>(x % 2001u) - 1000) / 1000.0f;
+  // n / 1000, correctly rounded, for |n| <= 1000: Markstein's correction of
+  // n * fl(1/1000) by its exact remainder (IBM J. Res. Dev. 34, 1990), checked
+  // for all 2001 values (tests/test_generators_hash.py).  A general division
+  // is three times as long, and the generators below are bound by their
+  // instructions.
+  const float n = static_cast<float>(static_cast<int>(x % 2001u) - 1000);
+  const float q = __fmul_rn(n, 0.001f);
+  return fmaf(fmaf(-q, 1000.0f, n), 0.001f, q);
 }
 
-__device__ __forceinline__ float PromptValue(int request_id, int page_idx, int token,
-                                             int element, int stream) {
+// The prompt hash up to its element; PromptValue finishes it for one element
+// and stream (1: keys, 2: values).
+__device__ __forceinline__ uint32_t PromptRow(int request_id, int page_idx, int token) {
   uint32_t x = 0x9e3779b9u;
   x = HashMix(x, request_id, 0x85ebca6bu);
   x = HashMix(x, page_idx, 0xc2b2ae35u);
-  x = HashMix(x, token, 0x27d4eb2fu);
-  x = HashMix(x, element, 0x165667b1u);
-  x = HashMix(x, stream, 0xd3a2646cu);
-  return HashValue(x);
+  return HashMix(x, token, 0x27d4eb2fu);
+}
+
+__device__ __forceinline__ float PromptValue(uint32_t row, int element, int stream) {
+  const uint32_t x = HashMix(row, element, 0x165667b1u);
+  return HashValue(HashMix(x, stream, 0xd3a2646cu));
 }
 
 __device__ __forceinline__ float DecodeValue(int request_id, int decode_step, int element,
@@ -149,7 +189,12 @@ __device__ __forceinline__ float DecodeValue(int request_id, int decode_step, in
   return HashValue(x);
 }
 
-// One workgroup per prompt page: K/V from the hash, summary by the host rule.
+// Workgroup (i, y): page i of the prompt, kPoolThreads * kVec elements of its
+// rows: K/V from the hash, summary by the host rule.  A prompt of a few
+// thousand tokens is a few hundred pages, so one workgroup per page left most
+// of the chip idle (128 pages of 16 x 4096: 50 us; this grid
+// 15-22; 8192 pages, 4.3 GB, 870 us, bound by the hash).
+template <int kVec>
 __global__ __launch_bounds__(kPoolThreads) void PrefillSyntheticKernel(
     PoolView pool, const int* __restrict__ page_ids, const int* __restrict__ token_counts,
     int n, int request_id) {
@@ -158,23 +203,31 @@ __global__ __launch_bounds__(kPoolThreads) void PrefillSyntheticKernel(
   const int page = page_ids[i];
   const int count = token_counts[i];
   const int E = pool.elements;
-  const size_t base = static_cast<size_t>(page) * pool.page_elems;
-  const float inv = __fdiv_rn(1.0f, static_cast<float>(count));
-  for (int e = threadIdx.x; e < E; e += blockDim.x) {
-    float acc = 0.0f;
-    for (int t = 0; t < count; ++t) {
-      const float k = PromptValue(request_id, i, t, e, 1);
-      const float v = PromptValue(request_id, i, t, e, 2);
-      pool.keys[base + static_cast<size_t>(t) * E + e] = k;
-      pool.values[base + static_cast<size_t>(t) * E + e] = v;
-      acc = __fadd_rn(acc, k);
-    }
-    pool.summaries[static_cast<size_t>(page) * E + e] = __fmul_rn(acc, inv);
-  }
-  if (threadIdx.x == 0) {
+  const int e = (static_cast<int>(blockIdx.y) * kPoolThreads + static_cast<int>(threadIdx.x)) * kVec;
+  if (blockIdx.y == 0 && threadIdx.x == 0) {
     pool.token_counts[page] = count;
     pool.live[page] = 1;
   }
+  if (e >= E) return;
+  const float inv = __fdiv_rn(1.0f, static_cast<float>(count));
+  size_t at = static_cast<size_t>(page) * pool.page_elems + e;
+  float acc[kVec] = {};
+  for (int t = 0; t < count; ++t) {
+    const uint32_t row = PromptRow(request_id, i, t);
+    float k[kVec], v[kVec];
+#pragma unroll
+    for (int x = 0; x < kVec; ++x) {
+      k[x] = PromptValue(row, e + x, 1);
+      v[x] = PromptValue(row, e + x, 2);
+      acc[x] = __fadd_rn(acc[x], k[x]);
+    }
+    StoreVec<kVec>(pool.keys + at, k);
+    StoreVec<kVec>(pool.values + at, v);
+    at += E;
+  }
+#pragma unroll
+  for (int x = 0; x < kVec; ++x) acc[x] = __fmul_rn(acc[x], inv);
+  StoreVec<kVec>(pool.summaries + static_cast<size_t>(page) * E + e, acc);
 }
 
 // One workgroup per (page segment, kPoolThreads elements of the token row),
@@ -232,11 +285,18 @@ __global__ __launch_bounds__(kPoolThreads) void AppendSyntheticKernel(PoolView p
 
 }  // namespace
 
+// Workgroups along a row of E elements, kVec per thread.
+static unsigned RowSlices(int elements, int vec) {
+  return static_cast<unsigned>((elements + kPoolThreads * vec - 1) / (kPoolThreads * vec));
+}
+
 void LaunchFinishPageUpload(const PoolView& pool, const int* d_page_ids,
                             const int* d_token_counts, const float* d_rows,
                             int n, hipStream_t stream) {
   if (n <= 0) return;
-  hipLaunchKernelGGL(FinishPageUploadKernel, dim3(n), dim3(kPoolThreads), 0,
+  const bool vec = pool.elements % 4 == 0;
+  const auto kernel = vec ? FinishPageUploadKernel<4> : FinishPageUploadKernel<1>;
+  hipLaunchKernelGGL(kernel, dim3(n, RowSlices(pool.elements, vec ? 4 : 1)), dim3(kPoolThreads), 0,
                      stream, pool, d_page_ids, d_token_counts, d_rows, n);
   DSD_HIP_CHECK(hipGetLastError());
 }
@@ -248,10 +308,11 @@ void LaunchAppendTokens(const PoolView& pool, const int* d_seg_start,
                         const float* d_rows, int num_segments,
                         hipStream_t stream) {
   if (num_segments <= 0) return;
-  hipLaunchKernelGGL(AppendTokensKernel, dim3(num_segments), dim3(kPoolThreads),
-                     0, stream, pool, d_seg_start, d_order, d_page_ids,
-                     d_offsets, d_counts, d_keys, d_values, d_rows,
-                     num_segments);
+  const bool vec = pool.elements % 4 == 0;
+  const auto kernel = vec ? AppendTokensKernel<4> : AppendTokensKernel<1>;
+  hipLaunchKernelGGL(kernel, dim3(num_segments, RowSlices(pool.elements, vec ? 4 : 1)),
+                     dim3(kPoolThreads), 0, stream, pool, d_seg_start, d_order, d_page_ids,
+                     d_offsets, d_counts, d_keys, d_values, d_rows, num_segments);
   DSD_HIP_CHECK(hipGetLastError());
 }
 
@@ -259,8 +320,10 @@ void LaunchPrefillSynthetic(const PoolView& pool, const int* d_page_ids,
                             const int* d_token_counts, int n, int request_id,
                             hipStream_t stream) {
   if (n <= 0) return;
-  hipLaunchKernelGGL(PrefillSyntheticKernel, dim3(n), dim3(kPoolThreads), 0, stream, pool,
-                     d_page_ids, d_token_counts, n, request_id);
+  const bool vec = pool.elements % 4 == 0;
+  const auto kernel = vec ? PrefillSyntheticKernel<4> : PrefillSyntheticKernel<1>;
+  hipLaunchKernelGGL(kernel, dim3(n, RowSlices(pool.elements, vec ? 4 : 1)), dim3(kPoolThreads), 0,
+                     stream, pool, d_page_ids, d_token_counts, n, request_id);
   DSD_HIP_CHECK(hipGetLastError());
 }
 
@@ -431,7 +494,7 @@ void PreloadPoolKernels() {
   PreloadKernel(StageInKernel);
   PreloadKernel(StepMarkKernel);
   PreloadKernel(AppendSyntheticKernel);
-  PreloadKernel(AppendTokensKernel);
+  PreloadKernel(AppendTokensKernel<4>);
 }
 
 }  // namespace dsdk
