@@ -1734,7 +1734,9 @@ struct dsd_sparse_ctx {
     const PoolView& v = pool->view;
     L.valid = true;
     L.certified = StepCertified(v, score_mode, max_n, top_k, need_exact_scores);
-    L.fused = StepFused(v, L.certified, fused_enabled, max_n, top_k);
+    L.fused = StepFused(v, L.certified, fused_enabled, max_n, top_k) ||
+              (L.certified && fused_enabled && wide_enabled &&
+               dsdk::FusedStepLong(v, batch, max_n, top_k));
     // The wide step takes the batches the single launch cannot (a request
     // beyond 256 candidates); DSD_FUSED_STEP=0 alone keeps three kernels.
     L.wide_shape = !L.fused && L.certified && batch > 0 &&
@@ -1743,7 +1745,7 @@ struct dsd_sparse_ctx {
     L.wide = L.wide_shape && wide_enabled;
     // Heads spread over workgroups, except for the shapes of the single
     // launches, whose outputs the three kernels reproduce bit for bit.
-    if (d_pieces.ptr != nullptr && !L.wide_shape &&
+    if (d_pieces.ptr != nullptr && !L.wide_shape && !L.fused &&
         !dsdk::FusedStepSupported(v, max_n, top_k)) {
       L.piece_room = dsdk::AttentionPieceRoom(
           v, batch, static_cast<long long>(std::max(1, top_k)) * v.page_size);
@@ -2907,7 +2909,8 @@ int dsd_sparse_run_batch_device_static(dsd_pool* pool, int top_k, int batch,
     L.valid = true;
     L.certified = StepCertified(v, DSD_SCORE_CERTIFIED, max_candidates, top_k,
                                 StepWantsExactScores(d_scores, max_candidates));
-    L.fused = StepFused(v, L.certified, true, max_candidates, top_k);
+    L.fused = StepFused(v, L.certified, true, max_candidates, top_k) ||
+              (L.certified && dsdk::FusedStepLong(v, batch, max_candidates, top_k));
     // (three kernels where a context would run the wide step, with its
     // attention partition: the same outputs)
     L.wide_shape = !L.fused && L.certified && batch > 0 &&

@@ -334,6 +334,9 @@ constexpr int kFRefineSlots = 8;
 
 // E = 4096, head_dim = 128, max_candidates <= 256, top_k <= 256.
 bool FusedStepSupported(const PoolView& pool, int max_candidates, int top_k);
+// The same at 257 to 512 candidates: top_k <= 64, batches large enough that it
+// beats the wide step.
+bool FusedStepLong(const PoolView& pool, int batch, int max_candidates, int top_k);
 // Heads per workgroup for a batch: the fewest (1, 2, 4, 8) that keep the grid
 // within `compute_units` workgroups, else 8.
 int FusedStepHeadsPerGroup(const PoolView& pool, int batch, int compute_units);

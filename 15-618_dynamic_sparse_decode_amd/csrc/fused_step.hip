@@ -1,6 +1,7 @@
 // fused_step.hip -- the whole sparse decode step in one launch (gfx950).
 //
-// For the hot shape (E = 4096, head_dim 128, at most 256 candidates and
+// For the hot shape (E = 4096, head_dim 128, at most 256 candidates -- 512 in
+// the long form -- and
 // top_k <= 256 per request, certified selection) the three stages of the
 // step -- page scoring (reference ScorePagesCpu, src/reference_kernels.cpp:
 // 59-80), top-k (SelectTopKPagesCpu, :82-107) and gather + attention
@@ -56,11 +57,24 @@ constexpr int kFD = 128;
 constexpr int kFMaxHeadsPerGroup = 8;       // workgroup = 1, 2, 4 or 8 heads (16/hpw waves each)
 constexpr int kFMaxCand = 256;
 constexpr int kFMaxK = 256;
+// The long form: up to 512 candidates per request (eight per lane in the
+// selection instead of four; a kernel of its own, so the short one keeps its
+// registers), at most 64 of them selected.  It takes batches of at least
+// kFLongBatch requests that attend at most kFLongTokens tokens each, where it
+// beats the wide step, whose items are one 1024-thread workgroup per head: 32
+// requests of 64-269 pages, top 8: 51 us against 78; 8 such requests 21.5
+// against 29.6; 64 of 269-500 pages, top 16: 176 against 201.  With more tokens
+// the wide step's evenly shared heads win (16 requests of 269-500 pages, top
+// 32: 88.5 us against 92; top 64: 141 against 150), and with few requests its
+// score slices (3 of 500 pages, top 16: 32 us against 34.5).
+constexpr int kFLongCand = 512;
+constexpr int kFLongK = 64;
+constexpr int kFLongBatch = 6;
+constexpr int kFLongTokens = 256;
 constexpr int kFLpt = 16;                 // lanes per token row (8 dims each)
 constexpr int kFDq = kFD / kFLpt;         // 8
 constexpr int kFTpc = kWave / kFLpt;      // 4 token rows per wave per chunk
 constexpr int kFUnroll = 4;               // chunks in flight per wave
-constexpr int kFSlots = kFMaxCand / kWave;  // candidates (or ranks) per lane: l + 64m
 constexpr int kFRescoreGroup = 16;            // exact chains per rescore group
 static_assert(kFMaxK <= kFMaxCand, "rank slots cover the candidate slots");
 // Timing mode: per-workgroup wall clocks at start, slice scored, counter
@@ -69,7 +83,10 @@ static_assert(kFMaxK <= kFMaxCand, "rank slots cover the candidate slots");
 constexpr int kStampsPerGroup = 10;
 enum Stamp { kStart, kScored, kReady, kRecords, kRanked, kSelected, kEnd, kRefine, kRefined, kHwId };
 
+template <int kCand>
 struct FusedShared {
+  static constexpr int kMaxCand = kCand;
+  static constexpr int kSlots = kCand / kWave;  // candidates (or ranks) per lane: l + 64m
   uint64_t stamp[kStampsPerGroup];  // timing mode: thread 0's clocks
   // score pass (per wave): float total (the carry into wave 2p+1) and the
   // bound sums
@@ -80,15 +97,15 @@ struct FusedShared {
   int nflag;
   int certified;  // FastSelect's verdict, for every wave
   // selection (attention item)
-  float mid[kFMaxCand];
-  uint64_t key[kFMaxCand];
-  float lo[kFMaxCand];
-  float hi[kFMaxCand];
-  int top[kFMaxCand];
-  int flag[kFMaxCand];
-  int rank[kFMaxCand];
-  int cpage[kFMaxCand];  // page id and token count of candidate i
-  int cntok[kFMaxCand];
+  float mid[kCand];
+  uint64_t key[kCand];
+  float lo[kCand];
+  float hi[kCand];
+  int top[kCand];
+  int flag[kCand];
+  int rank[kCand];
+  int cpage[kCand];  // page id and token count of candidate i
+  int cntok[kCand];
   float tlo[kFMaxK];    // intervals of the top-k members, in rank order
   float thi[kFMaxK];
   float red[2][kFWaves];
@@ -106,20 +123,21 @@ __device__ __forceinline__ uint64_t Now() { return static_cast<uint64_t>(wall_cl
 // Timing mode only: thread 0 records the wall clock for stamp `which` in
 // LDS (a global store here would make the next barrier wait for it); the
 // kernel's end writes them out.
-__device__ __forceinline__ void StampAt(const FusedArgs& a, FusedShared& sh, int which) {
+template <class Shared>
+__device__ __forceinline__ void StampAt(const FusedArgs& a, Shared& sh, int which) {
   if (a.stamps != nullptr && threadIdx.x == 0) sh.stamp[which] = Now();
 }
 
-// Ranks of the n <= 256 keys in sh.key (descending; equal keys by position):
+// Ranks of the n keys in sh.key (descending; equal keys by position):
 // kTpc threads per candidate count interleaved slices of the keys
 // (candidate j is read by part j % kTpc: contiguous LDS words per
 // instruction) and add their counts with shuffles.  Returns the rank to the
 // candidate's first thread (part 0), n elsewhere.  No barrier.
-constexpr int kTpc = 4;
-// Every candidate below kFMaxCand has a lead thread.
-static_assert(kFThreads / kTpc >= kFMaxCand, "PartialRanks must cover kFMaxCand");
-
-__device__ __forceinline__ int PartialRanks(const FusedShared& sh, int n, int* cand_out) {
+template <class Shared>
+__device__ __forceinline__ int PartialRanks(const Shared& sh, int n, int* cand_out) {
+  // Every candidate has a lead thread.
+  constexpr int kTpc = kFThreads / Shared::kMaxCand;
+  static_assert(kTpc >= 1, "PartialRanks must cover the candidates");
   const int t = threadIdx.x;
   const int cand = t / kTpc;
   const int part = t - cand * kTpc;
@@ -147,7 +165,8 @@ __device__ __forceinline__ int PartialRanks(const FusedShared& sh, int n, int* c
 }
 
 // Ranks of the keys into sh.rank (whole workgroup; ends with a barrier).
-__device__ void ParallelRanks(FusedShared& sh, int n) {
+template <class Shared>
+__device__ void ParallelRanks(Shared& sh, int n) {
   int cand;
   const int rank = PartialRanks(sh, n, &cand);
   if (rank < n) sh.rank[cand] = rank;
@@ -203,15 +222,16 @@ __device__ __forceinline__ int Popc(uint64_t m) { return __popcll(m); }
 // intervals from LDS, ranks, certifies; when some order is undecided, wave 0
 // also lists the flagged candidates and all keys for the exact path.
 // Returns whether anything is flagged (the same in every wave).
-template <int CS, int RS>
-__device__ bool RankAndCertify(const FusedArgs& a, int n, int kk, const int (&page)[kFSlots],
-                               const int (&ntok)[kFSlots], FusedShared& sh) {
+template <int CS, int RS, class Shared>
+__device__ bool RankAndCertify(const FusedArgs& a, int n, int kk,
+                               const int (&page)[Shared::kSlots],
+                               const int (&ntok)[Shared::kSlots], Shared& sh) {
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
   float mid[CS], lo[CS], hi[CS];
 #pragma unroll
   for (int m = 0; m < CS; ++m) {
-    const int i = lane + kWave * m;  // < kFMaxCand: the LDS reads stay in bounds
+    const int i = lane + kWave * m;  // < kMaxCand: the LDS reads stay in bounds
     const bool in = i < n;
     const float x = sh.mid[i], l = sh.lo[i], h = sh.hi[i];
     // Midpoints are finite; -inf marks the empty slots.
@@ -383,9 +403,9 @@ __device__ __forceinline__ uint32_t WaveMaxU32(uint32_t x) {
 // interval overlaps another member's) and writing every candidate's key to
 // sh.key; -1 when a round's maximum is not unique (equal midpoints: the
 // ballot ranks then order them).  Nothing else is written before a -1.
-template <int CS>
-__device__ int FastSelect(int n, int kk, const float (&mid)[kFSlots], const float (&hi)[kFSlots],
-                          FusedShared& sh, bool dry) {
+template <int CS, class Shared>
+__device__ int FastSelect(int n, int kk, const float (&mid)[Shared::kSlots],
+                          const float (&hi)[Shared::kSlots], Shared& sh, bool dry) {
   const int lane = threadIdx.x & (kWave - 1);
   uint32_t kh[CS];  // order bits of the midpoint; 0: empty or taken
 #pragma unroll
@@ -458,14 +478,26 @@ __device__ int FastSelect(int n, int kk, const float (&mid)[kFSlots], const floa
   return 0;
 }
 
-__device__ __forceinline__ int FastSelectSlots(int n, int kk, const float (&mid)[kFSlots],
-                                               const float (&hi)[kFSlots], FusedShared& sh,
+template <class Shared>
+__device__ __forceinline__ int FastSelectSlots(int n, int kk, const float (&mid)[Shared::kSlots],
+                                               const float (&hi)[Shared::kSlots], Shared& sh,
                                                bool dry) {
-  switch ((n + kWave - 1) / kWave) {
-    case 1: return FastSelect<1>(n, kk, mid, hi, sh, dry);
-    case 2: return FastSelect<2>(n, kk, mid, hi, sh, dry);
-    case 3: return FastSelect<3>(n, kk, mid, hi, sh, dry);
-    default: return FastSelect<4>(n, kk, mid, hi, sh, dry);
+  const int slots = (n + kWave - 1) / kWave;
+  if constexpr (Shared::kSlots == 4) {
+    switch (slots) {
+      case 1: return FastSelect<1>(n, kk, mid, hi, sh, dry);
+      case 2: return FastSelect<2>(n, kk, mid, hi, sh, dry);
+      case 3: return FastSelect<3>(n, kk, mid, hi, sh, dry);
+      default: return FastSelect<4>(n, kk, mid, hi, sh, dry);
+    }
+  } else {
+    // (fewer forms: the short requests of a long batch take an even count)
+    switch ((slots + 1) / 2) {
+      case 1: return FastSelect<2>(n, kk, mid, hi, sh, dry);
+      case 2: return FastSelect<4>(n, kk, mid, hi, sh, dry);
+      case 3: return FastSelect<6>(n, kk, mid, hi, sh, dry);
+      default: return FastSelect<8>(n, kk, mid, hi, sh, dry);
+    }
   }
 }
 
@@ -489,11 +521,13 @@ __device__ __forceinline__ int FastSelectSlots(int n, int kk, const float (&mid)
 //      sequential chain (as SelectCertifiedRankKernel) and ranked again.
 // Workgroup `group` of the request's `groups` (group 0 also writes the
 // selection out).
+template <class Shared>
 __device__ __forceinline__ int SelectForRequest(const PoolView& pool, const FusedArgs& a, int r, int begin,
-                                int n, int group, int groups, FusedShared& sh) {
+                                int n, int group, int groups, Shared& sh) {
+  constexpr int kFSlots = Shared::kSlots;
   const bool writer = group == 0;
   int kk = a.top_k <= 0 ? 0 : (a.top_k < n ? a.top_k : n);
-  if (n > a.max_candidates || n > kFMaxCand) {
+  if (n > a.max_candidates || n > Shared::kMaxCand) {
     // The caller's max_candidates understated the CSR: select nothing (the
     // outputs are zeros) and report it to the host.
     if (writer && threadIdx.x == 0) ReportFailure(a.fail, kFailShape);
@@ -625,7 +659,7 @@ __device__ __forceinline__ int SelectForRequest(const PoolView& pool, const Fuse
               float mid[kFSlots], hi[kFSlots];
   #pragma unroll
               for (int m = 0; m < kFSlots; ++m) {
-                const int i = lane + kWave * m;  // < kFMaxCand: in bounds
+                const int i = lane + kWave * m;  // < kMaxCand: in bounds
                 mid[m] = sh.mid[i];
                 hi[m] = sh.hi[i];
               }
@@ -638,17 +672,26 @@ __device__ __forceinline__ int SelectForRequest(const PoolView& pool, const Fuse
           ballot = verdict < 0;  // equal midpoints: rank with ballots instead
           any = verdict == 0;
         }
-        if (ballot) switch (cs * 8 + rs) {
-          case 1 * 8 + 1: any = RankAndCertify<1, 1>(a, n, kk, page, ntok, sh); break;
-          case 2 * 8 + 1: any = RankAndCertify<2, 1>(a, n, kk, page, ntok, sh); break;
-          case 2 * 8 + 2: any = RankAndCertify<2, 2>(a, n, kk, page, ntok, sh); break;
-          case 3 * 8 + 1: any = RankAndCertify<3, 1>(a, n, kk, page, ntok, sh); break;
-          case 3 * 8 + 2: any = RankAndCertify<3, 2>(a, n, kk, page, ntok, sh); break;
-          case 3 * 8 + 3: any = RankAndCertify<3, 3>(a, n, kk, page, ntok, sh); break;
-          case 4 * 8 + 1: any = RankAndCertify<4, 1>(a, n, kk, page, ntok, sh); break;
-          case 4 * 8 + 2: any = RankAndCertify<4, 2>(a, n, kk, page, ntok, sh); break;
-          case 4 * 8 + 3: any = RankAndCertify<4, 3>(a, n, kk, page, ntok, sh); break;
-          default: any = RankAndCertify<4, 4>(a, n, kk, page, ntok, sh); break;
+        if constexpr (kFSlots == 4) {
+          if (ballot) switch (cs * 8 + rs) {
+            case 1 * 8 + 1: any = RankAndCertify<1, 1>(a, n, kk, page, ntok, sh); break;
+            case 2 * 8 + 1: any = RankAndCertify<2, 1>(a, n, kk, page, ntok, sh); break;
+            case 2 * 8 + 2: any = RankAndCertify<2, 2>(a, n, kk, page, ntok, sh); break;
+            case 3 * 8 + 1: any = RankAndCertify<3, 1>(a, n, kk, page, ntok, sh); break;
+            case 3 * 8 + 2: any = RankAndCertify<3, 2>(a, n, kk, page, ntok, sh); break;
+            case 3 * 8 + 3: any = RankAndCertify<3, 3>(a, n, kk, page, ntok, sh); break;
+            case 4 * 8 + 1: any = RankAndCertify<4, 1>(a, n, kk, page, ntok, sh); break;
+            case 4 * 8 + 2: any = RankAndCertify<4, 2>(a, n, kk, page, ntok, sh); break;
+            case 4 * 8 + 3: any = RankAndCertify<4, 3>(a, n, kk, page, ntok, sh); break;
+            default: any = RankAndCertify<4, 4>(a, n, kk, page, ntok, sh); break;
+          }
+        } else if (ballot) {
+          switch ((cs + 1) / 2) {  // (at most 64 members: one rank slot)
+            case 1: any = RankAndCertify<2, 1>(a, n, kk, page, ntok, sh); break;
+            case 2: any = RankAndCertify<4, 1>(a, n, kk, page, ntok, sh); break;
+            case 3: any = RankAndCertify<6, 1>(a, n, kk, page, ntok, sh); break;
+            default: any = RankAndCertify<8, 1>(a, n, kk, page, ntok, sh); break;
+          }
         }
         if (!any || pass == 1) break;
         // 4a. Some order is not decided by the intervals: the flagged pages
@@ -783,8 +826,9 @@ __device__ __forceinline__ int SelectForRequest(const PoolView& pool, const Fuse
 // head softmax(q_h K^T * scale) V over the selected pages' valid tokens;
 // waves 0-7 take head h0 and waves 8-15 head h0+1, each as
 // AttentionFastKernel<128, 16, 8, 4>.
+template <class Shared>
 __device__ __forceinline__ void AttentionItem(const PoolView& pool, const FusedArgs& a, int r, int begin, int n,
-                              int group, FusedShared& sh) {
+                              int group, Shared& sh) {
   const int hpw = a.heads_per_group;
   const int wph = kFWaves / hpw;       // waves per head
   const int h0 = group * hpw;
@@ -915,9 +959,10 @@ __device__ __forceinline__ void AttentionItem(const PoolView& pool, const FusedA
 // slices pipeline their passes (each pass's rows load while the previous
 // pass reduces).  Single-pass launches keep the plain form, which measured
 // faster there.
-template <bool kMultiPass>
+template <bool kMultiPass, int kCand = kFMaxCand>
 __global__ __launch_bounds__(kFThreads) void FusedStepKernel(PoolView pool, FusedArgs a) {
-  __shared__ FusedShared sh;
+  static_assert(kCand >= kFMaxCand, "the member slots fit the candidates");
+  __shared__ FusedShared<kCand> sh;
   if (a.epoch_src != nullptr) {
     // Replayed from a captured graph: the epoch the bump kernel just set.
     a.epoch = *a.epoch_src;
@@ -944,9 +989,9 @@ __global__ __launch_bounds__(kFThreads) void FusedStepKernel(PoolView pool, Fuse
   // scored or selected, zero outputs) and reported.
   int begin, n;
   RequestRange(a.cand_offsets, r, a.total, g == 0 ? a.fail : FailReport{}, &begin, &n);
-  // A request beyond the caller's max_candidates (or kFMaxCand) selects
+  // A request beyond the caller's max_candidates (or kCand) selects
   // nothing (reported by the selection): its slices are not scored.
-  if (n <= a.max_candidates && n <= kFMaxCand) {
+  if (n <= a.max_candidates && n <= kCand) {
     ScoreSlice<kMultiPass>(pool, a, r, begin + (g * n) / groups,
                            begin + ((g + 1) * n) / groups, sh);
   }
@@ -1032,6 +1077,12 @@ bool FusedStepSupported(const PoolView& pool, int max_candidates, int top_k) {
          pool.num_heads % 2 == 0 && max_candidates <= kFMaxCand && top_k <= kFMaxK;
 }
 
+bool FusedStepLong(const PoolView& pool, int batch, int max_candidates, int top_k) {
+  return FusedStepSupported(pool, 0, top_k) && batch >= kFLongBatch &&
+         max_candidates > kFMaxCand && max_candidates <= kFLongCand && top_k <= kFLongK &&
+         static_cast<int64_t>(top_k) * pool.page_size <= kFLongTokens;
+}
+
 int FusedStepHeadsPerGroup(const PoolView& pool, int batch, int compute_units) {
   // The fewest heads per workgroup (most waves per head) that keeps the
   // grid within one dispatch wave; 8 when none does.
@@ -1072,7 +1123,13 @@ void LaunchFusedStep(const PoolView& pool, const FusedArgs& args, hipStream_t st
                        const_cast<unsigned*>(args.epoch_src));
     DSD_HIP_CHECK(hipGetLastError());
   }
-  if (FusedStepMultiPass(pool, args.max_candidates, hpw)) {
+  if (args.max_candidates > kFMaxCand) {
+    if (!FusedStepLong(pool, args.batch, args.max_candidates, args.top_k)) {
+      throw std::invalid_argument("the fused step does not take this many candidates");
+    }
+    hipLaunchKernelGGL((FusedStepKernel<true, kFLongCand>), dim3(grid), dim3(kFThreads), 0, stream,
+                       pool, args);
+  } else if (FusedStepMultiPass(pool, args.max_candidates, hpw)) {
     hipLaunchKernelGGL(FusedStepKernel<true>, dim3(grid), dim3(kFThreads), 0, stream, pool, args);
   } else {
     hipLaunchKernelGGL(FusedStepKernel<false>, dim3(grid), dim3(kFThreads), 0, stream, pool, args);
@@ -1083,6 +1140,7 @@ void LaunchFusedStep(const PoolView& pool, const FusedArgs& args, hipStream_t st
 void PreloadFusedKernels() {
   PreloadKernel(FusedStepKernel<true>);
   PreloadKernel(FusedStepKernel<false>);
+  PreloadKernel(FusedStepKernel<true, kFLongCand>);
   PreloadKernel(ScorePagesKernel);
   PreloadKernel(EpochBumpKernel);
 }
