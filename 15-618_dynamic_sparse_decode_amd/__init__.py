@@ -252,9 +252,24 @@ def synchronize() -> None:
 
 
 def _ptr(array, ctype):
+    """A pointer argument to a contiguous array's data.  By the buffer
+    protocol where it applies (writable, not empty): 0.4 us against 2.6 us for
+    data_as, and a host step passes seven."""
     if array is None:
         return None
-    return array.ctypes.data_as(ctypes.POINTER(ctype))
+    try:
+        return ctypes.byref(ctype.from_buffer(array))
+    except (TypeError, ValueError):
+        return array.ctypes.data_as(ctypes.POINTER(ctype))
+
+
+def _split(packed, counts, batch):
+    """The per-request id arrays of a packed selection (parts of it)."""
+    parts, w = [], 0
+    for c in counts[:batch].tolist():
+        parts.append(packed[w:w + c])
+        w += c
+    return parts
 
 
 def _f32(a):
@@ -525,8 +540,10 @@ class SparseContext:
         batch = len(offs) - 1
         total = int(offs[-1]) if batch > 0 else 0
         E = self.pool.elements
-        out = np.zeros((max(batch, 0), E), np.float32)
-        scores = np.zeros(max(total, 1), np.float32)
+        # (a step that returns outputs writes every row)
+        make = np.zeros if output_mode == OUTPUT_NONE else np.empty
+        out = make((max(batch, 0), E), np.float32)
+        scores = np.zeros(max(total, 1), np.float32) if output_mode == OUTPUT_DEBUG else None
         sel = np.zeros(max(1, batch * max(1, self.top_k)), np.int32)
         counts = np.zeros(max(batch, 1), np.int32)
         t = StepTimings()
@@ -543,12 +560,7 @@ class SparseContext:
         if debug:
             result["scores"] = scores[:total].copy()
         if ids_out:
-            selected, w = [], 0
-            for r in range(batch):
-                c = int(counts[r])
-                selected.append(sel[w:w + c].copy())
-                w += c
-            result["selected"] = selected
+            result["selected"] = _split(sel, counts, batch)
         return result
 
     def run_staged_rows(self, query_rows, cand_offsets, cand_ids, want_ids=False,
@@ -589,12 +601,7 @@ class SparseContext:
             ctypes.memmove(out.ctypes.data, out_st.value, 4 * batch * E)
         result = {"outputs": out, "timings": t.as_dict(), "staging_queries": q_st.value}
         if want_ids:
-            selected, w = [], 0
-            for r in range(batch):
-                c = int(counts[r])
-                selected.append(sel[w:w + c].copy())
-                w += c
-            result["selected"] = selected
+            result["selected"] = _split(sel, counts, batch)
         return result
 
     def run_table(self, table, slots, queries=None, query_rows=None, output_mode=OUTPUT_OUTPUTS,
@@ -606,7 +613,7 @@ class SparseContext:
         sl = _i32(slots)
         batch = len(sl)
         E = self.pool.elements
-        out = np.zeros((batch, E), np.float32)
+        out = (np.zeros if output_mode == OUTPUT_NONE else np.empty)((batch, E), np.float32)
         sel = np.zeros(max(1, batch * max(1, self.top_k)), np.int32)
         counts = np.zeros(max(batch, 1), np.int32)
         q = _f32(queries).reshape(-1) if queries is not None else None
@@ -622,12 +629,7 @@ class SparseContext:
             _ptr(counts, ctypes.c_int) if want_ids else None, ctypes.byref(t)))
         result = {"outputs": out, "timings": t.as_dict()}
         if want_ids:
-            selected, w = [], 0
-            for r in range(batch):
-                c = int(counts[r])
-                selected.append(sel[w:w + c].copy())
-                w += c
-            result["selected"] = selected
+            result["selected"] = _split(sel, counts, batch)
         return result
 
     def run_table_async(self, table, slots, queries=None, query_rows=None,
