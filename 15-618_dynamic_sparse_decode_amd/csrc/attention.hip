@@ -508,7 +508,7 @@ int AttentionPieceRoom(const PoolView& pool, int batch, long long max_slots) {
   const AttnShape shape = FastShape(pool.head_dim, false);
   const long long heads = pool.num_heads;
   if (shape.fn == nullptr || batch <= 0) return 0;
-  if (max_slots > 0 && max_slots <= shape.align) return 0;  // one step per head
+  if (max_slots > 0 && max_slots <= kAttnWhole * shape.align) return 0;  // one piece each
   if (batch * heads >= kAttnRound) return 0;
   // About one round of equal pieces for the smaller batches, which leaves the
   // least to merge (one request of 32 heads, 32768 tokens: 185 us with 512,

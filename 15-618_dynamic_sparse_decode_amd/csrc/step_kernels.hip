@@ -1332,12 +1332,12 @@ void LaunchScoreBounds(const PoolView& pool, const float* d_queries,
                      max_candidates, scale, d_mid, d_lo, d_hi, fail, stream);
     return;
   }
-  // Enough waves for the chip to hold (8192; 32 requests of 8 x 128 heads and
-  // 300 pages each: the step took 49.5 us, 51.6 with 4096 and 54.4 with 1024),
-  // fewer where a workgroup's copy of a long query weighs more (16 requests of
-  // 64 x 128 heads: 120.7 us with 4096, 124.0 with 8192, 137 with 1024); 1 to
-  // 64 pages each.
-  const int target_waves = pool.elements > 4096 ? 4096 : 8192;
+  // More waves than the chip holds at once (7168), so that one that ends makes
+  // room: a page per wave up to 16384 pages (32 requests of 8 x 128 heads and
+  // 300 pages each: the step took 42.9 us, 44.8 with 8192 waves, 47.0 with
+  // 4096); fewer where a workgroup's copy of a long query weighs more (16
+  // requests of 64 x 128 heads: 109.2 us with 4096, 112.4 with 8192).
+  const int target_waves = pool.elements > 4096 ? 4096 : 16384;
   const int per_wave = std::min(
       kWave, std::max(1, (total_candidates + target_waves - 1) / target_waves));
   const int per_group = per_wave * kBoundWaves;

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("H,D,ps,k,lengths", [
-    (1, 64, 1, 5, [1900, 2048, 1900, 1, 1900, 1900]),  # a quarter row; waves of 2 pages
+    (1, 64, 1, 5, [2048, 1901, 1] + [2047] * 8),  # a quarter row; waves of 2 pages
     (3, 64, 2, 7, [70, 3]),                 # E = 192
     (4, 64, 2, 7, [130]),                   # E = 256: one whole row
     (5, 64, 2, 7, [130, 64]),               # E = 320: a row and a quarter
@@ -46,4 +46,31 @@ def test_bounds_hold_and_select_like_the_oracle(gpu, H, D, ps, k, lengths):
     for r in range(B):
         assert cert["selected"][r].tolist() == selected[r].tolist()
     assert orc.max_abs_diff(cert["outputs"], outs) <= 1e-4
+    pool.close()
+
+
+def test_device_queries_need_no_alignment(gpu):
+    """A device step's queries at a 4-byte offset: the same ids and bits."""
+    import torch
+    H, D, ps, k = 8, 96, 4, 5
+    batch = gpu.SyntheticBatch(H, D, ps, [900, 33], seed=2)
+    E, total = H * D, batch.total_candidates
+    pool = gpu.DevicePagePool(H, D, ps, batch.capacity)
+    batch.upload(pool)
+    offs, ids = (torch.from_numpy(a).cuda() for a in (batch.cand_offsets, batch.cand_ids))
+    results = []
+    with gpu.SparseContext(pool, k, 2, total, 2 * k) as ctx:
+        for shift in (0, 1):
+            room = torch.zeros(2 * E + 4, device="cuda")
+            room[shift:shift + 2 * E] = torch.from_numpy(batch.queries.reshape(-1)).cuda()
+            out = torch.zeros(2, E, device="cuda")
+            sel = torch.full((2, k), -1, dtype=torch.int32, device="cuda")
+            torch.cuda.synchronize()
+            ctx.run_batch_device(2, total, batch.max_candidates, room.data_ptr() + 4 * shift,
+                                 offs.data_ptr(), ids.data_ptr(), out.data_ptr(), 0,
+                                 sel.data_ptr())
+            ctx.device_status()
+            results.append((out.cpu().numpy().view(np.uint32), sel.cpu().numpy()))
+    assert np.array_equal(results[0][0], results[1][0])
+    assert np.array_equal(results[0][1], results[1][1])
     pool.close()
