@@ -129,14 +129,14 @@ struct PinnedBuffer {
 };
 
 // The scratch of an attention launch that spreads heads over workgroups
-// (dsdk::AttentionArgs::piece_words, then its counters), zeroed.
-void ReservePieces(DeviceBuffer<unsigned long long>* pieces) {
-  pieces->Reserve(dsdk::AttentionPieceWords() + dsdk::AttentionPieceCounters() / 2);
-  DSD_HIP_CHECK(hipMemset(pieces->ptr, 0, pieces->count * sizeof(unsigned long long)));
-  DSD_HIP_CHECK(hipStreamSynchronize(nullptr));  // (the steps' streams do not wait for it)
+// (dsdk::AttentionArgs::piece_words, then its counters), in 64-bit words.  It
+// lies behind another buffer of its owner and exists from the start: made by
+// the first call that needed it, it took 50 us of a dense step of 26.
+size_t PieceScratchWords() {
+  return dsdk::AttentionPieceWords() + static_cast<size_t>(dsdk::AttentionPieceCounters()) / 2;
 }
-unsigned* PieceArrivals(const DeviceBuffer<unsigned long long>& pieces) {
-  return reinterpret_cast<unsigned*>(pieces.ptr + dsdk::AttentionPieceWords());
+unsigned* PieceArrivals(unsigned long long* pieces) {
+  return reinterpret_cast<unsigned*>(pieces + dsdk::AttentionPieceWords());
 }
 
 constexpr uint64_t kLargeCopyBytes = 1ull << 20;  // src/device_page_pool.cpp:13
@@ -248,11 +248,10 @@ struct dsd_pool {
   PinnedBuffer<float> h_dense_q, h_dense_out;
   PinnedBuffer<int> h_dense_offsets, h_dense_ids;
   hipEvent_t dense_start = nullptr, dense_stop = nullptr;
-  // The dense attention's pieces (attention.hip): one scratch per pool, made
-  // by the first call that needs it.  piece_ev marks the end of the last
-  // launch that used it, and every launch waits for it, so calls on several
-  // streams take turns.
-  DeviceBuffer<unsigned long long> pieces;
+  // The dense attention's pieces (attention.hip): one scratch per pool (2 MiB,
+  // behind the keys).  piece_ev marks the end of the last launch that used it,
+  // and every launch waits for it, so calls on several streams take turns.
+  unsigned long long* pieces = nullptr;
   hipEvent_t piece_ev = nullptr;
   uint64_t* k_offsets = nullptr;  // [capacity] element offset of each page
   uint64_t* v_offsets = nullptr;
@@ -418,7 +417,15 @@ int dsd_pool_create(int num_heads, int head_dim, int page_size,
                               static_cast<size_t>(v.page_elems) * sizeof(float);
       const size_t sum_bytes = static_cast<size_t>(capacity_pages) *
                                static_cast<size_t>(v.elements) * sizeof(float);
-      DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.keys), kv_bytes));
+      const bool pieces = dsdk::AttentionPieceRoom(v, 1, 0) > 0;
+      const size_t keys_end = (kv_bytes + 255) / 256 * 256;
+      const size_t piece_bytes = pieces ? PieceScratchWords() * sizeof(unsigned long long) : 0;
+      DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.keys), keys_end + piece_bytes));
+      if (pieces) {
+        pool->pieces = reinterpret_cast<unsigned long long*>(
+            reinterpret_cast<unsigned char*>(v.keys) + keys_end);
+        DSD_HIP_CHECK(hipMemsetAsync(pool->pieces, 0, piece_bytes, pool->stream));
+      }
       DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.values), kv_bytes));
       DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.summaries), sum_bytes));
       DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.token_counts),
@@ -1634,7 +1641,7 @@ struct dsd_sparse_ctx {
   DeviceBuffer<unsigned long long> d_sel_rec;
   DeviceBuffer<unsigned> d_wide_counters;
   DeviceBuffer<unsigned> d_wide_seq;
-  DeviceBuffer<unsigned long long> d_pieces;  // the attention's (attention.hip)
+  unsigned long long* pieces = nullptr;  // the attention's (attention.hip), behind d_rec
   mutable unsigned wide_launches = 0;  // host count of wide launches (picks the counter set)
   // The epoch of the step being enqueued: it tags the fused step's
   // publication words and every failure report of the step's kernels.
@@ -1745,12 +1752,12 @@ struct dsd_sparse_ctx {
     L.wide = L.wide_shape && wide_enabled;
     // Heads spread over workgroups, except for the shapes of the single
     // launches, whose outputs the three kernels reproduce bit for bit.
-    if (d_pieces.ptr != nullptr && !L.wide_shape && !L.fused &&
+    if (pieces != nullptr && !L.wide_shape && !L.fused &&
         !dsdk::FusedStepSupported(v, max_n, top_k)) {
       L.piece_room = dsdk::AttentionPieceRoom(
           v, batch, static_cast<long long>(std::max(1, top_k)) * v.page_size);
-      L.piece_words = d_pieces.ptr;
-      L.piece_arrivals = PieceArrivals(d_pieces);
+      L.piece_words = pieces;
+      L.piece_arrivals = PieceArrivals(pieces);
     }
     L.batch = batch;
     L.total = total;
@@ -1913,23 +1920,24 @@ int dsd_sparse_create(dsd_pool* pool, int top_k, int max_batch,
     DSD_HIP_CHECK(hipMemset(ctx->d_sel_rec.ptr, 0, (B * K + B) * sizeof(unsigned long long)));
     ctx->d_wide_counters.Reserve(4 * (B + 1));
     DSD_HIP_CHECK(hipMemset(ctx->d_wide_counters.ptr, 0, 4 * (B + 1) * sizeof(unsigned)));
-    if (dsdk::AttentionPieceRoom(pool->view, 1,
-                                 static_cast<long long>(K) * pool->view.page_size) > 0 &&
-        (!dsdk::FusedStepSupported(pool->view, 0, 0) ||
-         max_total_candidates > dsdk::WideStepMaxCandidates())) {
-      ReservePieces(&ctx->d_pieces);
-    }
     ctx->d_wide_seq.Reserve(1);
     DSD_HIP_CHECK(hipMemset(ctx->d_wide_seq.ptr, 0, sizeof(unsigned)));
     {
       const size_t rec = 3 * P;
+      const bool pieces =
+          dsdk::AttentionPieceRoom(pool->view, 1,
+                                   static_cast<long long>(K) * pool->view.page_size) > 0 &&
+          (!dsdk::FusedStepSupported(pool->view, 0, 0) ||
+           max_total_candidates > dsdk::WideStepMaxCandidates());
+      const size_t words = rec + (pieces ? PieceScratchWords() : 0);
       // The largest fused grid: one head per workgroup.
       const size_t stamps =
           static_cast<size_t>(dsdk::FusedStepGrid(pool->view, static_cast<int>(B), 1)) *
           dsdk::FusedStepStampsPerGroup();
-      ctx->d_rec.Reserve(rec);
+      ctx->d_rec.Reserve(words);
+      if (pieces) ctx->pieces = ctx->d_rec.ptr + rec;
       ctx->h_stamps.Reserve(stamps, hipHostMallocCoherent);
-      DSD_HIP_CHECK(hipMemset(ctx->d_rec.ptr, 0, rec * sizeof(unsigned long long)));
+      DSD_HIP_CHECK(hipMemset(ctx->d_rec.ptr, 0, words * sizeof(unsigned long long)));
       const size_t refined = 3 * dsdk::kFRefineSlots * B;
       ctx->d_refined.Reserve(refined);
       DSD_HIP_CHECK(hipMemset(ctx->d_refined.ptr, 0, refined * sizeof(unsigned long long)));
@@ -2850,10 +2858,11 @@ StaticScratch& StaticScratchOn(int device) {
 // in that order and stays unsplit.
 void LaunchDense(dsd_pool* pool, dsdk::AttentionArgs* a, hipStream_t s) {
   const bool capturing = s != nullptr && StreamCapturing(s);
-  if (!capturing) a->piece_room = dsdk::AttentionPieceRoom(pool->view, a->batch, 0);
+  if (!capturing && pool->pieces != nullptr) {
+    a->piece_room = dsdk::AttentionPieceRoom(pool->view, a->batch, 0);
+  }
   if (a->piece_room > 0) {
-    if (pool->pieces.ptr == nullptr) ReservePieces(&pool->pieces);
-    a->piece_words = pool->pieces.ptr;
+    a->piece_words = pool->pieces;
     a->piece_arrivals = PieceArrivals(pool->pieces);
   }
   if (a->piece_room > 0) DSD_HIP_CHECK(hipStreamWaitEvent(s, pool->piece_ev, 0));
