@@ -291,7 +291,9 @@ int dsd_synthetic_batch(int num_heads, int head_dim, int page_size, int batch,
  * enqueues work on `stream` (a hipStream_t; NULL = the context's stream).
  * total_candidates and max_candidates (largest n_r) must describe the CSR.
  * selected ([batch][top_k], unused slots untouched), selected_counts,
- * scores may be NULL (context scratch is used).
+ * scores may be NULL (context scratch is used).  Scores are the certified
+ * midpoints, or exact ones in exact mode and beyond 2048 candidates per
+ * request.
  * The inputs are checked on the device, not the host: a request whose
  * offsets leave [0, total_candidates] or whose list is longer than
  * max_candidates selects nothing, and a candidate id outside the pool scores
@@ -331,10 +333,11 @@ typedef struct dsd_launch_info {
   int score_pages_per_group; /* wide, three-kernel at E = 4096: pages per
                                 score workgroup */
   int wide;                  /* 1: the wide single launch (257 to 2048
-                                candidates per request: score slices, the
-                                select and the attention overlap in one
-                                kernel; DSD_WIDE_STEP=0 at context creation
-                                gives three kernels) */
+                                candidates per request, where the fused step
+                                does not take them: score slices, the select
+                                and the attention overlap in one kernel;
+                                DSD_WIDE_STEP=0 at context creation gives
+                                three kernels) */
 } dsd_launch_info;
 int dsd_sparse_last_launch(const dsd_sparse_ctx* ctx, dsd_launch_info* out);
 
