@@ -363,6 +363,15 @@ __global__ __launch_bounds__(WAVES * kWave) void AttentionFastKernel(
     if (tid < D) out[tid] = lt == 0.0f ? 0.0f : at / lt;
     return;
   }
+  if (tid < D && mx == -INFINITY) {
+    // No maximum: the sums are zeros (no valid token, or logits of -inf) or
+    // NaN (NaN logits), and a NaN must reach the merge, as one wave's reaches
+    // AttnCombine when another wave has a maximum.
+    for (int w = 0; w < WAVES; ++w) {
+      lt += sh.l[w];
+      at += sh.acc[w][tid];
+    }
+  }
   unsigned long long* words =
       args.piece_words +
       (static_cast<size_t>(blockIdx.y) * pool.num_heads + h) * static_cast<size_t>(D + 2);
@@ -422,7 +431,8 @@ __global__ __launch_bounds__(WAVES * kWave) void AttentionFastKernel(
       lt += sh.l[i];
       at += sh.acc[i][tid];
     }
-    out[tid] = lt == 0.0f ? 0.0f : at / lt;
+    // (no piece with a maximum: zeros, as for an unsplit head)
+    out[tid] = lt == 0.0f || m == -INFINITY ? 0.0f : at / lt;
   }
 }
 

@@ -101,7 +101,9 @@ __device__ __forceinline__ void AttnRange(const PoolView& pool, int head_off, in
       }
 #pragma unroll
       for (int o = 1; o < LPT; o <<= 1) dot += __shfl_xor(dot, o, kWave);
-      if (valid[u]) {
+      // (a logit of -inf ahead of the stream's first maximum weighs nothing:
+      // -inf - -inf would make it NaN, and a piece may well begin with one)
+      if (valid[u] && !(dot == -INFINITY && st.m == -INFINITY)) {
         const float m_new = fmaxf(st.m, dot);
         const float alpha = Exp2(st.m - m_new);
         const float beta = Exp2(dot - m_new);

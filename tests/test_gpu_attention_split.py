@@ -57,6 +57,42 @@ def test_dense_pieces_match_oracle(gpu, H, D, ps, lengths):
     pool.close()
 
 
+@pytest.mark.parametrize("bad", [np.nan, -np.inf])
+def test_nonfinite_keys_of_whole_pieces(gpu, bad):
+    """Pieces (of 128 slots here) whose logits are all NaN or -inf: the output
+    is NaN, or what the other tokens give, as of an unsplit head (the captured
+    step)."""
+    import torch
+    H, D, ps, lengths = 2, 128, 16, [3000, 3000, 500]
+    batch = gpu.SyntheticBatch(H, D, ps, lengths, seed=21)
+    keys = batch.key_pool.reshape(batch.capacity, ps, H, D)
+    queries = np.abs(batch.queries) + np.float32(0.1)  # (with -inf keys: logits of -inf)
+    offs, ids = batch.cand_offsets, batch.cand_ids
+    keys[ids[offs[0] + 64:offs[0] + 80], :, 0] = bad   # request 0, head 0: slots 1024-1279
+    keys[ids[offs[0] + 80], :8, 1] = -np.inf           # head 1: a piece's first eight
+    keys[ids[offs[1]:offs[2]], :, 1] = bad             # request 1, head 1: every slot
+    pool = gpu.DevicePagePool(H, D, ps, batch.capacity)
+    batch.upload(pool)
+    dev = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (queries, offs, ids)]
+    split, whole = (torch.full((3, H * D), 7.0, device="cuda") for _ in range(2))
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    gpu.dense_run_batch_device(pool, 3, *[t.data_ptr() for t in dev], split.data_ptr(),
+                               side.cuda_stream)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=side):
+        gpu.dense_run_batch_device(pool, 3, *[t.data_ptr() for t in dev], whole.data_ptr(),
+                                   side.cuda_stream)
+    graph.replay()
+    torch.cuda.synchronize()
+    split, whole = (t.cpu().numpy().reshape(3, H, D) for t in (split, whole))
+    assert np.isnan(whole[0, 0]).all() == np.isnan(bad) and not whole[1, 1].any()
+    assert np.array_equal(np.isnan(split), np.isnan(whole))
+    ok = ~np.isnan(whole)
+    assert np.abs(split[ok] - whole[ok]).max() <= 1e-4
+    pool.close()
+
+
 def test_captured_dense_step(gpu):
     import torch
     H, D, ps = 2, 128, 16
