@@ -107,6 +107,9 @@ __device__ __forceinline__ void WriteBounds(double s_hat, double abs_prefix, dou
   const double at_up = abs_prefix * (1.0 + 0x1p-40) + dn * dn * 0x1p-52 * abs_p;
   double err = u * at_up / (1.0 - dn * u) + dn * 0x1p-52 * abs_p + dn * 0x1p-149;
   err *= 1.001;
+  // Where a prefix may pass the float range the chain may overflow, which the
+  // double sums do not show; sum |T_i| bounds every prefix.
+  if (!(at_up < 0x1p127)) err = INFINITY;
   WriteInterval(s_hat, err, scale, mid_out, lo_out, hi_out, c);
 }
 

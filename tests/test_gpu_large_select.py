@@ -112,3 +112,31 @@ def test_scores_of_a_device_step_stay_exact(gpu):
             ctx.device_status()
         assert not out.cpu().numpy().any()
     pool.close()
+
+
+@pytest.mark.parametrize("n", [40, 300, 2100])
+def test_a_chain_that_overflows(gpu, n):
+    """A page whose fp32 chain passes the float range and stays infinite, though
+    its sum is 0, scores above a page of a large finite score."""
+    H, D, k = 4, 64, 1
+    E = H * D
+    rng = np.random.default_rng(n)
+    keys, values = (rng.standard_normal((n, E)).astype(np.float32) for _ in range(2))
+    summ = keys.copy()
+    summ[7] = 0.0
+    summ[7, 0] = 8e35
+    summ[11] = 0.0
+    summ[11, :4] = 3e38, 3e38, -3e38, -3e38
+    query, ones, ids = np.ones((1, E), np.float32), np.ones(n, np.int32), np.arange(n, dtype=np.int32)
+    offsets = np.array([0, n], np.int32)
+    with gpu.DevicePagePool(H, D, 1, n) as pool:
+        pool.upload_pages(ids, ones, ids.astype(np.int64) * E, keys, values, summ)
+        with gpu.SparseContext(pool, k, 1, n, k) as ctx:
+            got = ctx.run_batch(query, offsets, ids, output_mode=gpu.OUTPUT_OUTPUTS,
+                                want_ids=True)
+            assert ctx.last_launch()["certified"] == 1
+    _, want, outs = orc.sparse_batch(query, keys.reshape(n, 1, E), values.reshape(n, 1, E), summ,
+                                     ones, offsets, ids, H, D, 1, k)
+    assert want[0].tolist() == [11]
+    assert got["selected"][0].tolist() == [11]
+    assert orc.max_abs_diff(got["outputs"], outs) <= 1e-4
