@@ -719,8 +719,14 @@ __device__ __forceinline__ void SelectCertifiedRequest(
       PutTagged(words, assist.epoch, static_cast<uint32_t>(share ? nopen : 0));
     }
   }
+  // (the exact kernels then chain every candidate)
+  auto defer = [&] {
+    if (tid != 0) return;
+    if (exact_pages != nullptr) atomicAdd(exact_pages, n);
+    emit_count(kUndecided);
+  };
   if (nopen > Shared::kOpen) {
-    if (tid == 0) emit_count(kUndecided);
+    defer();
     return;
   }
   auto* order = &sh.b;
@@ -775,7 +781,7 @@ __device__ __forceinline__ void SelectCertifiedRequest(
       order = &sh.a;
       nopen = sh.nopen;
       if (nopen > Shared::kOpen) {
-        if (tid == 0) emit_count(kUndecided);
+        defer();
         return;
       }
     }
