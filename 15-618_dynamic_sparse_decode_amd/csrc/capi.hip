@@ -1520,8 +1520,8 @@ dsdk::FusedArgs FusedStepArgs(const PoolView& v, const StepLaunch& L) {
   return a;
 }
 
-// The wide step's arguments (dsdk::WideArgs): the fused step's, the score
-// slices of the stand-alone score kernel, and its scratch.
+// The wide step's arguments (dsdk::WideArgs): the fused step's, its score
+// slices and its scratch.
 dsdk::WideArgs WideStepArgs(const PoolView& v, const StepLaunch& L) {
   dsdk::WideArgs w;
   w.a = FusedStepArgs(v, L);
@@ -2741,7 +2741,7 @@ int dsd_sparse_last_launch(const dsd_sparse_ctx* ctx, dsd_launch_info* out) {
       out->multi_pass = dsdk::FusedStepMultiPass(v, L.max_n, hpw) ? 1 : 0;
       out->grid = dsdk::FusedStepGrid(v, L.batch, hpw);
     } else if (L.certified && v.elements == 4096) {
-      const int per = dsdk::ScorePagesPerGroup(L.total);
+      const int per = dsdk::ScoreLaunchPages(L.total);
       out->score_pages_per_group = per;
       out->grid = L.batch * ((L.max_n + per - 1) / per);
     }

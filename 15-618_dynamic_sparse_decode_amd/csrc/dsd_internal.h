@@ -346,7 +346,9 @@ int FusedStepStampsPerGroup();
 // Whether a launch takes FusedStepKernel<true> (a slice spans several score
 // passes of 8 pages, so each pass's rows load while the previous one reduces).
 bool FusedStepMultiPass(const PoolView& pool, int max_candidates, int heads_per_group);
-// Pages per workgroup of the stand-alone score kernel (E = 4096).
+// Pages per workgroup of the stand-alone score kernel (E = 4096), and per
+// score slice of the wide step.
+int ScoreLaunchPages(int total_candidates);
 int ScorePagesPerGroup(int total_candidates);
 void LaunchFusedStep(const PoolView& pool, const FusedArgs& args, hipStream_t stream);
 

@@ -46,6 +46,8 @@
 // 0 of each workgroup polls its request's words directly (a cached read
 // first, then coherent re-reads of the words whose tag is not yet current,
 // with a short sleep between rounds) and shares them through LDS.
+#include <algorithm>
+
 #include "dsd_internal.h"
 #include "step_common.h"
 #include "score_slice.h"
@@ -1038,16 +1040,7 @@ void LaunchScorePages(const PoolView& pool, const float* d_queries, const int* d
                       FailReport fail, hipStream_t stream) {
   if (batch <= 0 || max_candidates <= 0 || total_candidates <= 0) return;
   if (pool.elements != kFE) throw std::invalid_argument("ScorePages needs E = 4096");
-  // One round of workgroups, a few CUs short of full: a workgroup fills a CU,
-  // its first rows wait for a chain of loads, and a round that ragged requests
-  // fill a little past the last CU of one XCD costs a whole one more (8
-  // requests of 60000-130000 tokens, top 64: the step 254 us; with two full
-  // rounds, ScorePagesPerGroup, 296; 4 requests of 65536-131072: 137 and 138).
-  // Beyond 256 pages each, several rounds.
-  constexpr int kRound = 224, kMostPages = 256;
-  const int even = (total_candidates + kRound - 1) / kRound;
-  const int per = even > kMostPages ? ScorePagesPerGroup(total_candidates)
-                                    : (even + kFPagesPerPass - 1) / kFPagesPerPass * kFPagesPerPass;
+  const int per = ScoreLaunchPages(total_candidates);
   FusedArgs a;
   a.queries = d_queries;
   a.cand_offsets = d_cand_offsets;
@@ -1062,6 +1055,19 @@ void LaunchScorePages(const PoolView& pool, const float* d_queries, const int* d
   const dim3 grid((max_candidates + per - 1) / per, batch);
   hipLaunchKernelGGL(ScorePagesKernel, grid, dim3(kFThreads), 0, stream, pool, a, per);
   DSD_HIP_CHECK(hipGetLastError());
+}
+
+int ScoreLaunchPages(int total_candidates) {
+  // One round of workgroups, a few CUs short of full: a workgroup fills a CU,
+  // its first rows wait for a chain of loads, and a round that ragged requests
+  // fill a little past the last CU of one XCD costs a whole one more (8
+  // requests of 60000-130000 tokens, top 64: the step 254 us; with two full
+  // rounds, ScorePagesPerGroup, 296; 4 requests of 65536-131072: 137 and 138).
+  // Beyond 256 pages each, several rounds.
+  constexpr int kRound = 224, kMostPages = 256;
+  const int even = std::max(1, (total_candidates + kRound - 1) / kRound);
+  return even > kMostPages ? ScorePagesPerGroup(total_candidates)
+                           : (even + kFPagesPerPass - 1) / kFPagesPerPass * kFPagesPerPass;
 }
 
 int ScorePagesPerGroup(int total_candidates) {

@@ -49,6 +49,10 @@ def test_random_batches(gpu, H, D, n, k):
     info, _ = run(gpu, keys, values, queries, offsets, ids, H, D, k)
     assert info["certified"] == (1 if k <= 1024 else 0)
     assert info["fused"] == 0 and info["wide"] == 0
+    if H * D == 4096:  # the float score passes' launch: 224 workgroups, whole passes of 8
+        per = -(-sum(n) // (224 * 8)) * 8
+        assert info["score_pages_per_group"] == per == 24
+        assert info["grid"] == len(n) * -(-max(n) // per)
 
 
 @pytest.mark.parametrize("kind", ["near", "pairs", "many_equal", "zero_query", "infinite"])
