@@ -130,8 +130,8 @@ struct PinnedBuffer {
 
 // The scratch of an attention launch that spreads heads over workgroups
 // (dsdk::AttentionArgs::piece_words, then its counters), in 64-bit words.  It
-// lies behind another buffer of its owner and exists from the start: made by
-// the first call that needed it, it took 50 us of a dense step of 26.
+// lies behind another buffer of its owner and exists from the start: allocated
+// by the first dense step that needed it, it made that step 94 us, 22 the next.
 size_t PieceScratchWords() {
   return dsdk::AttentionPieceWords() + static_cast<size_t>(dsdk::AttentionPieceCounters()) / 2;
 }
@@ -248,10 +248,21 @@ struct dsd_pool {
   PinnedBuffer<float> h_dense_q, h_dense_out;
   PinnedBuffer<int> h_dense_offsets, h_dense_ids;
   hipEvent_t dense_start = nullptr, dense_stop = nullptr;
-  // The dense attention's pieces (attention.hip): one scratch per pool (2 MiB,
-  // behind the keys).  piece_ev marks the end of the last launch that used it,
-  // and every launch waits for it, so calls on several streams take turns.
+  // The dense attention's pieces (attention.hip): kDenseScratches scratches of
+  // 2 MiB, behind the summaries.  The first streams to use the pool own one
+  // each: their steps follow one another by the stream's own order and no
+  // stream waits for another's.  (A stream made later with the handle of a
+  // destroyed one takes its scratch: what ran on a destroyed stream has ended,
+  // or HIP does not say that it ever will.)  Every other stream uses the last
+  // scratch, whose steps take turns by piece_ev.  An event record per step
+  // would order them all, and did: it idles the stream for 2.5 us, as long as
+  // a small step (one request of 64 tokens: 6.8 us a step, 5.0 without).
+  // piece_mu: host threads that each have a stream of their own.
+  static constexpr int kDenseScratches = 4;
   unsigned long long* pieces = nullptr;
+  hipStream_t piece_owner[kDenseScratches - 1] = {};
+  int piece_owners = 0;
+  std::mutex piece_mu;
   hipEvent_t piece_ev = nullptr;
   uint64_t* k_offsets = nullptr;  // [capacity] element offset of each page
   uint64_t* v_offsets = nullptr;
@@ -418,21 +429,23 @@ int dsd_pool_create(int num_heads, int head_dim, int page_size,
       const size_t sum_bytes = static_cast<size_t>(capacity_pages) *
                                static_cast<size_t>(v.elements) * sizeof(float);
       const bool pieces = dsdk::AttentionPieceRoom(v, 1, 0) > 0;
-      const size_t keys_end = (kv_bytes + 255) / 256 * 256;
-      const size_t piece_bytes = pieces ? PieceScratchWords() * sizeof(unsigned long long) : 0;
-      DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.keys), keys_end + piece_bytes));
+      const size_t sum_end = (sum_bytes + 255) / 256 * 256;
+      const size_t zero_bytes =
+          pieces ? sum_end + dsd_pool::kDenseScratches * PieceScratchWords() *
+                                 sizeof(unsigned long long)
+                 : sum_bytes;
+      DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.keys), kv_bytes));
+      DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.values), kv_bytes));
+      DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.summaries), zero_bytes));
       if (pieces) {
         pool->pieces = reinterpret_cast<unsigned long long*>(
-            reinterpret_cast<unsigned char*>(v.keys) + keys_end);
-        DSD_HIP_CHECK(hipMemsetAsync(pool->pieces, 0, piece_bytes, pool->stream));
+            reinterpret_cast<unsigned char*>(v.summaries) + sum_end);
       }
-      DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.values), kv_bytes));
-      DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.summaries), sum_bytes));
       DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.token_counts),
                               sizeof(int) * static_cast<size_t>(capacity_pages)));
       DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.live),
                               static_cast<size_t>(capacity_pages)));
-      DSD_HIP_CHECK(hipMemsetAsync(v.summaries, 0, sum_bytes, pool->stream));
+      DSD_HIP_CHECK(hipMemsetAsync(v.summaries, 0, zero_bytes, pool->stream));
       DSD_HIP_CHECK(hipMemsetAsync(v.token_counts, 0,
                                    sizeof(int) * static_cast<size_t>(capacity_pages),
                                    pool->stream));
@@ -2853,21 +2866,29 @@ StaticScratch& StaticScratchOn(int device) {
 
 
 // The dense attention on stream s: spread over workgroups where few requests
-// would leave the chip idle, on the pool's one piece scratch (so it first
-// waits for the last launch that used it).  A captured launch has no place
-// in that order and stays unsplit.
+// would leave the chip idle, on the stream's scratch (dsd_pool::pieces).  A
+// captured launch has no place in an order of launches and stays unsplit.
 void LaunchDense(dsd_pool* pool, dsdk::AttentionArgs* a, hipStream_t s) {
   const bool capturing = s != nullptr && StreamCapturing(s);
   if (!capturing && pool->pieces != nullptr) {
     a->piece_room = dsdk::AttentionPieceRoom(pool->view, a->batch, 0);
   }
-  if (a->piece_room > 0) {
-    a->piece_words = pool->pieces;
-    a->piece_arrivals = PieceArrivals(pool->pieces);
+  if (a->piece_room == 0) {
+    dsdk::LaunchAttention(pool->view, *a, s);
+    return;
   }
-  if (a->piece_room > 0) DSD_HIP_CHECK(hipStreamWaitEvent(s, pool->piece_ev, 0));
+  std::lock_guard<std::mutex> lock(pool->piece_mu);
+  constexpr int kShared = dsd_pool::kDenseScratches - 1;
+  int slot = 0;
+  while (slot < pool->piece_owners && pool->piece_owner[slot] != s) ++slot;
+  // (hipStreamPerThread is one handle for a stream of each thread)
+  if (s == hipStreamPerThread) slot = kShared;
+  if (slot == pool->piece_owners && slot < kShared) pool->piece_owner[pool->piece_owners++] = s;
+  a->piece_words = pool->pieces + static_cast<size_t>(slot) * PieceScratchWords();
+  a->piece_arrivals = PieceArrivals(a->piece_words);
+  if (slot == kShared) DSD_HIP_CHECK(hipStreamWaitEvent(s, pool->piece_ev, 0));
   dsdk::LaunchAttention(pool->view, *a, s);
-  if (a->piece_room > 0) DSD_HIP_CHECK(hipEventRecord(pool->piece_ev, s));
+  if (slot == kShared) DSD_HIP_CHECK(hipEventRecord(pool->piece_ev, s));
 }
 
 }  // namespace

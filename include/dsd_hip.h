@@ -603,7 +603,13 @@ int dsd_dense_run_batch(dsd_pool* pool, int batch, const float* queries,
                         const int* cand_offsets, const int* cand_ids,
                         float* outputs, double* kernel_ms);
 
-/* Device-resident dense step on `stream` (NULL = default stream). */
+/* Device-resident dense step on `stream` (NULL = default stream).  Steps on
+ * one pool may run on several streams and be enqueued by several host threads
+ * (each on a stream of its own, with no other call on the pool meanwhile):
+ * the pool holds scratch for the first three streams that use it, whose steps
+ * are independent of each other; the steps of all further streams follow one
+ * another.  Under graph capture a head's tokens are not spread over
+ * workgroups: outputs agree with an eager step's within rounding. */
 int dsd_dense_run_batch_device(dsd_pool* pool, int batch,
                                const float* d_queries,
                                const int* d_cand_offsets,

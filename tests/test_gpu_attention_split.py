@@ -1,6 +1,6 @@
 """Attention whose heads are spread over several workgroups (attention.hip):
 pieces at their edges, the scratch left clean for the next launch, launches on
-two streams, and a captured step.
+several streams and from several threads, and a captured step.
 
 Tolerance: outputs within 1e-4 of the oracle, the path's bar.  The rounding
 bound behind it: a logit is a dot of D <= 256 products summed in fp32 along
@@ -10,6 +10,9 @@ and an output moves by at most twice that times the largest |value| (about 5)
 in the worst case.  Merging pieces adds one exponential and one product per
 piece, the same as merging waves.
 """
+import threading
+import time
+
 import numpy as np
 import pytest
 
@@ -54,6 +57,100 @@ def test_dense_pieces_match_oracle(gpu, H, D, ps, lengths):
     assert orc.max_abs_diff(host, np.asarray(want).reshape(host.shape)) <= 1e-4
     for out in outs:
         assert np.array_equal(out.cpu().numpy().view(np.uint32), host.view(np.uint32))
+    pool.close()
+
+
+def dense_inputs(H, D, ps, lengths, seed):
+    """One pool's list of device batches: its requests with other queries."""
+    import torch
+    rng = np.random.default_rng(seed)
+    return [torch.from_numpy(rng.standard_normal((len(lengths), H * D)).astype(np.float32)).cuda()
+            for _ in range(6)]
+
+
+def test_steps_on_many_streams_and_threads(gpu):
+    """Six host threads, each with a stream of its own (more than there are
+    scratches of streams), enqueue split steps on one pool at once: the bits of
+    the steps one after the other."""
+    import torch
+    H, D, ps, lengths = 4, 128, 16, [6000, 1700]
+    batch, pool = make_pool(gpu, H, D, ps, lengths, seed=31)
+    queries = dense_inputs(H, D, ps, lengths, 32)
+    offs, ids = (torch.from_numpy(a).cuda() for a in (batch.cand_offsets, batch.cand_ids))
+    streams = [torch.cuda.Stream() for _ in queries]
+    outs = [[torch.zeros(2, H * D, device="cuda") for _ in range(25)] for _ in queries]
+    torch.cuda.synchronize()
+
+    def step(i, out):
+        gpu.dense_run_batch_device(pool, 2, queries[i].data_ptr(), offs.data_ptr(),
+                                   ids.data_ptr(), out.data_ptr(), streams[i].cuda_stream)
+
+    want = []
+    for i in range(len(queries)):
+        out = torch.zeros(2, H * D, device="cuda")
+        torch.cuda.synchronize()
+        step(i, out)
+        torch.cuda.synchronize()
+        want.append(out.cpu().numpy().view(np.uint32))
+    start = threading.Barrier(len(queries))
+
+    def run(i):
+        start.wait()
+        for out in outs[i]:
+            step(i, out)
+
+    threads = [threading.Thread(target=run, args=(i,)) for i in range(len(queries))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for i, mine in enumerate(outs):
+        for out in mine:
+            assert np.array_equal(out.cpu().numpy().view(np.uint32), want[i]), i
+    pool.close()
+
+
+def test_a_stream_does_not_wait_for_another_streams_step(gpu):
+    import torch
+    H, D, ps, lengths = 4, 128, 16, [6000]
+    batch, pool = make_pool(gpu, H, D, ps, lengths, seed=33)
+    query = dense_inputs(H, D, ps, lengths, 34)[0]
+    offs, ids = (torch.from_numpy(a).cuda() for a in (batch.cand_offsets, batch.cand_ids))
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    out = {s: torch.zeros(1, H * D, device="cuda") for s in (a, b)}
+    scratch = torch.zeros(64, device="cuda")
+    torch.cuda.synchronize()
+
+    def step(s):
+        gpu.dense_run_batch_device(pool, 1, query.data_ptr(), offs.data_ptr(), ids.data_ptr(),
+                                   out[s].data_ptr(), s.cuda_stream)
+
+    def b_ends_first(work):
+        begin = time.perf_counter()
+        with torch.cuda.stream(a):
+            torch.cuda._sleep(200_000_000)
+        step(a)
+        work()
+        b.synchronize()
+        b_took = time.perf_counter() - begin
+        a.synchronize()
+        a_took = time.perf_counter() - begin
+        print(f"[streams] a {a_took * 1e3:.2f} ms, b {b_took * 1e3:.2f} ms", flush=True)
+        return b_took < a_took / 2
+
+    def plain():
+        with torch.cuda.stream(b):
+            scratch.add_(1.0)
+
+    step(a)
+    step(b)
+    plain()
+    torch.cuda.synchronize()
+    if not b_ends_first(plain):
+        pytest.skip("the two streams share a hardware queue")
+    assert b_ends_first(lambda: step(b))
+    assert torch.equal(out[a], out[b])
     pool.close()
 
 
