@@ -197,12 +197,13 @@ __global__ __launch_bounds__(kAttnThreads) void AttentionKernel(
 // the others publish (m, l, acc) as tagged words, and the workgroup that
 // arrives last at the request's counter merges them in piece order (the
 // result does not depend on which workgroup that is) and zeroes the words and
-// the counter for the next launch on the same scratch.  The words carry their
-// own tag, so nothing orders them but the tag (no fence, which would write
+// the counter for the next launch on the same scratch.  The words carry the
+// launch's tag, so nothing orders them but the tag (no fence, which would write
 // back the XCD's L2).  Every wait ends: the merging workgroup waits only for
 // words whose stores were issued before their workgroup arrived; the poll is
-// bounded anyway and a word that never came reads as NaN.  The request above
-// takes 185 us (5.8 TB/s).
+// bounded anyway, a word that never came is reported (kFailWait, zero outputs;
+// NaN from a dense step, which reports nothing) and not taken for a later
+// launch's.  The request above takes 185 us (5.8 TB/s).
 //
 // Either way the list's ids and token counts are staged in LDS, 256 entries
 // at a time, instead of a chain of two loads ahead of every chunk's rows
@@ -293,10 +294,18 @@ __device__ __forceinline__ bool FindPiece(const AttentionArgs& a, int ps, int g,
   return false;
 }
 
-__device__ __forceinline__ float TakeWord(unsigned long long* p) {
+// A published word's value once it carries the launch's tag, zeroed for the
+// next launch; *late when it never did (the word stays: the next launch has
+// another tag).
+__device__ __forceinline__ float TakeWord(const AttentionArgs& args, unsigned long long* p,
+                                          int* late) {
+  const unsigned tag = args.piece_tag | args.piece_wait_mask;
   unsigned long long w = LoadWord(p);
-  for (unsigned i = 0; (w >> 32) == 0; ++i) {
-    if (i >= (1u << 20)) return NAN;
+  for (unsigned i = 0; static_cast<unsigned>(w >> 32) != tag; ++i) {
+    if (i >= args.piece_spin_limit || *static_cast<volatile int*>(late) != 0) {
+      *late = 1;
+      return 0.0f;
+    }
     __builtin_amdgcn_s_sleep(1);
     w = LoadWord(p);
   }
@@ -317,6 +326,7 @@ __global__ __launch_bounds__(WAVES * kWave) void AttentionFastKernel(
   __shared__ float s_pm[kAttnMaxPieces];
   __shared__ float s_pl[kAttnMaxPieces];
   __shared__ int s_last;
+  __shared__ int s_late;
   const int h = blockIdx.x;
   const int tid = threadIdx.x;
   const int ps = pool.page_size;
@@ -377,10 +387,10 @@ __global__ __launch_bounds__(WAVES * kWave) void AttentionFastKernel(
       (static_cast<size_t>(blockIdx.y) * pool.num_heads + h) * static_cast<size_t>(D + 2);
   if (tid < D) {
     if (tid == 0) {
-      PutTagged(words, 1u, __float_as_uint(mx));
-      PutTagged(words + 1, 1u, __float_as_uint(lt));
+      PutTagged(words, args.piece_tag, __float_as_uint(mx));
+      PutTagged(words + 1, args.piece_tag, __float_as_uint(lt));
     }
-    PutTagged(words + 2 + tid, 1u, __float_as_uint(at));
+    PutTagged(words + 2 + tid, args.piece_tag, __float_as_uint(at));
   }
   __syncthreads();
   unsigned* arrivals = args.piece_arrivals + static_cast<size_t>(p.r) * pool.num_heads + h;
@@ -388,6 +398,7 @@ __global__ __launch_bounds__(WAVES * kWave) void AttentionFastKernel(
     const unsigned prev =
         __hip_atomic_fetch_add(arrivals, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     s_last = prev == static_cast<unsigned>(p.pieces - 1) ? 1 : 0;
+    s_late = 0;
   }
   __syncthreads();
   if (s_last == 0) return;
@@ -398,8 +409,8 @@ __global__ __launch_bounds__(WAVES * kWave) void AttentionFastKernel(
   const size_t stride = static_cast<size_t>(pool.num_heads) * (D + 2);
   unsigned long long* first = words - static_cast<size_t>(p.index) * stride;
   for (int i = tid; i < p.pieces; i += kThreads) {
-    s_pm[i] = TakeWord(first + i * stride);
-    s_pl[i] = TakeWord(first + i * stride + 1);
+    s_pm[i] = TakeWord(args, first + i * stride, &s_late);
+    s_pl[i] = TakeWord(args, first + i * stride + 1, &s_late);
   }
   __syncthreads();
   float m = -INFINITY;
@@ -411,7 +422,7 @@ __global__ __launch_bounds__(WAVES * kWave) void AttentionFastKernel(
   at = 0.0f;
   if (grp < kGroups) {
     for (int i = grp; i < p.pieces; i += kGroups) {
-      const float a = TakeWord(first + i * stride + 2 + d);
+      const float a = TakeWord(args, first + i * stride + 2 + d, &s_late);
       const float sw = s_pm[i] == -INFINITY ? 0.0f : Exp2(s_pm[i] - m);
       lt = fmaf(s_pl[i], sw, lt);
       at = fmaf(a, sw, at);
@@ -432,7 +443,14 @@ __global__ __launch_bounds__(WAVES * kWave) void AttentionFastKernel(
       at += sh.acc[i][tid];
     }
     // (no piece with a maximum: zeros, as for an unsplit head)
-    out[tid] = lt == 0.0f || m == -INFINITY ? 0.0f : at / lt;
+    float o = lt == 0.0f || m == -INFINITY ? 0.0f : at / lt;
+    if (s_late != 0) {
+      // Zeros and a report, as the step's other waits; NaN where the launch
+      // has nowhere to report to.
+      if (tid == 0) ReportFailure(args.fail, kFailWait);
+      o = args.fail.word != nullptr ? 0.0f : NAN;
+    }
+    out[tid] = o;
   }
 }
 
@@ -550,7 +568,7 @@ void LaunchAttention(const PoolView& pool, const AttentionArgs& args,
   if (shape.fn != nullptr) {
     if (args.piece_room < 0 || args.piece_room > kAttnMaxPieces ||
         (args.piece_room > 0 &&
-         (args.piece_words == nullptr || args.piece_arrivals == nullptr ||
+         (args.piece_words == nullptr || args.piece_arrivals == nullptr || args.piece_tag == 0 ||
           static_cast<long long>(args.batch) * pool.num_heads > kAttnPieceCounters ||
           static_cast<long long>(args.batch + args.piece_room) * pool.num_heads * (D + 2) >
               static_cast<long long>(kAttnPieceWords)))) {

@@ -262,6 +262,7 @@ struct dsd_pool {
   unsigned long long* pieces = nullptr;
   hipStream_t piece_owner[kDenseScratches - 1] = {};
   int piece_owners = 0;
+  unsigned piece_tag = 0;  // of the last launch on any of them
   std::mutex piece_mu;
   hipEvent_t piece_ev = nullptr;
   uint64_t* k_offsets = nullptr;  // [capacity] element offset of each page
@@ -1500,6 +1501,10 @@ void EnqueueAttentionStage(const PoolView& v, const StepLaunch& L, hipStream_t s
   a.piece_room = L.piece_room;
   a.piece_words = L.piece_words;
   a.piece_arrivals = L.piece_arrivals;
+  a.piece_tag = L.epoch;
+  a.piece_wait_mask = L.never_ready ? 0x80000000u : 0u;
+  a.piece_spin_limit = L.spin_limit;
+  a.fail = L.Fail();
   dsdk::LaunchAttention(v, a, s);
 }
 
@@ -1744,7 +1749,8 @@ struct dsd_sparse_ctx {
           "decode step: a selection slot held an id that is not one of the request's "
           "candidates (written as -1, not attended)");
     }
-    throw std::runtime_error("fused decode step: wait for page selection timed out");
+    throw std::runtime_error(
+        "decode step: wait for another workgroup's page selection or attention timed out");
   }
 
   // A launch over the context's scratch; the caller fills inputs and
@@ -2886,6 +2892,8 @@ void LaunchDense(dsd_pool* pool, dsdk::AttentionArgs* a, hipStream_t s) {
   if (slot == pool->piece_owners && slot < kShared) pool->piece_owner[pool->piece_owners++] = s;
   a->piece_words = pool->pieces + static_cast<size_t>(slot) * PieceScratchWords();
   a->piece_arrivals = PieceArrivals(a->piece_words);
+  if (++pool->piece_tag == 0) pool->piece_tag = 1;
+  a->piece_tag = pool->piece_tag;
   if (slot == kShared) DSD_HIP_CHECK(hipStreamWaitEvent(s, pool->piece_ev, 0));
   dsdk::LaunchAttention(pool->view, *a, s);
   if (slot == kShared) DSD_HIP_CHECK(hipEventRecord(pool->piece_ev, s));

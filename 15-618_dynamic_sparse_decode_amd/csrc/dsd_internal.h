@@ -268,8 +268,15 @@ struct AttentionArgs {
   // AttentionPieceRoom() > 0 and the scratch for it, AttentionPieceWords()
   // words and AttentionPieceCounters() counters, all zero before the first
   // launch that uses them (each launch leaves them zero).  Launches on one
-  // scratch must not overlap.
+  // scratch must not overlap.  piece_tag: non-zero, another one for every
+  // launch on the scratch (a graph's replays share the captured one).  A wait
+  // polls piece_spin_limit times, for the tag with piece_wait_mask added (a
+  // mask makes every wait give up), and reports to `fail`.
   int piece_room = 0;
+  unsigned piece_tag = 0;
+  unsigned piece_wait_mask = 0;
+  unsigned piece_spin_limit = 1u << 20;
+  FailReport fail;
   unsigned long long* piece_words = nullptr;
   unsigned* piece_arrivals = nullptr;
 };

@@ -369,10 +369,13 @@ int dsd_sparse_step_stamps(const dsd_sparse_ctx* ctx, int* grid, int* per_group,
  * src/cuda/sparse_batched_attention.cu:600-608). */
 int dsd_sparse_device_status(dsd_sparse_ctx* ctx);
 
-/* The single-launch step's cross-workgroup waits poll at most spin_limit
+/* The cross-workgroup waits of a step (a single launch's, and the merge of
+ * heads whose tokens are spread over workgroups) poll at most spin_limit
  * times (default 2^17, about 0.1-0.3 s) before they give up: the step then
- * selects nothing for the request, its outputs are zeros and the failure is
- * reported (DSD_ERR_RUNTIME).  never_ready != 0 makes every wait look for a
+ * selects nothing for the request, or does not merge its heads, its outputs
+ * are zeros and the failure is reported (DSD_ERR_RUNTIME).  The select's wait
+ * for its helper workgroups polls at most 256 times and falls back to exact
+ * scores, with no failure.  never_ready != 0 makes every wait look for a
  * tag no workgroup writes, so every wait gives up: a test hook for that
  * path, which never reaches a GPU hang.  No reference counterpart. */
 int dsd_sparse_set_wait_limit(dsd_sparse_ctx* ctx, unsigned spin_limit, int never_ready);

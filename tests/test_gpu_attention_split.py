@@ -256,3 +256,38 @@ def test_sparse_step_with_pieces_eager_and_captured(gpu):
             assert np.array_equal(out.cpu().numpy().view(np.uint32), eager[i].view(np.uint32))
         ctx.device_status()
     pool.close()
+
+
+def test_a_merge_that_gives_up_is_reported_and_recovers(gpu):
+    """Every wait of the merge gives up (it polls for a tag nobody writes): the
+    split requests' outputs are zeros and the step reports it; what it left in
+    the scratch is not taken for the next step's."""
+    import torch
+    H, D, ps, k = 8, 128, 16, 40
+    batch, pool = make_pool(gpu, H, D, ps, [2100, 90, 700], seed=13)
+    dev = [torch.from_numpy(a).cuda() for a in (batch.queries, batch.cand_offsets,
+                                                batch.cand_ids)]
+    other = torch.from_numpy(np.ascontiguousarray(batch.queries[::-1])).cuda()
+    total, most = batch.total_candidates, batch.max_candidates
+    with gpu.SparseContext(pool, k, 3, total, 3 * k) as ctx:
+        def step(queries):
+            out = torch.full((3, H * D), 7.0, device="cuda")
+            torch.cuda.synchronize()
+            ctx.run_batch_device(3, total, most, queries.data_ptr(), dev[1].data_ptr(),
+                                 dev[2].data_ptr(), out.data_ptr())
+            torch.cuda.synchronize()
+            return out.cpu().numpy()
+
+        good, turned = step(dev[0]), step(other)
+        ctx.device_status()
+        ctx.set_wait_limit(4, True)
+        late = step(other)
+        with pytest.raises(gpu.DsdError, match="timed out"):
+            ctx.device_status()
+        assert not late[0].any() and not late[2].any()  # 640 slots each
+        assert np.array_equal(late[1].view(np.uint32), turned[1].view(np.uint32))  # one piece
+        ctx.set_wait_limit(1 << 17, False)
+        for queries, want in ((dev[0], good), (other, turned)):
+            assert np.array_equal(step(queries).view(np.uint32), want.view(np.uint32))
+        ctx.device_status()
+    pool.close()
