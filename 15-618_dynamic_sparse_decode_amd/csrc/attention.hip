@@ -211,8 +211,6 @@ __global__ __launch_bounds__(kAttnThreads) void AttentionKernel(
 // ---------------------------------------------------------------------------
 constexpr int kAttnTile = 256;       // list entries per LDS tile
 constexpr int kAttnMaxPieces = 256;  // per request (room), the merge's LDS
-constexpr size_t kAttnPieceWords = 1u << 18;
-constexpr int kAttnPieceCounters = 4096;
 // Workgroups of 8 waves the chip runs at once (two per CU).
 constexpr int kAttnRound = 512;
 constexpr int kAttnWhole = 3;
@@ -528,9 +526,6 @@ AttnShape FastShape(int head_dim, bool wide) {
 }
 
 }  // namespace
-
-size_t AttentionPieceWords() { return kAttnPieceWords; }
-int AttentionPieceCounters() { return kAttnPieceCounters; }
 
 int AttentionPieceRoom(const PoolView& pool, int batch, long long max_slots) {
   const AttnShape shape = FastShape(pool.head_dim, false);

@@ -132,11 +132,10 @@ struct PinnedBuffer {
 // (dsdk::AttentionArgs::piece_words, then its counters), in 64-bit words.  It
 // lies behind another buffer of its owner and exists from the start: allocated
 // by the first dense step that needed it, it made that step 94 us, 22 the next.
-size_t PieceScratchWords() {
-  return dsdk::AttentionPieceWords() + static_cast<size_t>(dsdk::AttentionPieceCounters()) / 2;
-}
+constexpr size_t kPieceScratchWords =
+    dsdk::kAttnPieceWords + static_cast<size_t>(dsdk::kAttnPieceCounters) / 2;
 unsigned* PieceArrivals(unsigned long long* pieces) {
-  return reinterpret_cast<unsigned*>(pieces + dsdk::AttentionPieceWords());
+  return reinterpret_cast<unsigned*>(pieces + dsdk::kAttnPieceWords);
 }
 
 constexpr uint64_t kLargeCopyBytes = 1ull << 20;  // src/device_page_pool.cpp:13
@@ -432,7 +431,7 @@ int dsd_pool_create(int num_heads, int head_dim, int page_size,
       const bool pieces = dsdk::AttentionPieceRoom(v, 1, 0) > 0;
       const size_t sum_end = (sum_bytes + 255) / 256 * 256;
       const size_t zero_bytes =
-          pieces ? sum_end + dsd_pool::kDenseScratches * PieceScratchWords() *
+          pieces ? sum_end + dsd_pool::kDenseScratches * kPieceScratchWords *
                                  sizeof(unsigned long long)
                  : sum_bytes;
       DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.keys), kv_bytes));
@@ -1454,6 +1453,21 @@ bool StepFused(const PoolView& v, bool certified, bool enabled, int max_n, int t
   return certified && enabled && dsdk::FusedStepSupported(v, max_n, top_k);
 }
 
+// Heads spread over workgroups (scratch `pieces`, may be null), except for the
+// shapes of the single launches, whose outputs the three kernels reproduce bit
+// for bit.
+void UsePieces(StepLaunch* L, const PoolView& v, int batch, int max_n, int top_k,
+               unsigned long long* pieces) {
+  if (pieces == nullptr || L->wide_shape || L->fused ||
+      dsdk::FusedStepSupported(v, max_n, top_k)) {
+    return;
+  }
+  L->piece_room = dsdk::AttentionPieceRoom(
+      v, batch, static_cast<long long>(std::max(1, top_k)) * v.page_size);
+  L->piece_words = pieces;
+  L->piece_arrivals = PieceArrivals(pieces);
+}
+
 void EnqueueScoreStage(const PoolView& v, const StepLaunch& L, hipStream_t s) {
   if (L.total <= 0) return;
   if (L.certified) {
@@ -1769,15 +1783,7 @@ struct dsd_sparse_ctx {
                    !dsdk::FusedStepSupported(v, max_n, top_k) &&
                    dsdk::WideStepSupported(v, max_n, top_k);
     L.wide = L.wide_shape && wide_enabled;
-    // Heads spread over workgroups, except for the shapes of the single
-    // launches, whose outputs the three kernels reproduce bit for bit.
-    if (pieces != nullptr && !L.wide_shape && !L.fused &&
-        !dsdk::FusedStepSupported(v, max_n, top_k)) {
-      L.piece_room = dsdk::AttentionPieceRoom(
-          v, batch, static_cast<long long>(std::max(1, top_k)) * v.page_size);
-      L.piece_words = pieces;
-      L.piece_arrivals = PieceArrivals(pieces);
-    }
+    UsePieces(&L, v, batch, max_n, top_k, pieces);
     L.batch = batch;
     L.total = total;
     L.max_n = max_n;
@@ -1945,10 +1951,8 @@ int dsd_sparse_create(dsd_pool* pool, int top_k, int max_batch,
       const size_t rec = 3 * P;
       const bool pieces =
           dsdk::AttentionPieceRoom(pool->view, 1,
-                                   static_cast<long long>(K) * pool->view.page_size) > 0 &&
-          (!dsdk::FusedStepSupported(pool->view, 0, 0) ||
-           max_total_candidates > dsdk::WideStepMaxCandidates());
-      const size_t words = rec + (pieces ? PieceScratchWords() : 0);
+                                   static_cast<long long>(K) * pool->view.page_size) > 0;
+      const size_t words = rec + (pieces ? kPieceScratchWords : 0);
       // The largest fused grid: one head per workgroup.
       const size_t stamps =
           static_cast<size_t>(dsdk::FusedStepGrid(pool->view, static_cast<int>(B), 1)) *
@@ -2817,7 +2821,7 @@ constexpr size_t Align256(size_t bytes) { return (bytes + 255) / 256 * 256; }
 // Byte offsets of the scratch's parts: publication words (3 per candidate),
 // midpoints, lower and upper bounds, selected ids, selected counts, the
 // device epoch, refined-interval words (3 per flagged-page slot of each
-// request).
+// request), the attention's pieces.
 constexpr size_t kStaticRec = 0;
 constexpr size_t kStaticMid =
     Align256(kStaticRec + sizeof(unsigned long long) * 3 * kStaticMaxCandidates);
@@ -2827,12 +2831,14 @@ constexpr size_t kStaticSel = Align256(kStaticHi + sizeof(float) * kStaticMaxCan
 constexpr size_t kStaticCounts = Align256(kStaticSel + sizeof(int) * kStaticMaxSelected);
 constexpr size_t kStaticEpoch = Align256(kStaticCounts + sizeof(int) * kStaticMaxBatch);
 constexpr size_t kStaticRefined = Align256(kStaticEpoch + sizeof(unsigned));
-constexpr size_t kStaticBytes = Align256(
+constexpr size_t kStaticPieces = Align256(
     kStaticRefined + sizeof(unsigned long long) * 3 * dsdk::kFRefineSlots * kStaticMaxBatch);
+constexpr size_t kStaticBytes =
+    Align256(kStaticPieces + sizeof(unsigned long long) * kPieceScratchWords);
 
 }  // namespace
 
-// The scratch of dsd_sparse_run_batch_device_static (2.7 MiB): one copy per
+// The scratch of dsd_sparse_run_batch_device_static (4.7 MiB): one copy per
 // GPU, held until the process ends, shared by every call on that GPU.  Host
 // code never names it except to look up its device address.
 static __device__ __align__(256) unsigned char scratch[kStaticBytes];
@@ -2890,7 +2896,7 @@ void LaunchDense(dsd_pool* pool, dsdk::AttentionArgs* a, hipStream_t s) {
   // (hipStreamPerThread is one handle for a stream of each thread)
   if (s == hipStreamPerThread) slot = kShared;
   if (slot == pool->piece_owners && slot < kShared) pool->piece_owner[pool->piece_owners++] = s;
-  a->piece_words = pool->pieces + static_cast<size_t>(slot) * PieceScratchWords();
+  a->piece_words = pool->pieces + static_cast<size_t>(slot) * kPieceScratchWords;
   a->piece_arrivals = PieceArrivals(a->piece_words);
   if (++pool->piece_tag == 0) pool->piece_tag = 1;
   a->piece_tag = pool->piece_tag;
@@ -2954,6 +2960,8 @@ int dsd_sparse_run_batch_device_static(dsd_pool* pool, int top_k, int batch,
     L.wide_shape = !L.fused && L.certified && batch > 0 &&
                    !dsdk::FusedStepSupported(v, max_candidates, top_k) &&
                    dsdk::WideStepSupported(v, max_candidates, top_k);
+    UsePieces(&L, v, batch, max_candidates, top_k,
+              reinterpret_cast<unsigned long long*>(st.ptr + kStaticPieces));
     L.batch = batch;
     L.total = total_candidates;
     L.max_n = max_candidates;

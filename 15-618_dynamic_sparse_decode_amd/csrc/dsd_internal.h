@@ -248,6 +248,10 @@ void LaunchSelectTopK(const float* d_scores, const int* d_cand_offsets,
                       int max_candidates, int top_k, int* d_selected, int* d_counts,
                       FailReport fail, hipStream_t stream, bool undecided_only = false);
 
+// The scratch of an attention launch that spreads heads over workgroups.
+constexpr size_t kAttnPieceWords = 1u << 18;
+constexpr int kAttnPieceCounters = 4096;
+
 // Fused gather + softmax attention over page lists.  Request r attends over
 // list_ids[start_r .. start_r + count_r): with list_stride > 0, start_r =
 // r*list_stride and count_r = list_counts[r]; otherwise CSR list_offsets.
@@ -265,8 +269,8 @@ struct AttentionArgs {
   // do (bit-identical outputs), for the batches that step takes.
   bool wide_partition = false;
   // Spread each head's tokens over several workgroups (attention.hip):
-  // AttentionPieceRoom() > 0 and the scratch for it, AttentionPieceWords()
-  // words and AttentionPieceCounters() counters, all zero before the first
+  // AttentionPieceRoom() > 0 and the scratch for it, kAttnPieceWords words
+  // and kAttnPieceCounters counters, all zero before the first
   // launch that uses them (each launch leaves them zero).  Launches on one
   // scratch must not overlap.  piece_tag: non-zero, another one for every
   // launch on the scratch (a graph's replays share the captured one).  A wait
@@ -280,8 +284,6 @@ struct AttentionArgs {
   unsigned long long* piece_words = nullptr;
   unsigned* piece_arrivals = nullptr;
 };
-size_t AttentionPieceWords();
-int AttentionPieceCounters();
 // The piece_room for a batch whose lists hold at most max_slots token slots
 // each (0: unknown); 0: one workgroup per (head, request).
 int AttentionPieceRoom(const PoolView& pool, int batch, long long max_slots);

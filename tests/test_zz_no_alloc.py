@@ -31,6 +31,7 @@ def both_entries(gpu, pool, k, queries, offs, ids, static_ids):
     """(context path, static path) results: outputs, and ids/counts."""
     import torch
     B = len(offs) - 1
+    E = pool.elements
     total = int(offs[-1])
     max_n = int(np.max(np.diff(offs)))
     q, o, i = device(queries), device(offs), device(ids)
@@ -87,6 +88,20 @@ def test_static_entry_equals_the_context_entry(gpu, lengths, k, fused):
         n = max(1, batch.batch // 3)
         second = both_entries(gpu, pool, k, *sub_batch(batch, n), static_ids=True)
         assert second["out_st"].shape[0] == n
+
+
+@pytest.mark.parametrize("heads,lengths,k", [
+    (8, [2100, 90, 700], 40),              # heads spread over workgroups
+    (1, [9000], 300),
+    (32, [2500 * PS, 300, 700 * PS], 64),  # beyond 2048 candidates
+])
+def test_static_entry_spreads_heads_as_the_context_entry(gpu, heads, lengths, k):
+    batch = gpu.SyntheticBatch(heads, D, PS, lengths, seed=47)
+    with gpu.DevicePagePool(heads, D, PS, batch.capacity) as pool:
+        batch.upload(pool)
+        for n in (batch.batch, 1):
+            got = both_entries(gpu, pool, k, *sub_batch(batch, n), static_ids=True)
+            assert got["info"]["fused"] == 0 and got["info"]["wide"] == 0
 
 
 def test_static_entry_allocates_nothing(gpu):
