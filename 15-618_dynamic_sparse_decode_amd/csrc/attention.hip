@@ -215,7 +215,7 @@ constexpr int kAttnMaxPieces = 256;  // per request (room), the merge's LDS
 constexpr int kAttnRound = 512;
 constexpr int kAttnWhole = 3;
 
-// Token slots of request b (a malformed or negative length holds none).
+// Token slots of request b (a malformed, negative or overflowing length holds none).
 __device__ __forceinline__ int ListSlots(const AttentionArgs& a, int b, int ps, int* start) {
   int count;
   if (a.list_stride > 0) {
@@ -225,7 +225,7 @@ __device__ __forceinline__ int ListSlots(const AttentionArgs& a, int b, int ps, 
     *start = a.list_offsets[b];
     count = a.list_offsets[b + 1] - *start;
   }
-  return count > 0 ? count * ps : 0;
+  return count > 0 ? max(count * ps, 0) : 0;
 }
 
 struct AttnPiece {
@@ -237,15 +237,53 @@ struct AttnPiece {
   int f1 = 0;
 };
 
+// x of the DPP source lane (step_common.h), 0 where there is none.
+template <int kCtrl, int kRowMask = 0xf>
+__device__ __forceinline__ int DppMoveI(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, kCtrl, kRowMask, 0xf, true);
+}
+
+__device__ __forceinline__ int WaveInclusiveScanI(int x) {
+  x += DppMoveI<kRowShr1>(x);
+  x += DppMoveI<kRowShr2>(x);
+  x += DppMoveI<kRowShr4>(x);
+  x += DppMoveI<kRowShr8>(x);
+  x += DppMoveI<kRowBcast15, 0xa>(x);
+  x += DppMoveI<kRowBcast31, 0xc>(x);
+  return x;
+}
+
+// The largest of the lanes' x >= 0, in every lane.
+__device__ __forceinline__ int WaveMaxI(int x) {
+  x = max(x, DppMoveI<kRowShr1>(x));
+  x = max(x, DppMoveI<kRowShr2>(x));
+  x = max(x, DppMoveI<kRowShr4>(x));
+  x = max(x, DppMoveI<kRowShr8>(x));
+  x = max(x, DppMoveI<kRowBcast15, 0xa>(x));
+  x = max(x, DppMoveI<kRowBcast31, 0xc>(x));
+  return __builtin_amdgcn_readlane(x, kWave - 1);
+}
+
 // Piece g of the batch, pieces of a multiple of kAlign slots; false beyond
-// the last one.  Every wave computes the same.  A request of at most
-// kAttnWhole steps is one piece: below that the merge costs what the shorter
-// stream saves (one request of 32 heads x 128: 300 tokens 11.0 us in three
-// pieces and 10.4 in one).
+// the last one.  Every wave computes the same.
+//
+// Whether to split at all.  A head's workgroup streams about 27 GB/s, so
+// kAttnFull of them load the chip and the longest request is the launch's tail
+// only where it has more slots than its share of the chip's time, the mean
+// times min(heads, kAttnFull) / kAttnFull.  Splitting costs a merge (7-11 us
+// of a head's stream: kAttnWhole steps, 384 slots at least).  Measured, split
+// and whole, 128 dims: 4 x 32 equal heads of 600 slots 20.5 and 18.8 us, of 1500
+// 35.6 and 39.8; 8 x 32 of 1500 72.3 and 67.1, of 375-1500 44.8 and 45.6, of
+// 1250-5000 164 and 174; 15 x 32 of 600 57.2 and 50.3; 60 x 4 of 256 dims, 600
+// slots, 57.2 and 45.4.  A request of at most kAttnWhole steps is one piece
+// (one of 32 heads: 300 tokens 11.0 us in three pieces and 10.4 in one).
+constexpr int kAttnFull = 214;
 template <int kAlign>
 __device__ __forceinline__ bool FindPiece(const AttentionArgs& a, int ps, int g, AttnPiece* out) {
+  constexpr int kGain = kAttnWhole * kAlign > 384 ? kAttnWhole * kAlign : 384;
   const int lane = threadIdx.x & (kWave - 1);
-  long long total = 0;
+  double total = 0.0;  // (exact: below 2^53)
+  int longest = 0;
   int start0 = 0, slots0 = 0;  // requests 0..63 (loaded once)
   for (int b = lane; b < a.batch; b += kWave) {
     int start;
@@ -254,13 +292,26 @@ __device__ __forceinline__ bool FindPiece(const AttentionArgs& a, int ps, int g,
       start0 = start;
       slots0 = slots;
     }
-    total += slots;
+    total += static_cast<double>(slots);
+    longest = max(longest, slots);
   }
-#pragma unroll
-  for (int o = 1; o < kWave; o <<= 1) total += __shfl_xor(total, o, kWave);
-  long long per = (total + a.piece_room - 1) / a.piece_room;
-  per = (per + kAlign - 1) / kAlign * kAlign;
-  const int P = per < kAlign ? kAlign : (per > 0x40000000 ? 0x40000000 : static_cast<int>(per));
+  total = ReadLaneD(WaveInclusiveScanD(total), kWave - 1);
+  longest = WaveMaxI(longest);
+  if (static_cast<double>(longest - kGain) <= total * static_cast<double>(a.piece_share)) {
+    if (g >= a.batch) return false;
+    out->r = g;
+    if (g < kWave) {
+      out->start = __builtin_amdgcn_readlane(start0, g);
+      out->f1 = __builtin_amdgcn_readlane(slots0, g);
+    } else {
+      out->f1 = ListSlots(a, g, ps, &out->start);
+    }
+    return true;
+  }
+  const double share = ceil(total / static_cast<double>(a.piece_room));
+  const int P = share >= 0x1p30
+                    ? 0x40000000
+                    : max(1, (static_cast<int>(share) + kAlign - 1) / kAlign) * kAlign;
   int before = 0;
   for (int b0 = 0; b0 < a.batch; b0 += kWave) {
     const int b = b0 + lane;
@@ -268,12 +319,7 @@ __device__ __forceinline__ bool FindPiece(const AttentionArgs& a, int ps, int g,
     if (b0 > 0) slots = b < a.batch ? ListSlots(a, b, ps, &start) : 0;
     int n = b < a.batch ? 1 : 0;
     if (slots > kAttnWhole * kAlign) n = (slots - 1) / P + 1;
-    int incl = n;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-      const int y = __shfl_up(incl, o, kWave);
-      if (lane >= o) incl += y;
-    }
+    const int incl = WaveInclusiveScanI(n);
     const int first = before + incl - n;
     const uint64_t mine = __ballot(g >= first && g < first + n);
     if (mine != 0) {
@@ -287,7 +333,7 @@ __device__ __forceinline__ bool FindPiece(const AttentionArgs& a, int ps, int g,
       out->f1 = out->pieces == 1 || all - out->f0 < P ? all : out->f0 + P;
       return true;
     }
-    before += __shfl(incl, kWave - 1, kWave);
+    before += __builtin_amdgcn_readlane(incl, kWave - 1);
   }
   return false;
 }
@@ -569,8 +615,12 @@ void LaunchAttention(const PoolView& pool, const AttentionArgs& args,
               static_cast<long long>(kAttnPieceWords)))) {
       throw std::invalid_argument("attention pieces do not fit their scratch");
     }
+    AttentionArgs a = args;
+    const long long heads = static_cast<long long>(args.batch) * pool.num_heads;
+    a.piece_share = static_cast<float>(std::min<long long>(heads, kAttnFull)) /
+                    (static_cast<float>(kAttnFull) * static_cast<float>(args.batch));
     const dim3 grid(pool.num_heads, args.batch + args.piece_room);
-    hipLaunchKernelGGL(shape.fn, grid, dim3(shape.waves * kWave), 0, stream, pool, args);
+    hipLaunchKernelGGL(shape.fn, grid, dim3(shape.waves * kWave), 0, stream, pool, a);
     DSD_HIP_CHECK(hipGetLastError());
     return;
   }

@@ -2880,10 +2880,16 @@ StaticScratch& StaticScratchOn(int device) {
 // The dense attention on stream s: spread over workgroups where few requests
 // would leave the chip idle, on the stream's scratch (dsd_pool::pieces).  A
 // captured launch has no place in an order of launches and stays unsplit.
-void LaunchDense(dsd_pool* pool, dsdk::AttentionArgs* a, hipStream_t s) {
+// max_slots: the longest list's token slots, 0 where only the device knows
+// (then a launch of short lists pays about 1 us for workgroups that find none).
+void LaunchDense(dsd_pool* pool, dsdk::AttentionArgs* a, long long max_slots, hipStream_t s) {
   const bool capturing = s != nullptr && StreamCapturing(s);
   if (!capturing && pool->pieces != nullptr) {
-    a->piece_room = dsdk::AttentionPieceRoom(pool->view, a->batch, 0);
+    // (the room itself must not depend on what the caller knows: one call's
+    // bits are the other's)
+    if (max_slots == 0 || dsdk::AttentionPieceRoom(pool->view, a->batch, max_slots) > 0) {
+      a->piece_room = dsdk::AttentionPieceRoom(pool->view, a->batch, 0);
+    }
   }
   if (a->piece_room == 0) {
     dsdk::LaunchAttention(pool->view, *a, s);
@@ -3016,8 +3022,10 @@ int dsd_dense_run_batch(dsd_pool* pool, int batch, const float* queries,
     Require(pool->view.head_dim > 0 && pool->view.head_dim <= 256,
             "head_dim must be in (0, 256]");
     Require(cand_offsets[0] == 0, "cand_offsets[0] must be 0");
+    long long most = 1;  // pages of the longest list
     for (int r = 0; r < batch; ++r) {
       Require(cand_offsets[r + 1] >= cand_offsets[r], "cand_offsets must be non-decreasing");
+      most = std::max<long long>(most, cand_offsets[r + 1] - cand_offsets[r]);
     }
     const int total = cand_offsets[batch];
     if (total > 0) Require(cand_ids != nullptr, "cand_ids must be non-null");
@@ -3059,7 +3067,7 @@ int dsd_dense_run_batch(dsd_pool* pool, int batch, const float* queries,
     a.scale = 1.0f / std::sqrt(static_cast<float>(pool->view.head_dim));
     a.outputs = pool->h_dense_out.ptr;
     DSD_HIP_CHECK(hipEventRecord(pool->dense_start, pool->stream));
-    LaunchDense(pool, &a, pool->stream);
+    LaunchDense(pool, &a, most * pool->view.page_size, pool->stream);
     DSD_HIP_CHECK(hipEventRecord(pool->dense_stop, pool->stream));
     pool->Sync();
     std::memcpy(outputs, pool->h_dense_out.ptr, sizeof(float) * qn);
@@ -3091,7 +3099,7 @@ int dsd_dense_run_batch_device(dsd_pool* pool, int batch,
     a.batch = batch;
     a.scale = 1.0f / std::sqrt(static_cast<float>(pool->view.head_dim));
     a.outputs = d_outputs;
-    LaunchDense(pool, &a, reinterpret_cast<hipStream_t>(stream));
+    LaunchDense(pool, &a, 0, reinterpret_cast<hipStream_t>(stream));
   });
 }
 

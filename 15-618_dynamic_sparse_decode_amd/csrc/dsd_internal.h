@@ -277,6 +277,7 @@ struct AttentionArgs {
   // polls piece_spin_limit times, for the tag with piece_wait_mask added (a
   // mask makes every wait give up), and reports to `fail`.
   int piece_room = 0;
+  float piece_share = 0.0f;  // set by the launch
   unsigned piece_tag = 0;
   unsigned piece_wait_mask = 0;
   unsigned piece_spin_limit = 1u << 20;

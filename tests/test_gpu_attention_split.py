@@ -154,6 +154,43 @@ def test_a_stream_does_not_wait_for_another_streams_step(gpu):
     pool.close()
 
 
+@pytest.mark.parametrize("H,D,lengths,whole", [
+    (8, 128, [700] * 30, True),              # 240 even heads load the chip
+    (2, 128, [300] * 70, True),              # more requests than lanes, short lists
+    (2, 64, [769] + [5] * 6, False),         # one request past three steps
+    (4, 64, [900] * 32, True),
+    (2, 128, [100] * 69 + [3000], False),    # the tail, in the second 64 requests
+])
+def test_where_heads_are_split(gpu, H, D, lengths, whole):
+    """Even batches stay unsplit (the captured step's bits); a long tail is
+    split, and either way the outputs are the oracle's."""
+    import torch
+    ps, B = 16, len(lengths)
+    batch, pool = make_pool(gpu, H, D, ps, lengths, seed=B + H)
+    want = orc.dense_batch(batch.queries, batch.key_pool, batch.value_pool, batch.token_counts,
+                           batch.cand_offsets, batch.cand_ids, H, D, ps)
+    dev = [torch.from_numpy(a).cuda() for a in (batch.queries, batch.cand_offsets,
+                                                batch.cand_ids)]
+    eager, captured = (torch.full((B, H * D), 7.0, device="cuda") for _ in range(2))
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    gpu.dense_run_batch_device(pool, B, *[t.data_ptr() for t in dev], eager.data_ptr(),
+                               side.cuda_stream)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=side):
+        gpu.dense_run_batch_device(pool, B, *[t.data_ptr() for t in dev], captured.data_ptr(),
+                                   side.cuda_stream)
+    graph.replay()
+    torch.cuda.synchronize()
+    host, _ = gpu.dense_run_batch(pool, batch.queries, batch.cand_offsets, batch.cand_ids)
+    eager = eager.cpu().numpy()
+    assert orc.max_abs_diff(eager, np.asarray(want).reshape(eager.shape)) <= 1e-4
+    assert np.array_equal(host.view(np.uint32), eager.view(np.uint32))
+    same = np.array_equal(eager.view(np.uint32), captured.cpu().numpy().view(np.uint32))
+    assert same == whole
+    pool.close()
+
+
 @pytest.mark.parametrize("bad", [np.nan, -np.inf])
 def test_nonfinite_keys_of_whole_pieces(gpu, bad):
     """Pieces (of 128 slots here) whose logits are all NaN or -inf: the output
