@@ -414,17 +414,8 @@ __global__ __launch_bounds__(WAVES * kWave) void AttentionFastKernel(
   float mx = 0.0f, lt = 0.0f, at = 0.0f;
   if (tid < D) AttnCombine<D, WAVES>(sh, tid, &mx, &lt, &at);
   if (p.pieces == 1) {
-    if (tid < D) out[tid] = lt == 0.0f ? 0.0f : at / lt;
+    if (tid < D) out[tid] = AttnOutput(mx, lt, at);
     return;
-  }
-  if (tid < D && mx == -INFINITY) {
-    // No maximum: the sums are zeros (no valid token, or logits of -inf) or
-    // NaN (NaN logits), and a NaN must reach the merge, as one wave's reaches
-    // AttnCombine when another wave has a maximum.
-    for (int w = 0; w < WAVES; ++w) {
-      lt += sh.l[w];
-      at += sh.acc[w][tid];
-    }
   }
   unsigned long long* words =
       args.piece_words +
@@ -457,7 +448,7 @@ __global__ __launch_bounds__(WAVES * kWave) void AttentionFastKernel(
     s_pl[i] = TakeWord(args, first + i * stride + 1, &s_late);
   }
   __syncthreads();
-  float m = -INFINITY;
+  float m = kNoMax;
   for (int i = 0; i < p.pieces; ++i) m = fmaxf(m, s_pm[i]);
   constexpr int kGroups = kThreads / D;  // piece i by thread group i mod kGroups
   const int d = tid % D;
@@ -467,7 +458,7 @@ __global__ __launch_bounds__(WAVES * kWave) void AttentionFastKernel(
   if (grp < kGroups) {
     for (int i = grp; i < p.pieces; i += kGroups) {
       const float a = TakeWord(args, first + i * stride + 2 + d, &s_late);
-      const float sw = s_pm[i] == -INFINITY ? 0.0f : Exp2(s_pm[i] - m);
+      const float sw = Exp2(s_pm[i] - m);
       lt = fmaf(s_pl[i], sw, lt);
       at = fmaf(a, sw, at);
     }
@@ -486,8 +477,7 @@ __global__ __launch_bounds__(WAVES * kWave) void AttentionFastKernel(
       lt += sh.l[i];
       at += sh.acc[i][tid];
     }
-    // (no piece with a maximum: zeros, as for an unsplit head)
-    float o = lt == 0.0f || m == -INFINITY ? 0.0f : at / lt;
+    float o = AttnOutput(m, lt, at);
     if (s_late != 0) {
       // Zeros and a report, as the step's other waits; NaN where the launch
       // has nowhere to report to.

@@ -29,6 +29,11 @@ constexpr int kWideAttnLpt = 16;
 constexpr int kWideAttnWaves = 16;
 constexpr int kWideAttnUnroll = 4;
 
+// A stream's maximum before its first token: the lowest float, not -inf, so
+// that a logit of -inf weighs exp2(-inf) = 0 also there (-inf - -inf would make
+// the stream NaN), with no test in the loop.
+constexpr float kNoMax = -0x1.fffffep127f;
+
 template <int WAVES, int D>
 struct AttnFastShared {
   float m[WAVES];
@@ -54,7 +59,7 @@ __device__ __forceinline__ void AttnBegin(const float* __restrict__ query_row, f
     st.q[i] *= qscale;
     st.acc[i] = 0.0f;
   }
-  st.m = -INFINITY;
+  st.m = kNoMax;
   st.l = 0.0f;
 }
 
@@ -101,9 +106,7 @@ __device__ __forceinline__ void AttnRange(const PoolView& pool, int head_off, in
       }
 #pragma unroll
       for (int o = 1; o < LPT; o <<= 1) dot += __shfl_xor(dot, o, kWave);
-      // (a logit of -inf ahead of the stream's first maximum weighs nothing:
-      // -inf - -inf would make it NaN, and a piece may well begin with one)
-      if (valid[u] && !(dot == -INFINITY && st.m == -INFINITY)) {
+      if (valid[u]) {
         const float m_new = fmaxf(st.m, dot);
         const float alpha = Exp2(st.m - m_new);
         const float beta = Exp2(dot - m_new);
@@ -129,7 +132,7 @@ __device__ __forceinline__ void AttnMergeWave(int tid, AttnState<D / LPT>& st,
   float wm = st.m;
 #pragma unroll
   for (int o = LPT; o < kWave; o <<= 1) wm = fmaxf(wm, __shfl_xor(wm, o, kWave));
-  const float sc = (st.m == -INFINITY) ? 0.0f : Exp2(st.m - wm);
+  const float sc = Exp2(st.m - wm);
   float wl = st.l * sc;
 #pragma unroll
   for (int i = 0; i < DQ; ++i) st.acc[i] *= sc;
@@ -150,26 +153,30 @@ __device__ __forceinline__ void AttnMergeWave(int tid, AttnState<D / LPT>& st,
   __syncthreads();
 }
 
-// The waves' states in LDS merged: *mx their largest maximum (-inf: no valid
-// token), *lt and *at (dim d) their sums relative to it.
+// The waves' states in LDS merged: *mx their largest maximum, *lt and *at (dim
+// d) their sums relative to it.
 template <int D, int WAVES>
 __device__ __forceinline__ void AttnCombine(const AttnFastShared<WAVES, D>& sh, int d, float* mx,
                                             float* lt, float* at) {
-  float m = -INFINITY;
+  float m = kNoMax;
 #pragma unroll
   for (int w = 0; w < WAVES; ++w) m = fmaxf(m, sh.m[w]);
   float l = 0.0f, a = 0.0f;
-  if (m != -INFINITY) {
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
-      const float sw = (sh.m[w] == -INFINITY) ? 0.0f : Exp2(sh.m[w] - m);
-      l = fmaf(sh.l[w], sw, l);
-      a = fmaf(sh.acc[w][d], sw, a);
-    }
+  for (int w = 0; w < WAVES; ++w) {
+    const float sw = Exp2(sh.m[w] - m);
+    l = fmaf(sh.l[w], sw, l);
+    a = fmaf(sh.acc[w][d], sw, a);
   }
   *mx = m;
   *lt = l;
   *at = a;
+}
+
+// The output of a head's merged sums: zero where no token weighs anything (none
+// is valid, or every logit is NaN or -inf).
+__device__ __forceinline__ float AttnOutput(float m, float l, float a) {
+  return l == 0.0f || (m == kNoMax && !(l > 0.0f)) ? 0.0f : a / l;
 }
 
 // Head h of request r over the `count` pages of `list` (global or LDS), by
@@ -195,7 +202,7 @@ __device__ __forceinline__ void AttentionFastHead(const PoolView& pool, const At
   for (int d = tid; d < D; d += WAVES * kWave) {
     float mx, lt, at;
     AttnCombine<D, WAVES>(sh, d, &mx, &lt, &at);
-    out[d] = lt == 0.0f ? 0.0f : at / lt;
+    out[d] = AttnOutput(mx, lt, at);
   }
 }
 
