@@ -267,17 +267,15 @@ __device__ __forceinline__ int WaveMaxI(int x) {
 // Piece g of the batch, pieces of a multiple of kAlign slots; false beyond
 // the last one.  Every wave computes the same.
 //
-// Whether to split at all.  A head's workgroup streams about 27 GB/s, so
-// kAttnFull of them load the chip and the longest request is the launch's tail
-// only where it has more slots than its share of the chip's time, the mean
-// times min(heads, kAttnFull) / kAttnFull.  Splitting costs a merge (7-11 us
-// of a head's stream: kAttnWhole steps, 384 slots at least).  Measured, split
-// and whole, 128 dims: 4 x 32 equal heads of 600 slots 20.5 and 18.8 us, of 1500
+// Whether to split at all.  The longest request is the launch's tail only where
+// it has more slots than its share of the chip's time, the mean times
+// piece_share * batch (PieceShare), and splitting costs a merge (7-11 us of a
+// head's stream: kAttnWhole steps, 384 slots at least).  Measured, split and
+// whole, 128 dims: 4 x 32 equal heads of 600 slots 20.5 and 18.8 us, of 1500
 // 35.6 and 39.8; 8 x 32 of 1500 72.3 and 67.1, of 375-1500 44.8 and 45.6, of
 // 1250-5000 164 and 174; 15 x 32 of 600 57.2 and 50.3; 60 x 4 of 256 dims, 600
 // slots, 57.2 and 45.4.  A request of at most kAttnWhole steps is one piece
 // (one of 32 heads: 300 tokens 11.0 us in three pieces and 10.4 in one).
-constexpr int kAttnFull = 214;
 template <int kAlign>
 __device__ __forceinline__ bool FindPiece(const AttentionArgs& a, int ps, int g, AttnPiece* out) {
   constexpr int kGain = kAttnWhole * kAlign > 384 ? kAttnWhole * kAlign : 384;
@@ -488,6 +486,18 @@ __global__ __launch_bounds__(WAVES * kWave) void AttentionFastKernel(
   }
 }
 
+// The share of the chip's time that a launch of `heads` equal unsplit heads
+// leaves to each head's slots.  About 214 workgroups load the chip; up to 256 run
+// one on a CU.  Just beyond, the CUs that got a second one are a tail of their
+// own, which thins out as more do: 288 heads of 128 dims and 3000 slots take
+// 150 us split and 183 whole, 352 183 and 193, 384 204 and 202, 448 229 and 225
+// (64 dims: 92 and 116, 114 and 122, 125 and 126, 135 and 134).
+float PieceShare(long long heads) {
+  if (heads <= 214) return static_cast<float>(heads) / 214.0f;
+  if (heads <= 256 || heads >= 448) return 1.0f;
+  return 0.5f + 0.5f * static_cast<float>(heads - 256) / 192.0f;
+}
+
 using AttnKernelFn = void (*)(PoolView, AttentionArgs);
 
 struct AttnVariant {
@@ -607,8 +617,7 @@ void LaunchAttention(const PoolView& pool, const AttentionArgs& args,
     }
     AttentionArgs a = args;
     const long long heads = static_cast<long long>(args.batch) * pool.num_heads;
-    a.piece_share = static_cast<float>(std::min<long long>(heads, kAttnFull)) /
-                    (static_cast<float>(kAttnFull) * static_cast<float>(args.batch));
+    a.piece_share = PieceShare(heads) / static_cast<float>(args.batch);
     const dim3 grid(pool.num_heads, args.batch + args.piece_room);
     hipLaunchKernelGGL(shape.fn, grid, dim3(shape.waves * kWave), 0, stream, pool, a);
     DSD_HIP_CHECK(hipGetLastError());

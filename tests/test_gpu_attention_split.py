@@ -156,6 +156,7 @@ def test_a_stream_does_not_wait_for_another_streams_step(gpu):
 
 @pytest.mark.parametrize("H,D,lengths,whole", [
     (8, 128, [700] * 30, True),              # 240 even heads load the chip
+    (8, 128, [1100] * 35, False),            # 280: a few CUs would run two
     (2, 128, [300] * 70, True),              # more requests than lanes, short lists
     (2, 64, [769] + [5] * 6, False),         # one request past three steps
     (4, 64, [900] * 32, True),
