@@ -554,13 +554,23 @@ AttnShape ShapeOf() {
   return AttnShape{WAVES, WAVES * (kWave / LPT) * UNROLL, AttentionFastKernel<D, LPT, WAVES, UNROLL>};
 }
 
-AttnShape FastShape(int head_dim, bool wide) {
+// heads: workgroups of the unsplit launch; max_slots: the lists' longest, 0:
+// unknown (dense steps).  Short lists, and lists of up to 1024 slots where heads
+// fill the chip, take 64 dims with one chunk in flight: half the registers, so
+// more workgroups share a CU, and a short list spreads over more waves (16
+// heads of 64 slots 4.6 and 5.2 us, 32 x 16 heads of 128 slots 8.8 and 9.0, of
+// 512 24.2 and 25.6); four in flight stream longer lists faster (24 x 12 heads
+// of 3000 slots: 109 and 93 us).  80 dims: four waves for short lists, which
+// wait for eight waves' merge (16 heads of 64 slots 4.5 and 5.1 us), eight for
+// longer ones (16 heads of 1500 slots: 15.6 and 11.8).
+AttnShape FastShape(int head_dim, bool wide, long long heads, long long max_slots) {
   if (head_dim == 128 && wide) {
     return ShapeOf<128, kWideAttnLpt, kWideAttnWaves, kWideAttnUnroll>();
   }
+  const bool is_short = max_slots > 0 && max_slots <= (heads >= kAttnRound ? 1024 : 128);
   switch (head_dim) {
-    case 64: return ShapeOf<64, 8, 8, 4>();
-    case 80: return ShapeOf<80, 4, 8, 1>();
+    case 64: return is_short ? ShapeOf<64, 8, 8, 1>() : ShapeOf<64, 8, 8, 4>();
+    case 80: return is_short ? ShapeOf<80, 4, 4, 1>() : ShapeOf<80, 4, 8, 1>();
     case 96: return ShapeOf<96, 8, 8, 2>();
     case 128: {
       const AttnVariant& v = SelectAttnVariant();
@@ -574,8 +584,8 @@ AttnShape FastShape(int head_dim, bool wide) {
 }  // namespace
 
 int AttentionPieceRoom(const PoolView& pool, int batch, long long max_slots) {
-  const AttnShape shape = FastShape(pool.head_dim, false);
   const long long heads = pool.num_heads;
+  const AttnShape shape = FastShape(pool.head_dim, false, batch * heads, max_slots);
   if (shape.fn == nullptr || batch <= 0) return 0;
   if (max_slots > 0 && max_slots <= kAttnWhole * shape.align) return 0;  // one piece each
   if (batch * heads >= kAttnRound) return 0;
@@ -605,7 +615,9 @@ void LaunchAttention(const PoolView& pool, const AttentionArgs& args,
   if (D <= 0 || D > 256) {
     throw std::invalid_argument("head_dim must be in (0, 256]");
   }
-  const AttnShape shape = FastShape(D, args.wide_partition && pool.elements == kFE);
+  const long long heads = static_cast<long long>(args.batch) * pool.num_heads;
+  const AttnShape shape =
+      FastShape(D, args.wide_partition && pool.elements == kFE, heads, args.max_slots);
   if (shape.fn != nullptr) {
     if (args.piece_room < 0 || args.piece_room > kAttnMaxPieces ||
         (args.piece_room > 0 &&
@@ -616,7 +628,6 @@ void LaunchAttention(const PoolView& pool, const AttentionArgs& args,
       throw std::invalid_argument("attention pieces do not fit their scratch");
     }
     AttentionArgs a = args;
-    const long long heads = static_cast<long long>(args.batch) * pool.num_heads;
     a.piece_share = PieceShare(heads) / static_cast<float>(args.batch);
     const dim3 grid(pool.num_heads, args.batch + args.piece_room);
     hipLaunchKernelGGL(shape.fn, grid, dim3(shape.waves * kWave), 0, stream, pool, a);
@@ -634,9 +645,11 @@ void LaunchAttention(const PoolView& pool, const AttentionArgs& args,
 }
 
 void PreloadAttentionKernels(const PoolView& pool) {
-  const AttnShape shape = FastShape(pool.head_dim, false);
-  if (shape.fn != nullptr) PreloadKernel(shape.fn);
-  if (pool.head_dim == 128 && pool.elements == kFE) PreloadKernel(FastShape(128, true).fn);
+  for (long long max_slots : {0, 1}) {
+    const AttnShape shape = FastShape(pool.head_dim, false, 1, max_slots);
+    if (shape.fn != nullptr) PreloadKernel(shape.fn);
+  }
+  if (pool.head_dim == 128 && pool.elements == kFE) PreloadKernel(FastShape(128, true, 1, 0).fn);
 }
 
 }  // namespace dsdk

@@ -1512,6 +1512,7 @@ void EnqueueAttentionStage(const PoolView& v, const StepLaunch& L, hipStream_t s
   a.scale = L.scale;
   a.outputs = L.outputs;
   a.wide_partition = L.wide_shape;
+  a.max_slots = static_cast<long long>(a.list_stride) * v.page_size;
   a.piece_room = L.piece_room;
   a.piece_words = L.piece_words;
   a.piece_arrivals = L.piece_arrivals;

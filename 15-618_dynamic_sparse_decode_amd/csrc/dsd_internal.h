@@ -268,6 +268,8 @@ struct AttentionArgs {
   // D = 128, E = 4096: split each head as the wide step's attention items
   // do (bit-identical outputs), for the batches that step takes.
   bool wide_partition = false;
+  // The lists' longest in token slots, 0: unknown (the kernel's variant).
+  long long max_slots = 0;
   // Spread each head's tokens over several workgroups (attention.hip):
   // AttentionPieceRoom() > 0 and the scratch for it, kAttnPieceWords words
   // and kAttnPieceCounters counters, all zero before the first

@@ -329,3 +329,26 @@ def test_a_merge_that_gives_up_is_reported_and_recovers(gpu):
             assert np.array_equal(step(queries).view(np.uint32), want.view(np.uint32))
         ctx.device_status()
     pool.close()
+
+
+@pytest.mark.parametrize("H,D,batch,k", [
+    (2, 64, 2, 8), (2, 64, 2, 9),         # 128 and 144 slots: one chunk in flight, four
+    (8, 64, 64, 16), (8, 64, 64, 65),     # 512 heads: 256 and 1040 slots
+    (2, 80, 2, 8), (2, 80, 2, 9),         # four waves, eight
+])
+def test_sparse_lists_by_length(gpu, H, D, batch, k):
+    """Either side of the list lengths that choose the kernel's form."""
+    ps = 16
+    lengths = [k * ps + 37] + [ps * (k // 2) + r for r in range(batch - 1)]
+    batch_, pool = make_pool(gpu, H, D, ps, lengths, seed=D + k)
+    summ = orc.pool_summaries(batch_.key_pool, batch_.token_counts, H * D)
+    with gpu.SparseContext(pool, k, batch, batch_.total_candidates, batch * k) as ctx:
+        got = ctx.run_batch(batch_.queries, batch_.cand_offsets, batch_.cand_ids,
+                            output_mode=gpu.OUTPUT_OUTPUTS, want_ids=True)
+    _, selected, outs = orc.sparse_batch(batch_.queries, batch_.key_pool, batch_.value_pool, summ,
+                                         batch_.token_counts, batch_.cand_offsets,
+                                         batch_.cand_ids, H, D, ps, k)
+    for r in range(batch):
+        assert got["selected"][r].tolist() == selected[r].tolist(), r
+    assert orc.max_abs_diff(got["outputs"], outs) <= 1e-4
+    pool.close()
