@@ -32,8 +32,9 @@ namespace {
 // (1207 pages): 25 us; 108 us with the kernel below, whose 32 waves were all
 // there was and read 64 rows a line at a time.
 //
-// ScoreExactKernel (other E): a wave of 64 candidates, each lane walking its
-// own row in memory.
+// ScoreExactKernel (other E, and batches of more pages than the chains kernel
+// takes in one round): a wave of 64 candidates, each lane walking its own row in
+// memory.
 // ---------------------------------------------------------------------------
 constexpr int kChainPages = 32;
 constexpr int kChainThreads = 512;
@@ -72,9 +73,8 @@ __global__ __launch_bounds__(kWave) void ScoreExactKernel(
     const float* __restrict__ queries, const float* __restrict__ summaries,
     const int* __restrict__ token_counts, int capacity, const int* __restrict__ cand_offsets,
     const int* __restrict__ cand_ids, int total, int E, float scale,
-    float* __restrict__ scores, const int* __restrict__ only, FailReport fail) {
+    float* __restrict__ scores, FailReport fail) {
   const int r = blockIdx.y;
-  if (only != nullptr && only[r] >= 0) return;  // decided without exact scores
   int begin, n;
   if (!RequestRange(cand_offsets, r, total, fail, &begin, &n)) return;
   const int end = begin + n;
@@ -1292,9 +1292,18 @@ void LaunchScoreExact(const PoolView& pool, const float* d_queries,
                       float* d_scores, FailReport fail, hipStream_t stream,
                       const int* d_undecided) {
   if (batch <= 0 || max_candidates <= 0) return;
-  if (pool.elements % kWave == 0) {
-    // The fewest pages per workgroup that keep the batch within a round of
-    // workgroups (two per CU).
+  // The chains kernel up to a round of its workgroups (two per CU); beyond it
+  // runs several, and a lane per page then fills the chip as well (E = 1024:
+  // 16000 pages 20.8 us and 25.0 with lanes, 30000 38.2 and 28.8, 60000 92 and
+  // 50; E = 512: 12.3 and 14.1, 22.0 and 16.8, 39.9 and 23.3).  Requests left
+  // undecided are few of the batch: always chains.
+  const bool chains = pool.elements % kWave == 0 &&
+                      (d_undecided != nullptr || total_candidates <= 512 * kChainPages);
+  if (!chains && d_undecided != nullptr) {
+    throw std::invalid_argument("undecided requests need E % 64 == 0");
+  }
+  if (chains) {
+    // The fewest pages per workgroup that keep the batch within that round.
     int pages = kChainPages / 4;
     while (pages < kChainPages && total_candidates > 512 * pages) pages *= 2;
     hipLaunchKernelGGL(ScoreChainsKernel, dim3((max_candidates + pages - 1) / pages, batch),
@@ -1309,12 +1318,12 @@ void LaunchScoreExact(const PoolView& pool, const float* d_queries,
     hipLaunchKernelGGL(ScoreExactKernel<true>, grid, dim3(kWave), 0, stream,
                        d_queries, pool.summaries, pool.token_counts, pool.capacity,
                        d_cand_offsets, d_cand_ids, total_candidates, pool.elements, scale,
-                       d_scores, d_undecided, fail);
+                       d_scores, fail);
   } else {
     hipLaunchKernelGGL(ScoreExactKernel<false>, grid, dim3(kWave), 0, stream,
                        d_queries, pool.summaries, pool.token_counts, pool.capacity,
                        d_cand_offsets, d_cand_ids, total_candidates, pool.elements, scale,
-                       d_scores, d_undecided, fail);
+                       d_scores, fail);
   }
   DSD_HIP_CHECK(hipGetLastError());
 }

@@ -147,3 +147,27 @@ def test_a_chain_that_overflows(gpu, n):
     assert want[0].tolist() == [11]
     assert got["selected"][0].tolist() == [11]
     assert orc.max_abs_diff(got["outputs"], outs) <= 1e-4
+
+
+@pytest.mark.parametrize("n", [[8192, 8192], [8192, 8191, 2], [8192, 1, 8191, 8192, 5]])
+def test_exact_scores_of_many_pages(gpu, n):
+    """Either side of the 16384 pages up to which exact scores come from the
+    chains kernel."""
+    H, D, k = 1, 64, 3
+    E, cap = H * D, 8192
+    rng = np.random.default_rng(len(n))
+    keys, values = (rng.standard_normal((cap, E)).astype(np.float32) for _ in range(2))
+    queries = rng.standard_normal((len(n), E)).astype(np.float32)
+    offsets = np.concatenate([[0], np.cumsum(n)]).astype(np.int32)
+    ids = np.concatenate([rng.permutation(cap)[:c] for c in n]).astype(np.int32)
+    ones, all_ids = np.ones(cap, np.int32), np.arange(cap, dtype=np.int32)
+    with gpu.DevicePagePool(H, D, 1, cap) as pool:
+        pool.upload_pages(all_ids, ones, all_ids.astype(np.int64) * E, keys, values)
+        with gpu.SparseContext(pool, k, len(n), len(ids), len(n) * k) as ctx:
+            got = ctx.run_batch(queries, offsets, ids)
+    scores, selected, _ = orc.sparse_batch(queries, keys.reshape(cap, 1, E),
+                                           values.reshape(cap, 1, E), keys, ones, offsets, ids,
+                                           H, D, 1, k)
+    assert np.array_equal(got["scores"].view(np.uint32), scores.view(np.uint32))
+    for r in range(len(n)):
+        assert got["selected"][r].tolist() == selected[r].tolist(), r
