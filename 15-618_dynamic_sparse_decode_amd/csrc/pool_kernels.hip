@@ -189,12 +189,14 @@ __device__ __forceinline__ float DecodeValue(int request_id, int decode_step, in
   return HashValue(x);
 }
 
-// Workgroup (i, y): page i of the prompt, kPoolThreads * kVec elements of its
-// rows: K/V from the hash, summary by the host rule.  A prompt of a few
-// thousand tokens is a few hundred pages, so one workgroup per page left most
-// of the chip idle (128 pages of 16 x 4096: 50 us; this grid
-// 15-22; 8192 pages, 4.3 GB, 870 us, bound by the hash).
-template <int kVec>
+// Workgroup (i, y): page i of the prompt, kPoolThreads elements of its rows: K/V
+// from the hash, summary by the host rule.  A prompt of a few thousand tokens is
+// a few hundred pages, so one workgroup per page left most of the chip idle (128
+// pages of 16 x 4096: 50 us; this grid 15-22; 8192 pages, 4.3 GB, 870 us, bound
+// by the hash).  One element a thread: the hash takes the time, not the stores,
+// and four make its chain four times as long (8 pages of 16 x 4096 26.0 us and
+// now 22.7, of 16 x 512 25.6 and 22.0; 4096 pages of 16 x 64 55 and 33, of 16 x
+// 4096 455 and 463).
 __global__ __launch_bounds__(kPoolThreads) void PrefillSyntheticKernel(
     PoolView pool, const int* __restrict__ page_ids, const int* __restrict__ token_counts,
     int n, int request_id) {
@@ -203,7 +205,7 @@ __global__ __launch_bounds__(kPoolThreads) void PrefillSyntheticKernel(
   const int page = page_ids[i];
   const int count = token_counts[i];
   const int E = pool.elements;
-  const int e = (static_cast<int>(blockIdx.y) * kPoolThreads + static_cast<int>(threadIdx.x)) * kVec;
+  const int e = static_cast<int>(blockIdx.y) * kPoolThreads + static_cast<int>(threadIdx.x);
   if (blockIdx.y == 0 && threadIdx.x == 0) {
     pool.token_counts[page] = count;
     pool.live[page] = 1;
@@ -211,23 +213,16 @@ __global__ __launch_bounds__(kPoolThreads) void PrefillSyntheticKernel(
   if (e >= E) return;
   const float inv = __fdiv_rn(1.0f, static_cast<float>(count));
   size_t at = static_cast<size_t>(page) * pool.page_elems + e;
-  float acc[kVec] = {};
+  float acc = 0.0f;
   for (int t = 0; t < count; ++t) {
     const uint32_t row = PromptRow(request_id, i, t);
-    float k[kVec], v[kVec];
-#pragma unroll
-    for (int x = 0; x < kVec; ++x) {
-      k[x] = PromptValue(row, e + x, 1);
-      v[x] = PromptValue(row, e + x, 2);
-      acc[x] = __fadd_rn(acc[x], k[x]);
-    }
-    StoreVec<kVec>(pool.keys + at, k);
-    StoreVec<kVec>(pool.values + at, v);
+    const float k = PromptValue(row, e, 1);
+    pool.keys[at] = k;
+    pool.values[at] = PromptValue(row, e, 2);
+    acc = __fadd_rn(acc, k);
     at += E;
   }
-#pragma unroll
-  for (int x = 0; x < kVec; ++x) acc[x] = __fmul_rn(acc[x], inv);
-  StoreVec<kVec>(pool.summaries + static_cast<size_t>(page) * E + e, acc);
+  pool.summaries[static_cast<size_t>(page) * E + e] = __fmul_rn(acc, inv);
 }
 
 // One workgroup per (page segment, kPoolThreads elements of the token row),
@@ -320,10 +315,9 @@ void LaunchPrefillSynthetic(const PoolView& pool, const int* d_page_ids,
                             const int* d_token_counts, int n, int request_id,
                             hipStream_t stream) {
   if (n <= 0) return;
-  const bool vec = pool.elements % 4 == 0;
-  const auto kernel = vec ? PrefillSyntheticKernel<4> : PrefillSyntheticKernel<1>;
-  hipLaunchKernelGGL(kernel, dim3(n, RowSlices(pool.elements, vec ? 4 : 1)), dim3(kPoolThreads), 0,
-                     stream, pool, d_page_ids, d_token_counts, n, request_id);
+  hipLaunchKernelGGL(PrefillSyntheticKernel, dim3(n, RowSlices(pool.elements, 1)),
+                     dim3(kPoolThreads), 0, stream, pool, d_page_ids, d_token_counts, n,
+                     request_id);
   DSD_HIP_CHECK(hipGetLastError());
 }
 
