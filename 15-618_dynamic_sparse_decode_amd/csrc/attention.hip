@@ -551,7 +551,8 @@ struct AttnShape {
 
 template <int D, int LPT, int WAVES, int UNROLL>
 AttnShape ShapeOf() {
-  return AttnShape{WAVES, WAVES * (kWave / LPT) * UNROLL, AttentionFastKernel<D, LPT, WAVES, UNROLL>};
+  return AttnShape{WAVES, WAVES * (kWave / LPT) * UNROLL,
+                   AttentionFastKernel<D, LPT, WAVES, UNROLL>};
 }
 
 // heads: workgroups of the unsplit launch; max_slots: the lists' longest, 0:

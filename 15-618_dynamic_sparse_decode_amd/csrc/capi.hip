@@ -1777,7 +1777,7 @@ struct dsd_sparse_ctx {
     L.certified = StepCertified(v, score_mode, max_n, top_k, need_exact_scores);
     L.fused = StepFused(v, L.certified, fused_enabled, max_n, top_k) ||
               (L.certified && fused_enabled && wide_enabled &&
-               dsdk::FusedStepLong(v, batch, max_n, top_k));
+               dsdk::FusedStepLong(v, batch, total, max_n, top_k));
     // The wide step takes the batches the single launch cannot (a request
     // beyond 256 candidates); DSD_FUSED_STEP=0 alone keeps three kernels.
     L.wide_shape = !L.fused && L.certified && batch > 0 &&
@@ -2961,7 +2961,8 @@ int dsd_sparse_run_batch_device_static(dsd_pool* pool, int top_k, int batch,
     L.certified = StepCertified(v, DSD_SCORE_CERTIFIED, max_candidates, top_k,
                                 StepWantsExactScores(d_scores, max_candidates));
     L.fused = StepFused(v, L.certified, true, max_candidates, top_k) ||
-              (L.certified && dsdk::FusedStepLong(v, batch, max_candidates, top_k));
+              (L.certified &&
+               dsdk::FusedStepLong(v, batch, total_candidates, max_candidates, top_k));
     // (three kernels where a context would run the wide step, with its
     // attention partition: the same outputs)
     L.wide_shape = !L.fused && L.certified && batch > 0 &&

@@ -348,7 +348,7 @@ constexpr int kFRefineSlots = 8;
 bool FusedStepSupported(const PoolView& pool, int max_candidates, int top_k);
 // The same at 257 to 512 candidates: top_k <= 64, batches large enough that it
 // beats the wide step.
-bool FusedStepLong(const PoolView& pool, int batch, int max_candidates, int top_k);
+bool FusedStepLong(const PoolView& pool, int batch, int total, int max_candidates, int top_k);
 // Heads per workgroup for a batch: the fewest (1, 2, 4, 8) that keep the grid
 // within `compute_units` workgroups, else 8.
 int FusedStepHeadsPerGroup(const PoolView& pool, int batch, int compute_units);

@@ -68,11 +68,19 @@ constexpr int kFMaxK = 256;
 // against 29.6; 64 of 269-500 pages, top 16: 176 against 201.  With more tokens
 // the wide step's evenly shared heads win (16 requests of 269-500 pages, top
 // 32: 88.5 us against 92; top 64: 141 against 150), and with few requests its
-// score slices (3 of 500 pages, top 16: 32 us against 34.5).
+// score slices (3 of 500 pages, top 16: 32 us against 34.5).  Fewer than
+// kFLongEven requests that attend more than kFLongFew tokens are taken only if
+// they hold at most 340 pages on average, 256 from 9 requests on, where a
+// workgroup has two heads (means of four inputs, top 16: 6 of 420 pages 43.5 us
+// and 39.8 wide, 6 of 260 30.7 and 32.9; 10 of 420 52.5 and 43.9, of 260 43.8
+// and 41.5; 10 of 64-340 36.4 and 41.4; 16 of 420 62.0 and 59.8, of 512 63.7 and
+// 66.0; top 8 wins at every size: 6 of 512 33.6 and 37.6).
 constexpr int kFLongCand = 512;
 constexpr int kFLongK = 64;
 constexpr int kFLongBatch = 6;
 constexpr int kFLongTokens = 256;
+constexpr int kFLongFew = 128;
+constexpr int kFLongEven = 16;
 constexpr int kFLpt = 16;                 // lanes per token row (8 dims each)
 constexpr int kFDq = kFD / kFLpt;         // 8
 constexpr int kFTpc = kWave / kFLpt;      // 4 token rows per wave per chunk
@@ -1092,10 +1100,15 @@ bool FusedStepSupported(const PoolView& pool, int max_candidates, int top_k) {
          pool.num_heads % 2 == 0 && max_candidates <= kFMaxCand && top_k <= kFMaxK;
 }
 
-bool FusedStepLong(const PoolView& pool, int batch, int max_candidates, int top_k) {
-  return FusedStepSupported(pool, 0, top_k) && batch >= kFLongBatch &&
-         max_candidates > kFMaxCand && max_candidates <= kFLongCand && top_k <= kFLongK &&
-         static_cast<int64_t>(top_k) * pool.page_size <= kFLongTokens;
+bool FusedStepLong(const PoolView& pool, int batch, int total, int max_candidates, int top_k) {
+  if (!FusedStepSupported(pool, 0, top_k) || batch < kFLongBatch || max_candidates <= kFMaxCand ||
+      max_candidates > kFLongCand || top_k > kFLongK) {
+    return false;
+  }
+  const int64_t tokens = static_cast<int64_t>(top_k) * pool.page_size;
+  if (tokens > kFLongTokens) return false;
+  return tokens <= kFLongFew || batch >= kFLongEven ||
+         total <= static_cast<int64_t>(batch) * (batch <= 8 ? 340 : 256);
 }
 
 int FusedStepHeadsPerGroup(const PoolView& pool, int batch, int compute_units) {
@@ -1139,7 +1152,7 @@ void LaunchFusedStep(const PoolView& pool, const FusedArgs& args, hipStream_t st
     DSD_HIP_CHECK(hipGetLastError());
   }
   if (args.max_candidates > kFMaxCand) {
-    if (!FusedStepLong(pool, args.batch, args.max_candidates, args.top_k)) {
+    if (!FusedStepLong(pool, args.batch, args.total, args.max_candidates, args.top_k)) {
       throw std::invalid_argument("the fused step does not take this many candidates");
     }
     hipLaunchKernelGGL((FusedStepKernel<true, kFLongCand>), dim3(grid), dim3(kFThreads), 0, stream,

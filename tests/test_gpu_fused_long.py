@@ -52,6 +52,12 @@ def check(gpu, counts, ps, k, edit=None, seed=0, fused=1):
     ([300, 20, 20, 20, 20, 20], 1, 65, 0),        # too many members
     ([300, 20, 20, 20, 20, 20], 16, 17, 0),       # too many tokens
     ([300, 20, 20, 20, 20], 1, 8, 0),             # too few requests
+    ([340] * 6, 4, 33, 1),                        # more than 128 tokens: few pages on average
+    ([341] + [340] * 5, 4, 33, 0),                # one more
+    ([341] * 6, 4, 32, 1),
+    ([512] + [224] * 8, 4, 33, 1),
+    ([512] + [224] * 7 + [225], 4, 33, 0),
+    ([300] * 16, 4, 33, 1),
 ])
 def test_long_form_matches_oracle(gpu, counts, ps, k, fused):
     check(gpu, counts, ps, k, fused=fused)
