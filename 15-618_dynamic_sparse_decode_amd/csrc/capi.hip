@@ -248,7 +248,7 @@ struct dsd_pool {
   PinnedBuffer<int> h_dense_offsets, h_dense_ids;
   hipEvent_t dense_start = nullptr, dense_stop = nullptr;
   // The dense attention's pieces (attention.hip): kDenseScratches scratches of
-  // 2 MiB, behind the summaries.  The first streams to use the pool own one
+  // 2 MiB, behind the keys.  The first streams to use the pool own one
   // each: their steps follow one another by the stream's own order and no
   // stream waits for another's.  (A stream made later with the handle of a
   // destroyed one takes its scratch: what ran on a destroyed stream has ended,
@@ -429,23 +429,23 @@ int dsd_pool_create(int num_heads, int head_dim, int page_size,
       const size_t sum_bytes = static_cast<size_t>(capacity_pages) *
                                static_cast<size_t>(v.elements) * sizeof(float);
       const bool pieces = dsdk::AttentionPieceRoom(v, 1, 0) > 0;
-      const size_t sum_end = (sum_bytes + 255) / 256 * 256;
-      const size_t zero_bytes =
-          pieces ? sum_end + dsd_pool::kDenseScratches * kPieceScratchWords *
-                                 sizeof(unsigned long long)
-                 : sum_bytes;
-      DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.keys), kv_bytes));
-      DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.values), kv_bytes));
-      DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.summaries), zero_bytes));
+      // (behind the keys: an allocation of its own takes the runtime 23 us)
+      const size_t keys_end = (kv_bytes + 255) / 256 * 256;
+      const size_t piece_bytes =
+          pieces ? dsd_pool::kDenseScratches * kPieceScratchWords * sizeof(unsigned long long) : 0;
+      DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.keys), keys_end + piece_bytes));
       if (pieces) {
         pool->pieces = reinterpret_cast<unsigned long long*>(
-            reinterpret_cast<unsigned char*>(v.summaries) + sum_end);
+            reinterpret_cast<unsigned char*>(v.keys) + keys_end);
+        DSD_HIP_CHECK(hipMemsetAsync(pool->pieces, 0, piece_bytes, pool->stream));
       }
+      DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.values), kv_bytes));
+      DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.summaries), sum_bytes));
       DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.token_counts),
                               sizeof(int) * static_cast<size_t>(capacity_pages)));
       DSD_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&v.live),
                               static_cast<size_t>(capacity_pages)));
-      DSD_HIP_CHECK(hipMemsetAsync(v.summaries, 0, zero_bytes, pool->stream));
+      DSD_HIP_CHECK(hipMemsetAsync(v.summaries, 0, sum_bytes, pool->stream));
       DSD_HIP_CHECK(hipMemsetAsync(v.token_counts, 0,
                                    sizeof(int) * static_cast<size_t>(capacity_pages),
                                    pool->stream));
