@@ -462,6 +462,7 @@ int dsd_pool_create(int num_heads, int head_dim, int page_size,
       DSD_HIP_CHECK(hipMemcpy(pool->v_offsets, offsets.data(), off_bytes, hipMemcpyHostToDevice));
       pool->Sync();
     }
+    dsdk::PreloadAttentionKernels(v);
     *out_pool = pool.release();
   });
 }

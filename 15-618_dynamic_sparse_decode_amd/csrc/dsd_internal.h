@@ -46,7 +46,7 @@ void PreloadKernel(K kernel) {
   hipFuncAttributes attr{};
   DSD_HIP_CHECK(hipFuncGetAttributes(&attr, reinterpret_cast<const void*>(kernel)));
 }
-// The hot kernels of each translation unit (sparse contexts and tables
+// The hot kernels of each translation unit (pools, sparse contexts and tables
 // call these at creation).
 void PreloadStepKernels();
 void PreloadFusedKernels();

@@ -1506,8 +1506,13 @@ void PreloadStepKernels() {
   PreloadKernel(WideStepKernel);
   PreloadKernel(WideBumpKernel);
   PreloadKernel(SelectCertifiedKernel<kCertMaxKeys / kSelThreads, CertShared>);
+  PreloadKernel(SelectCertifiedKernel<kLargeMaxKeys / 2 / kSelThreads, CertSharedLarge>);
+  PreloadKernel(SelectCertifiedKernel<kLargeMaxKeys / kSelThreads, CertSharedLarge>);
   PreloadKernel(SelectCertifiedRankKernel);
+  PreloadKernel(SelectTopKKernel);
   PreloadKernel(ScoreBoundGenericKernel<true, kBoundRows>);
+  PreloadKernel(ScoreBoundGenericKernel<false, 1>);
+  PreloadKernel(ScoreChainsKernel);
 }
 
 }  // namespace dsdk
