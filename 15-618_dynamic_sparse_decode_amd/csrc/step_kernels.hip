@@ -462,11 +462,20 @@ struct CertSharedT {
 using CertShared = CertSharedT<kCertMaxKeys, kCertMaxKeys>;
 using CertSharedLarge = CertSharedT<kLargeMaxK + kLargeMaxOpen, kLargeMaxOpen>;
 
-// Threads per element of a loop over `count` elements (a power of two, <= 16).
+// Threads per element of a pass over the set (a power of two, 4 to 16).  The
+// loops below compare every pair, about ten instructions each on all four SIMDs
+// (512 members: 18 us a sort, 22 a certification), so what matters is that no
+// wave runs without elements: sets beyond 256 take several passes of 256, and a
+// wave past the last element skips its loop.  (One thread an element from 513
+// on, nine waves' elements and sixteen waves' loops: 36 and 43 us.)
 __device__ __forceinline__ int SetParts(int count) {
   int parts = 16;
-  while (parts > 1 && parts * count > kSelThreads) parts >>= 1;
+  while (parts > 4 && parts * count > kSelThreads) parts >>= 1;
   return parts;
+}
+// Whether this wave has an element in the pass from element `base` on.
+__device__ __forceinline__ bool SetWaveBusy(int base, int parts, int count) {
+  return base + static_cast<int>(threadIdx.x) / kWave * kWave / parts < count;
 }
 
 // from, sorted by key (descending; equal keys by position), into to: ranks by
@@ -476,6 +485,7 @@ __device__ __forceinline__ void SortSet(const Set& from, Set& to, int count) {
   const int parts = SetParts(count);
   const int part = threadIdx.x & (parts - 1);
   for (int base = 0; base < count; base += kSelThreads / parts) {
+    if (!SetWaveBusy(base, parts, count)) break;
     const int t = base + static_cast<int>(threadIdx.x) / parts;
     const uint64_t k = t < count ? from.key[t] : 0ull;
     int rank = 0;
@@ -507,6 +517,7 @@ __device__ __forceinline__ void CertifySet(Shared& sh, const Set& set, int count
   const int parts = SetParts(count);
   const int part = threadIdx.x & (parts - 1);
   for (int base = 0; base < count; base += kSelThreads / parts) {
+    if (!SetWaveBusy(base, parts, count)) break;
     const int t = base + static_cast<int>(threadIdx.x) / parts;
     const bool in = t < count;
     const float l = in ? set.lo[t] : INFINITY;

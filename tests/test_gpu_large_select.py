@@ -36,6 +36,8 @@ def run(gpu, keys, values, queries, offsets, ids, H, D, k):
     (4, 64, [4096, 0, 300], 64),         # four candidates per thread
     (4, 64, [4097, 2048], 7),            # eight
     (3, 64, [8192, 8191], 1024),         # E = 192: no refinement; the most members
+    (4, 64, [2000, 257], 257),           # up to 2048: sets of a pass of 256 and a bit more
+    (4, 64, [2048, 600], 513),
     (4, 64, [2500], 1025),               # more members: the exact path
     (32, 128, [2600, 2100], 64),         # E = 4096: the float score passes
 ])
