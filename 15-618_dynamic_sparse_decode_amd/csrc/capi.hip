@@ -1485,7 +1485,8 @@ void EnqueueSelectStage(const PoolView& v, const StepLaunch& L, hipStream_t s) {
     dsdk::SelectAssist assist;
     assist.words = L.rec;
     // (a captured step's epoch would repeat: no helpers)
-    assist.epoch = L.epoch_src != nullptr || L.never_ready ? 0u : L.epoch;
+    assist.epoch = L.epoch_src != nullptr ? 0u : L.epoch;
+    assist.wait_mask = L.never_ready ? 0x80000000u : 0u;
     assist.spin_limit = std::min(L.spin_limit, kAssistSpins);
     assist.compute_units = L.compute_units;
     dsdk::LaunchSelectCertified(v, L.scores, L.lo, L.hi, L.queries, L.offsets, L.ids, L.batch,

@@ -225,9 +225,11 @@ void LaunchScoreBounds(const PoolView& pool, const float* d_queries,
 struct SelectAssist {
   unsigned long long* words = nullptr;
   unsigned epoch = 0;
+  unsigned wait_mask = 0;  // non-zero: every wait gives up
   unsigned spin_limit = 0;
   int compute_units = 0;
   int helpers = 0;  // per request; set by the launch
+  __host__ __device__ unsigned WaitTag() const { return epoch | wait_mask; }
 };
 void LaunchSelectCertified(const PoolView& pool, const float* d_mid, const float* d_lo,
                            const float* d_hi,

@@ -561,7 +561,7 @@ __device__ __forceinline__ void AssistSelect(Shared& sh, const SelectAssist& ass
   const int tid = threadIdx.x;
   if (tid == 0) {
     unsigned long long w = 0;
-    const bool ok = AwaitTagged(words, assist.epoch, assist.spin_limit, &w);
+    const bool ok = AwaitTagged(words, assist.WaitTag(), assist.spin_limit, &w);
     const int pages = ok ? static_cast<int>(static_cast<uint32_t>(w)) : 0;
     sh.nopen = pages <= kAssistMaxPages ? pages : 0;
     sh.all = 1;
@@ -572,7 +572,7 @@ __device__ __forceinline__ void AssistSelect(Shared& sh, const SelectAssist& ass
   if (mine == 0) return;
   if (tid < mine) {
     unsigned long long w = 0;
-    const bool ok = AwaitTagged(words + 1 + index + tid * assist.helpers, assist.epoch,
+    const bool ok = AwaitTagged(words + 1 + index + tid * assist.helpers, assist.WaitTag(),
                                 assist.spin_limit, &w);
     const int c = static_cast<int>(static_cast<uint32_t>(w));
     if (!ok || c < 0 || c >= n) {
@@ -757,7 +757,8 @@ __device__ __forceinline__ void SelectCertifiedRequest(
       // Thread 3f + x: word x of open position f's interval.
       if (tid < 3 * nopen) {
         unsigned long long w = 0;
-        if (AwaitTagged(words + 1 + kAssistMaxPages + tid, assist.epoch, assist.spin_limit, &w)) {
+        if (AwaitTagged(words + 1 + kAssistMaxPages + tid, assist.WaitTag(), assist.spin_limit,
+                        &w)) {
           float* to = tid % 3 == 0 ? sh.r_mid : (tid % 3 == 1 ? sh.r_lo : sh.r_hi);
           to[tid / 3] = __uint_as_float(static_cast<uint32_t>(w));
         } else {

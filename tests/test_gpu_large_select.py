@@ -1,6 +1,7 @@
-"""The certified select for 2049 to 8192 candidates per request
-(SelectCertifiedLargeKernel) and the exact kernels that finish the requests it
-leaves undecided: ids equal to the oracle's, scores and counts included."""
+"""The certified select for 257 to 8192 candidates per request
+(SelectCertifiedKernel), its helper workgroups, and the exact kernels that
+finish the requests it leaves undecided: ids equal to the oracle's, scores and
+counts included."""
 import numpy as np
 import pytest
 
@@ -173,3 +174,69 @@ def test_exact_scores_of_many_pages(gpu, n):
     assert np.array_equal(got["scores"].view(np.uint32), scores.view(np.uint32))
     for r in range(len(n)):
         assert got["selected"][r].tolist() == selected[r].tolist(), r
+
+
+def open_positions(mid, lo, hi, ids, k):
+    """How many candidates the first-pass intervals leave open: members whose
+    interval meets another's that can still be selected, and outsiders that meet
+    a member's."""
+    order = np.lexsort((ids, -mid))
+    members, others = order[:k], order[k:]
+    others = others[hi[others] >= lo[members].min()]
+    some = np.concatenate([members, others])
+    meets = (lo[some][:, None] <= hi[some]) & (lo[some] <= hi[some][:, None])
+    np.fill_diagonal(meets, False)
+    return int(meets[:k].any(1).sum() + meets[k:, :k].any(1).sum())
+
+
+@pytest.mark.parametrize("batch,n,near,k", [
+    (1, 300, 20, 12),   # more than the 8 that the selecting workgroup refines itself
+    (3, 1900, 40, 40),
+    (1, 2300, 12, 5),   # beyond 2048 candidates
+    (2, 8192, 50, 30),
+])
+def test_helpers_refine_the_open_pages(gpu, batch, n, near, k):
+    """near pages whose first-pass intervals overlap and whose refined ones do
+    not: the helper workgroups settle them without an exact chain.  Where every
+    wait for them gives up, the same pages take the chain and the ids stay."""
+    H, D = 8, 128
+    E = H * D
+    rng = np.random.default_rng(n)
+    scale = 1.0 / np.sqrt(np.float32(D))
+    query = np.repeat(rng.standard_normal((1, E)).astype(np.float32), batch, axis=0)
+    m = int(np.argmax(np.abs(query)))
+    base = (0.2 * query[0] + 0.25 * rng.standard_normal(E)).astype(np.float32)
+    summ = (0.25 * rng.standard_normal((n, E))).astype(np.float32)
+    for j in range(near):
+        summ[j] = base
+        summ[j, m] += np.float32(j * 1e-4 / (query[0, m] * scale))
+    keys, values = (rng.standard_normal((n, E)).astype(np.float32) for _ in range(2))
+    ones, all_ids = np.ones(n, np.int32), np.arange(n, dtype=np.int32)
+    ids = np.concatenate([rng.permutation(n) for _ in range(batch)]).astype(np.int32)
+    offsets = np.arange(0, (batch + 1) * n, n, dtype=np.int32)
+    _, want, outs = orc.sparse_batch(query, keys.reshape(n, 1, E), values.reshape(n, 1, E), summ,
+                                     ones, offsets, ids, H, D, 1, k)
+    with gpu.DevicePagePool(H, D, 1, n) as pool:
+        pool.upload_pages(all_ids, ones, all_ids.astype(np.int64) * E, keys, values, summ)
+        with gpu.SparseContext(pool, k, batch, batch * n, batch * k) as ctx:
+            def step():
+                got = ctx.run_batch(query, offsets, ids, output_mode=gpu.OUTPUT_OUTPUTS,
+                                    want_ids=True)
+                for r in range(batch):
+                    assert got["selected"][r].tolist() == want[r].tolist(), r
+                assert orc.max_abs_diff(got["outputs"], outs) <= 1e-4
+                return ctx.exact_rescored_pages(reset=True)
+
+            chained = step()
+            info = ctx.last_launch()
+            assert info["certified"] == 1 and info["fused"] == 0 and info["wide"] == 0
+            bounds = [np.split(a, batch) for a in (*ctx.score_bounds(batch * n), ids)]
+            opened = [open_positions(*request, k) for request in zip(*bounds)]
+            print(f"[helpers] n={n} open={opened} chained={chained}", flush=True)
+            assert all(8 < o <= 64 for o in opened) and chained == 0
+            ctx.set_wait_limit(1 << 17, True)
+            assert step() == sum(opened)
+            ctx.set_wait_limit(1)
+            assert step() <= sum(opened)   # (a helper may be that quick)
+            ctx.set_wait_limit(1 << 17)
+            assert step() == 0
