@@ -217,11 +217,11 @@ void LaunchScoreBounds(const PoolView& pool, const float* d_queries,
 // candidate list is longer than max_candidates (the score kernels covered
 // only that many) or whose offsets leave [0, total_candidates] selects
 // nothing and is reported (kFailShape).
-// assist: for more than 2048 candidates per request, helper workgroups that
+// assist: for more than 256 candidates per request, helper workgroups that
 // refine a request's flagged pages.  words: the publication words of the
 // candidates (3 each, FusedArgs::rec), epoch a tag no earlier launch on them
-// used (0: no helpers), spin_limit polls until a wait gives up (its request
-// then goes to the exact chains).
+// used (0: no helpers), spin_limit polls until a wait gives up (the request's
+// open pages then take the exact chains).
 struct SelectAssist {
   unsigned long long* words = nullptr;
   unsigned epoch = 0;

@@ -137,7 +137,7 @@ __global__ __launch_bounds__(kWave) void ScoreExactKernel(
 // per lane, so every load reads 1 KiB contiguously (a block of E/64
 // consecutive products per lane, read one at a time, took 94 us for the 40 MB
 // of 32 requests of 8 x 128 heads, about 300 pages each; this form
-// 17 us).  Prefix sums: within the float4, then a wave scan of the lanes'
+// 15 us).  Prefix sums: within the float4, then a wave scan of the lanes'
 // sums, then the rows' totals one after the other; on any product's path at
 // most 3 + 6 + E/256 + 2 double additions, far below the n roundings that
 // WriteBounds allows for.  A wave takes `per_wave` pages of its request: their
@@ -363,8 +363,8 @@ __global__ __launch_bounds__(256) void SelectTopKKernel(
 // 4 requests of up to 8192 pages) and a bitonic sort of them (165 us): that
 // step took 363 us and takes 137.  Up to 2048 candidates it replaces a select
 // that kept every candidate in LDS and gave each member one thread (32 requests
-// of 8 x 128 heads, 300 pages each: the step 50 us, now 45.5; the wide step of
-// one request of 2048 pages, 64 selected: 71 us, now 59).
+// of 8 x 128 heads, 300 pages each: the step 50 us, 45.5 with this select alone
+// changed; the wide step of one request of 2048 pages, 64 selected: 71 us, 59).
 //
 // Beyond 2048 candidates LDS holds kLargeMaxK members and kLargeMaxOpen open
 // candidates: a request with more open (equal pages, a zero query) is left
@@ -653,7 +653,7 @@ __device__ __forceinline__ void SelectCertifiedRequest(
       return;
     }
   }
-  // 1. The kk-th largest key, 8 bits a round (RadixSelectKth).
+  // 1. The kk-th largest key, 8 bits a round.
   uint64_t prefix = 0;
   int need = kk;
   int shift = 56;
@@ -748,7 +748,7 @@ __device__ __forceinline__ void SelectCertifiedRequest(
   }
   auto* order = &sh.b;
   if (share || (refine && RefineWorthwhile<kSelThreads>(nopen))) {
-    // 4. Refined intervals of the open positions (sh.flag_*), by the helpers
+    // 4. Refined intervals of the open positions (sh.r_*), by the helpers
     //    or here, and the set's order again.  A wait that gives up leaves the
     //    first-pass intervals, which are sound, to the exact chains.
     if (tid == 0) sh.all = 1;
@@ -1367,10 +1367,13 @@ void LaunchScoreBounds(const PoolView& pool, const float* d_queries,
   }
   // More waves than the chip holds at once (7168), so that one that ends makes
   // room: a page per wave up to 16384 pages (32 requests of 8 x 128 heads and
-  // 300 pages each: the step took 42.9 us, 44.8 with 8192 waves, 47.0 with
-  // 4096); fewer where a workgroup's copy of a long query weighs more (16
-  // requests of 64 x 128 heads: 109.2 us with 4096, 112.4 with 8192).
-  const int target_waves = pool.elements > 4096 ? 4096 : 16384;
+  // 300 pages each, with the present select: the step 42.9 us, 44.8 with 8192
+  // waves, 47.0 with 4096).  Beyond E = 4096 a workgroup's copy of the query
+  // weighs more, and up to 8192 pages a wave takes two (16 requests of 500 pages,
+  // 40, 64 and 80 heads of 128: 52.2, 84.0 and 112.2 us; 54.3, 85.7 and 112.4 with
+  // one; 32 of 300 pages, one a wave: 76.1, 108.3 and 143.9 us; 81.6, 116.2 and
+  // 153.2 with three).
+  const int target_waves = pool.elements > 4096 && total_candidates <= 8192 ? 4096 : 16384;
   const int per_wave = std::min(
       kWave, std::max(1, (total_candidates + target_waves - 1) / target_waves));
   const int per_group = per_wave * kBoundWaves;
