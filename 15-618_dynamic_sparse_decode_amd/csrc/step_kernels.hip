@@ -462,40 +462,49 @@ struct CertSharedT {
 using CertShared = CertSharedT<kCertMaxKeys, kCertMaxKeys>;
 using CertSharedLarge = CertSharedT<kLargeMaxK + kLargeMaxOpen, kLargeMaxOpen>;
 
-// Threads per element of a pass over the set (a power of two, 4 to 16).  The
-// loops below compare every pair, about ten instructions each on all four SIMDs
-// (512 members: 18 us a sort, 22 a certification), so what matters is that no
-// wave runs without elements: sets beyond 256 take several passes of 256, and a
-// wave past the last element skips its loop.  (One thread an element from 513
-// on, nine waves' elements and sixteen waves' loops: 36 and 43 us.)
-__device__ __forceinline__ int SetParts(int count) {
-  int parts = 16;
-  while (parts > 4 && parts * count > kSelThreads) parts >>= 1;
-  return parts;
+// Threads per element of a pass over the set: 1 << shift, 4 to 16.  The loops
+// below compare every pair, about ten instructions each on all four SIMDs, so
+// what matters is that no wave runs without elements and that the reads need no
+// bounds test: sets beyond 256 take several passes of 256, a wave past the last
+// element skips its loop, and four reads at a time are whole.  The select of 512
+// of 520 candidates takes 100 us (111 with a test per read), of 513 of 1040
+// 106 (170 with one thread an element and every wave in the loop).
+__device__ __forceinline__ int SetShift(int count) {
+  int shift = 4;
+  while (shift > 2 && (count << shift) > kSelThreads) --shift;
+  return shift;
 }
 // Whether this wave has an element in the pass from element `base` on.
-__device__ __forceinline__ bool SetWaveBusy(int base, int parts, int count) {
-  return base + static_cast<int>(threadIdx.x) / kWave * kWave / parts < count;
+__device__ __forceinline__ bool SetWaveBusy(int base, int shift, int count) {
+  const int wave_first = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x));
+  return base + (wave_first >> shift) < count;
 }
 
 // from, sorted by key (descending; equal keys by position), into to: ranks by
 // counting, `parts` threads per element.  Ends with a barrier.
 template <class Set>
 __device__ __forceinline__ void SortSet(const Set& from, Set& to, int count) {
-  const int parts = SetParts(count);
+  const int shift = SetShift(count);
+  const int parts = 1 << shift;
   const int part = threadIdx.x & (parts - 1);
-  for (int base = 0; base < count; base += kSelThreads / parts) {
-    if (!SetWaveBusy(base, parts, count)) break;
-    const int t = base + static_cast<int>(threadIdx.x) / parts;
+  for (int base = 0; base < count; base += kSelThreads >> shift) {
+    if (!SetWaveBusy(base, shift, count)) break;
+    const int t = base + (static_cast<int>(threadIdx.x) >> shift);
     const uint64_t k = t < count ? from.key[t] : 0ull;
     int rank = 0;
-    for (int u0 = part; u0 < count; u0 += 4 * parts) {
+    int u = part;
+    for (; u + 3 * parts < count; u += 4 * parts) {
+      uint64_t ku[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) ku[v] = from.key[u + v * parts];
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int u = u0 + v * parts;
-        const uint64_t ku = u < count ? from.key[u] : 0ull;
-        rank += (u < count) & ((ku > k) | ((ku == k) & (u < t)));
+        rank += (ku[v] > k) | ((ku[v] == k) & (u + v * parts < t));
       }
+    }
+    for (; u < count; u += parts) {
+      const uint64_t ku = from.key[u];
+      rank += (ku > k) | ((ku == k) & (u < t));
     }
     for (int o = 1; o < parts; o <<= 1) rank += __shfl_xor(rank, o, kWave);
     if (t < count && part == 0) {
@@ -514,24 +523,32 @@ __device__ __forceinline__ void SortSet(const Set& from, Set& to, int count) {
 // Appends them to sh.open (sh.nopen counts all of them).  Ends with a barrier.
 template <class Shared, class Set>
 __device__ __forceinline__ void CertifySet(Shared& sh, const Set& set, int count, int kk) {
-  const int parts = SetParts(count);
+  const int shift = SetShift(count);
+  const int parts = 1 << shift;
   const int part = threadIdx.x & (parts - 1);
-  for (int base = 0; base < count; base += kSelThreads / parts) {
-    if (!SetWaveBusy(base, parts, count)) break;
-    const int t = base + static_cast<int>(threadIdx.x) / parts;
+  for (int base = 0; base < count; base += kSelThreads >> shift) {
+    if (!SetWaveBusy(base, shift, count)) break;
+    const int t = base + (static_cast<int>(threadIdx.x) >> shift);
     const bool in = t < count;
     const float l = in ? set.lo[t] : INFINITY;
     const float h = in ? set.hi[t] : -INFINITY;
     const int others = t < kk ? count : kk;
     int open = 0;
-    for (int u0 = part; u0 < others; u0 += 4 * parts) {
+    int u = part;
+    for (; u + 3 * parts < others; u += 4 * parts) {
+      float lu[4], hu[4];
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int u = u0 + v * parts;
-        const float lu = u < others ? set.lo[u] : INFINITY;
-        const float hu = u < others ? set.hi[u] : -INFINITY;
-        open |= (u != t) & (l <= hu) & (lu <= h);
+        lu[v] = set.lo[u + v * parts];
+        hu[v] = set.hi[u + v * parts];
       }
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        open |= (u + v * parts != t) & (l <= hu[v]) & (lu[v] <= h);
+      }
+    }
+    for (; u < others; u += parts) {
+      open |= (u != t) & (l <= set.hi[u]) & (set.lo[u] <= h);
     }
     for (int o = 1; o < parts; o <<= 1) open |= __shfl_xor(open, o, kWave);
     if (in && open != 0 && part == 0) {
