@@ -184,7 +184,9 @@ __global__ __launch_bounds__(kAttnThreads) void AttentionKernel(
 //
 // Bound by HBM: each K and V row is read once (0.5 flop per byte).
 //
-// Unsplit (piece_room = 0): workgroup (h, r) attends request r's whole list.
+// Unsplit (kSplit false, piece_room 0): workgroup (h, r) attends request r's
+// whole list.  A kernel of its own: beside the pieces' code the compiler gives
+// the token loop a schedule that is 1-5% slower.
 // A batch of few requests then runs few workgroups: one request of 32 heads
 // and 32768 tokens kept 32 of 256 CUs busy (dense, 1.07 GB: 1234 us).
 //
@@ -355,66 +357,18 @@ __device__ __forceinline__ float TakeWord(const AttentionArgs& args, unsigned lo
   return __uint_as_float(static_cast<uint32_t>(w));
 }
 
-template <int D, int LPT, int WAVES, int UNROLL>
-__global__ __launch_bounds__(WAVES * kWave) void AttentionFastKernel(
-    PoolView pool, AttentionArgs args) {
-  constexpr int DQ = D / LPT;
+// A split head's piece p (its waves' merged state in thread tid < D): published,
+// and all of the head's merged by the last workgroup to arrive.
+template <int D, int WAVES>
+__device__ __forceinline__ void MergePieces(const PoolView& pool, const AttentionArgs& args,
+                                            const AttnPiece& p, int h, float mx, float lt,
+                                            float at, AttnFastShared<WAVES, D>& sh, float* out) {
   constexpr int kThreads = WAVES * kWave;
-  constexpr int kAlign = WAVES * (kWave / LPT) * UNROLL;
-  static_assert(kThreads >= D, "a thread per dim");
-  __shared__ AttnFastShared<WAVES, D> sh;
-  __shared__ int s_page[kAttnTile];
-  __shared__ int s_ntok[kAttnTile];
   __shared__ float s_pm[kAttnMaxPieces];
   __shared__ float s_pl[kAttnMaxPieces];
   __shared__ int s_last;
   __shared__ int s_late;
-  const int h = blockIdx.x;
   const int tid = threadIdx.x;
-  const int ps = pool.page_size;
-  AttnPiece p;
-  if (args.piece_room == 0) {
-    p.r = blockIdx.y;
-    p.f1 = ListSlots(args, p.r, ps, &p.start);
-  } else if (!FindPiece<kAlign>(args, ps, blockIdx.y, &p)) {
-    return;
-  }
-  const int head_off = h * D + (tid & (kWave - 1)) % LPT * DQ;
-  AttnState<DQ> st;
-  AttnBegin<DQ>(args.queries + static_cast<size_t>(p.r) * pool.elements + head_off, args.scale,
-                st);
-  // Tiles of list entries: ids and token counts in LDS, so that a chunk's
-  // rows load without a chain of two loads before them.  (256 entries are a
-  // whole number of steps whatever the page size, so an unsplit head's waves
-  // see the slots they would see without tiles.)
-  const int s_end = (p.f1 + ps - 1) / ps;
-  for (int s0 = p.f0 / ps; s0 < s_end; s0 += kAttnTile) {
-    const int n = s_end - s0 < kAttnTile ? s_end - s0 : kAttnTile;
-    if (s0 * ps > p.f0) __syncthreads();  // the previous tile has been read
-    for (int i = tid; i < n; i += kThreads) {
-      const int page = args.list_ids[p.start + s0 + i];
-      s_page[i] = page;
-      s_ntok[i] = InPool(page, pool.capacity) ? pool.token_counts[page] : 0;
-    }
-    __syncthreads();
-    const int f0 = s0 * ps > p.f0 ? s0 * ps : p.f0;
-    const int f1 = n < kAttnTile || (s0 + n) * ps > p.f1 ? p.f1 : (s0 + n) * ps;
-    AttnRange<D, LPT, WAVES, UNROLL>(
-        pool, head_off, tid, f0, f1,
-        [&](int s, int t, int* page) {
-          *page = s_page[s - s0];
-          return t < s_ntok[s - s0];
-        },
-        st);
-  }
-  AttnMergeWave<D, LPT, WAVES>(tid, st, sh);
-  float* out = args.outputs + static_cast<size_t>(p.r) * pool.elements + static_cast<size_t>(h) * D;
-  float mx = 0.0f, lt = 0.0f, at = 0.0f;
-  if (tid < D) AttnCombine<D, WAVES>(sh, tid, &mx, &lt, &at);
-  if (p.pieces == 1) {
-    if (tid < D) out[tid] = AttnOutput(mx, lt, at);
-    return;
-  }
   unsigned long long* words =
       args.piece_words +
       (static_cast<size_t>(blockIdx.y) * pool.num_heads + h) * static_cast<size_t>(D + 2);
@@ -486,6 +440,65 @@ __global__ __launch_bounds__(WAVES * kWave) void AttentionFastKernel(
   }
 }
 
+template <int D, int LPT, int WAVES, int UNROLL, bool kSplit>
+__global__ __launch_bounds__(WAVES * kWave) void AttentionFastKernel(
+    PoolView pool, AttentionArgs args) {
+  constexpr int DQ = D / LPT;
+  constexpr int kThreads = WAVES * kWave;
+  constexpr int kAlign = WAVES * (kWave / LPT) * UNROLL;
+  static_assert(kThreads >= D, "a thread per dim");
+  __shared__ AttnFastShared<WAVES, D> sh;
+  __shared__ int s_page[kAttnTile];
+  __shared__ int s_ntok[kAttnTile];
+  const int h = blockIdx.x;
+  const int tid = threadIdx.x;
+  const int ps = pool.page_size;
+  AttnPiece p;
+  if constexpr (!kSplit) {
+    p.r = blockIdx.y;
+    p.f1 = ListSlots(args, p.r, ps, &p.start);
+  } else if (!FindPiece<kAlign>(args, ps, blockIdx.y, &p)) {
+    return;
+  }
+  const int head_off = h * D + (tid & (kWave - 1)) % LPT * DQ;
+  AttnState<DQ> st;
+  AttnBegin<DQ>(args.queries + static_cast<size_t>(p.r) * pool.elements + head_off, args.scale,
+                st);
+  // Tiles of list entries: ids and token counts in LDS, so that a chunk's
+  // rows load without a chain of two loads before them.  (256 entries are a
+  // whole number of steps whatever the page size, so an unsplit head's waves
+  // see the slots they would see without tiles.)
+  const int s_end = (p.f1 + ps - 1) / ps;
+  for (int s0 = p.f0 / ps; s0 < s_end; s0 += kAttnTile) {
+    const int n = s_end - s0 < kAttnTile ? s_end - s0 : kAttnTile;
+    if (s0 * ps > p.f0) __syncthreads();  // the previous tile has been read
+    for (int i = tid; i < n; i += kThreads) {
+      const int page = args.list_ids[p.start + s0 + i];
+      s_page[i] = page;
+      s_ntok[i] = InPool(page, pool.capacity) ? pool.token_counts[page] : 0;
+    }
+    __syncthreads();
+    const int f0 = s0 * ps > p.f0 ? s0 * ps : p.f0;
+    const int f1 = n < kAttnTile || (s0 + n) * ps > p.f1 ? p.f1 : (s0 + n) * ps;
+    AttnRange<D, LPT, WAVES, UNROLL>(
+        pool, head_off, tid, f0, f1,
+        [&](int s, int t, int* page) {
+          *page = s_page[s - s0];
+          return t < s_ntok[s - s0];
+        },
+        st);
+  }
+  AttnMergeWave<D, LPT, WAVES>(tid, st, sh);
+  float* out = args.outputs + static_cast<size_t>(p.r) * pool.elements + static_cast<size_t>(h) * D;
+  float mx = 0.0f, lt = 0.0f, at = 0.0f;
+  if (tid < D) AttnCombine<D, WAVES>(sh, tid, &mx, &lt, &at);
+  if (!kSplit || p.pieces == 1) {
+    if (tid < D) out[tid] = AttnOutput(mx, lt, at);
+    return;
+  }
+  if constexpr (kSplit) MergePieces<D, WAVES>(pool, args, p, h, mx, lt, at, sh, out);
+}
+
 // The share of the chip's time that a launch of `heads` equal unsplit heads
 // leaves to each head's slots.  About 214 workgroups load the chip; up to 256 run
 // one on a CU.  Just beyond, the CUs that got a second one are a tail of their
@@ -502,11 +515,12 @@ using AttnKernelFn = void (*)(PoolView, AttentionArgs);
 
 struct AttnVariant {
   int lpt, waves, unroll;
-  AttnKernelFn fn;
+  AttnKernelFn fn, split;
 };
 
 #define DSD_ATTN_VARIANT(L, W, U) \
-  AttnVariant{L, W, U, AttentionFastKernel<128, L, W, U>}
+  AttnVariant{L, W, U, AttentionFastKernel<128, L, W, U, false>, \
+              AttentionFastKernel<128, L, W, U, true>}
 const AttnVariant kAttnVariants[] = {
     DSD_ATTN_VARIANT(4, 4, 1),  DSD_ATTN_VARIANT(4, 4, 2),  DSD_ATTN_VARIANT(4, 8, 1),
     DSD_ATTN_VARIANT(8, 4, 1),  DSD_ATTN_VARIANT(8, 4, 2),  DSD_ATTN_VARIANT(8, 4, 4),
@@ -546,13 +560,15 @@ void LaunchAttentionT(const PoolView& pool, const AttentionArgs& args,
 // a float4 lane split.
 struct AttnShape {
   int waves = 0, align = 0;
-  AttnKernelFn fn = nullptr;
+  AttnKernelFn fn = nullptr, split = nullptr;  // split: null where none ever is
 };
 
-template <int D, int LPT, int WAVES, int UNROLL>
+template <int D, int LPT, int WAVES, int UNROLL, bool kMaySplit = true>
 AttnShape ShapeOf() {
-  return AttnShape{WAVES, WAVES * (kWave / LPT) * UNROLL,
-                   AttentionFastKernel<D, LPT, WAVES, UNROLL>};
+  AttnShape shape{WAVES, WAVES * (kWave / LPT) * UNROLL,
+                  AttentionFastKernel<D, LPT, WAVES, UNROLL, false>};
+  if constexpr (kMaySplit) shape.split = AttentionFastKernel<D, LPT, WAVES, UNROLL, true>;
+  return shape;
 }
 
 // heads: workgroups of the unsplit launch; max_slots: the lists' longest, 0:
@@ -560,22 +576,23 @@ AttnShape ShapeOf() {
 // fill the chip, take 64 dims with one chunk in flight: half the registers, so
 // more workgroups share a CU, and a short list spreads over more waves (16
 // heads of 64 slots 4.6 and 5.2 us, 32 x 16 heads of 128 slots 8.8 and 9.0, of
-// 512 24.2 and 25.6); four in flight stream longer lists faster (24 x 12 heads
-// of 3000 slots: 109 and 93 us).  80 dims: four waves for short lists, which
-// wait for eight waves' merge (16 heads of 64 slots 4.5 and 5.1 us), eight for
-// longer ones (16 heads of 1500 slots: 15.6 and 11.8).
+// 512 24.2 and 25.6); with four in flight a workgroup streams longer lists
+// faster where the launch waits for a few (dense, 17 x 32 heads of 500-2000
+// slots 77 us, 94 with one; 20 of 200-4000 153 and 160).  80 dims: four waves for
+// short lists, which wait for eight waves' merge (16 heads of 64 slots 4.5 and
+// 5.1 us), eight for longer ones (16 heads of 1500 slots: 15.6 and 11.8).
 AttnShape FastShape(int head_dim, bool wide, long long heads, long long max_slots) {
   if (head_dim == 128 && wide) {
-    return ShapeOf<128, kWideAttnLpt, kWideAttnWaves, kWideAttnUnroll>();
+    return ShapeOf<128, kWideAttnLpt, kWideAttnWaves, kWideAttnUnroll, false>();
   }
   const bool is_short = max_slots > 0 && max_slots <= (heads >= kAttnRound ? 1024 : 128);
   switch (head_dim) {
-    case 64: return is_short ? ShapeOf<64, 8, 8, 1>() : ShapeOf<64, 8, 8, 4>();
-    case 80: return is_short ? ShapeOf<80, 4, 4, 1>() : ShapeOf<80, 4, 8, 1>();
+    case 64: return is_short ? ShapeOf<64, 8, 8, 1, false>() : ShapeOf<64, 8, 8, 4>();
+    case 80: return is_short ? ShapeOf<80, 4, 4, 1, false>() : ShapeOf<80, 4, 8, 1>();
     case 96: return ShapeOf<96, 8, 8, 2>();
     case 128: {
       const AttnVariant& v = SelectAttnVariant();
-      return AttnShape{v.waves, v.waves * (kWave / v.lpt) * v.unroll, v.fn};
+      return AttnShape{v.waves, v.waves * (kWave / v.lpt) * v.unroll, v.fn, v.split};
     }
     case 256: return ShapeOf<256, 16, 8, 2>();
     default: return AttnShape{};
@@ -587,7 +604,7 @@ AttnShape FastShape(int head_dim, bool wide, long long heads, long long max_slot
 int AttentionPieceRoom(const PoolView& pool, int batch, long long max_slots) {
   const long long heads = pool.num_heads;
   const AttnShape shape = FastShape(pool.head_dim, false, batch * heads, max_slots);
-  if (shape.fn == nullptr || batch <= 0) return 0;
+  if (shape.split == nullptr || batch <= 0) return 0;
   if (max_slots > 0 && max_slots <= kAttnWhole * shape.align) return 0;  // one piece each
   if (batch * heads >= kAttnRound) return 0;
   // About one round of equal pieces for the smaller batches, which leaves the
@@ -622,7 +639,8 @@ void LaunchAttention(const PoolView& pool, const AttentionArgs& args,
   if (shape.fn != nullptr) {
     if (args.piece_room < 0 || args.piece_room > kAttnMaxPieces ||
         (args.piece_room > 0 &&
-         (args.piece_words == nullptr || args.piece_arrivals == nullptr || args.piece_tag == 0 ||
+         (shape.split == nullptr || args.piece_words == nullptr ||
+          args.piece_arrivals == nullptr || args.piece_tag == 0 ||
           static_cast<long long>(args.batch) * pool.num_heads > kAttnPieceCounters ||
           static_cast<long long>(args.batch + args.piece_room) * pool.num_heads * (D + 2) >
               static_cast<long long>(kAttnPieceWords)))) {
@@ -631,7 +649,8 @@ void LaunchAttention(const PoolView& pool, const AttentionArgs& args,
     AttentionArgs a = args;
     a.piece_share = PieceShare(heads) / static_cast<float>(args.batch);
     const dim3 grid(pool.num_heads, args.batch + args.piece_room);
-    hipLaunchKernelGGL(shape.fn, grid, dim3(shape.waves * kWave), 0, stream, pool, a);
+    hipLaunchKernelGGL(a.piece_room > 0 ? shape.split : shape.fn, grid, dim3(shape.waves * kWave),
+                       0, stream, pool, a);
     DSD_HIP_CHECK(hipGetLastError());
     return;
   }
@@ -648,7 +667,9 @@ void LaunchAttention(const PoolView& pool, const AttentionArgs& args,
 void PreloadAttentionKernels(const PoolView& pool) {
   for (long long max_slots : {0, 1}) {
     const AttnShape shape = FastShape(pool.head_dim, false, 1, max_slots);
-    if (shape.fn != nullptr) PreloadKernel(shape.fn);
+    if (shape.fn == nullptr) continue;
+    PreloadKernel(shape.fn);
+    if (shape.split != nullptr) PreloadKernel(shape.split);
   }
   if (pool.head_dim == 128 && pool.elements == kFE) PreloadKernel(FastShape(128, true, 1, 0).fn);
 }
