@@ -480,7 +480,7 @@ __global__ __launch_bounds__(WAVES * kWave) void AttentionFastKernel(
     __syncthreads();
     const int f0 = s0 * ps > p.f0 ? s0 * ps : p.f0;
     const int f1 = n < kAttnTile || (s0 + n) * ps > p.f1 ? p.f1 : (s0 + n) * ps;
-    AttnRange<D, LPT, WAVES, UNROLL>(
+    AttnRange<D, LPT, WAVES, UNROLL, kSplit>(
         pool, head_off, tid, f0, f1,
         [&](int s, int t, int* page) {
           *page = s_page[s - s0];

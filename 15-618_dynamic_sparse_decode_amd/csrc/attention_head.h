@@ -66,7 +66,10 @@ __device__ __forceinline__ void AttnBegin(const float* __restrict__ query_row, f
 // The token slots [f0, f1) of the head's page list (slot f: token f mod
 // page_size of list entry f / page_size), wave by wave from f0 in chunks.
 // row(s, t, &page): whether token t of list entry s is valid, and its page.
-template <int D, int LPT, int WAVES, int UNROLL, class Row>
+// kPin: keep a row's addresses apart from the registers its loads fill.  Where
+// the allocator shares them (it does in the split attention kernel), a chunk's
+// loads wait for every load before them.
+template <int D, int LPT, int WAVES, int UNROLL, bool kPin = false, class Row>
 __device__ __forceinline__ void AttnRange(const PoolView& pool, int head_off, int tid, int f0,
                                           int f1, Row row, AttnState<D / LPT>& st) {
   constexpr int DQ = D / LPT;
@@ -92,8 +95,11 @@ __device__ __forceinline__ void AttnRange(const PoolView& pool, int head_off, in
         if (valid[u]) {
           const size_t off = static_cast<size_t>(page) * pool.page_elems +
                              static_cast<size_t>(t) * E + head_off;
-          LoadDims<DQ>(pool.keys + off, kv[u]);
-          LoadDims<DQ>(pool.values + off, vv[u]);
+          const float* key = pool.keys + off;
+          const float* value = pool.values + off;
+          LoadDims<DQ>(key, kv[u]);
+          LoadDims<DQ>(value, vv[u]);
+          if constexpr (kPin) asm volatile("" : : "v"(key), "v"(value));
         }
       }
     }
